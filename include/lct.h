@@ -738,9 +738,9 @@ int32_t lct_compress_buffered_noalloc(const void *source, int64_t logical_numel,
 int32_t lct_set_wait_limits(int32_t lock_polls, int32_t ready_polls);
 
 /* ---- which decoder kernel lct_decode launches: LCT_DECODER_AUTO (the
- * default: the wide-tile kernel, or the compact one when only it holds the
- * whole grid at once), LCT_DECODER_WIDE or LCT_DECODER_COMPACT.  Both write
- * the same output.  Applies to launches made after the call.  No counterpart
+ * default: the grouped kernel, or the wide-tile or compact one for whole grids
+ * that they hold at once and it does not), LCT_DECODER_WIDE or
+ * LCT_DECODER_COMPACT.  All write the same output.  Applies to launches made after the call.  No counterpart
  * in the reference: tests pin each kernel on the same inputs. */
 #define LCT_DECODER_AUTO 0
 #define LCT_DECODER_WIDE 1

@@ -8,6 +8,10 @@
 // past a stream's overflow start take their exponent from the tail bytes and
 // consume no payload bits.
 //
+// Three kernels share that work: the wide one described here, a compact one
+// and a grouped one, which most grids take (choose_decoder); the latter two
+// have their own comments.
+//
 // The step loop runs in 16-step chunks, each in two phases.  The decode
 // phase walks the 16 steps using only LDS (payload, tables, overflow tails)
 // and keeps the exponent fields in registers.  The store phase then waits for
@@ -238,11 +242,16 @@ struct DecodeBatch {
     DecodeBatchJob jobs[LCT_MAX_DECODE_BATCH];
 };
 
-__global__ __launch_bounds__(kLanes, 8) void decode_batch_kernel(DecodeBatch batch) {
-    const int32_t b = static_cast<int32_t>(blockIdx.x);
+__device__ __forceinline__ int batch_job(const DecodeBatch &batch, int32_t b) {
     int j = 0;
     for (int k = 1; k < batch.n_jobs; ++k)
         if (b >= batch.first_block[k]) j = k;
+    return j;
+}
+
+__global__ __launch_bounds__(kLanes, 8) void decode_batch_kernel(DecodeBatch batch) {
+    const int32_t b = static_cast<int32_t>(blockIdx.x);
+    const int j = batch_job(batch, b);
     const DecodeBatchJob &job = batch.jobs[j];
     decode_block_wide(job.encoded, job.side, job.output, job.shifted_decode, job.center,
                       job.n_blocks, job.logical_numel, job.steps, job.fixed_words, job.rare,
@@ -471,40 +480,437 @@ __global__ __launch_bounds__(kLanes, 8) void decode_kernel_compact(
     }
 }
 
+// ---- the grouped decoder: several symbols per table lookup
+//
+// The kernels above take two dependent LDS lookups per symbol pair, so a
+// stream of 256 symbols is a chain of 256 lookups: with a few workgroups per
+// CU (a layer's weights, one activation) that chain is the launch's time, not
+// HBM.  Here one lookup of 10 bits gives up to four whole symbols (3.2 to 3.4
+// on the codebooks' own data), three lookups are taken from each 32-bit
+// window, and the exponent bytes go to an LDS tile of rows instead of staying
+// in registers in lock step, so lanes may run ahead of one another:
+//  * a wave decodes its 64 streams until each has kTileSteps more rows (or is
+//    at its end: its first overflow step, or the tensor's end), every lane at
+//    its own pace; a lookup's four exponent bytes are stored at the lane's
+//    next four rows, and those past its symbol count are overwritten later;
+//  * rows at and past a stream's overflow start are then filled from its tail;
+//  * the wave joins the tile's rows with their side bytes, fetched one tile
+//    ahead: lane j takes 8 columns of row 8 (j >> 3) + 2 i + h for i < 4,
+//    h < 2, so the swizzle's XOR within the 8 columns is the constant 2 i and
+//    every wave store is 8 whole 128-byte lines;
+//  * rows already decoded past the tile's end move to its start.
+// The tensor's last, partial block differs only in its streams' ends and in
+// the stores of the piece that holds the tensor's end.
+//
+// What bounds it: with up to one workgroup per CU the chain of lookups (27 turns
+// of three per 256 symbols; 15.6 us per public decompress at 36 blocks of 256
+// steps against the wide kernel's 24.8), then the LDS (23.0 us at 512 blocks),
+// from about 688 blocks on HBM (28.8 us, 5.3 TB/s; 85.6 us at 4096 blocks of
+// 128 steps against 90.5, inputs and outputs rotating over three sets).
+// Measured against it: the exponent bytes stored one by one in row-major tiles
+// (12 byte stores per turn: 29.6 against 28.8 us at 688 blocks, 23.2 at 512);
+// 9-bit tables or 32-row tiles (more workgroups per CU, but 15.3 to 17.7 us at
+// 36 blocks and 0.4 to 2 us slower at 4096).
+constexpr int kGroupBits = 10;      // table index bits: three lookups fit a 32-bit window
+constexpr int kGroupLookups = 3;
+constexpr int kGroupSymbols = 4;    // symbols per entry at most
+constexpr int kTileSteps = 64;
+constexpr int kUnits = kTileSteps / 32;
+// A lane passes its target by at most 3 lookups of 4 symbols less one.
+constexpr int kTileSpare = kGroupLookups * kGroupSymbols;
+// The tile holds dwords of four rows of one lane, the 64 lanes' dwords of a
+// row quad side by side, so lanes at different rows still hit 64 banks.
+constexpr int kQuadBytes = kWave * 4;
+constexpr int kTileBytes = (kTileSteps + kTileSpare + 4) / 4 * kQuadBytes;   // one wave's
+
+// Entries {up to 4 exponent bytes, total length | symbols * 8 << 8}; y = 0
+// where the first symbol is an escape.
+struct GroupTables {
+    uint2 entry[1 << kGroupBits];
+};
+
+// From the 1024-entry shifted decode table's first 256 entries: `base` (LDS,
+// 256 dwords) holds length | exponent << 8, 0 for an escape or a code longer
+// than 8 bits.  Bits past the index read as 0: a symbol is taken only if its
+// code ends within the index, and then those bits had no part in it.
+__device__ __forceinline__ void build_group_tables(GroupTables &tb, uint32_t *base,
+                                                   int32_t packed) {
+    const int t = threadIdx.x;
+    const int32_t length = packed & 255;
+    const uint32_t exponent = static_cast<uint32_t>((packed >> 8) + 127) & 255u;
+    base[t] = length >= 1 && length <= 8 ? static_cast<uint32_t>(length) | (exponent << 8) : 0u;
+    __syncthreads();
+    constexpr int kPer = (1 << kGroupBits) / kLanes;
+    uint32_t at[kPer], bytes[kPer], count[kPer];
+    bool open[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        at[k] = bytes[k] = count[k] = 0u;
+        open[k] = true;
+    }
+#pragma unroll
+    for (int s = 0; s < kGroupSymbols; ++s) {
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+            const uint32_t index = static_cast<uint32_t>(t + k * kLanes);
+            const uint32_t b = base[(index >> at[k]) & 255u];
+            const uint32_t end = at[k] + (b & 255u);
+            open[k] = open[k] && b != 0u && end <= static_cast<uint32_t>(kGroupBits);
+            if (open[k]) {
+                bytes[k] |= (b >> 8) << (8 * s);
+                count[k] += 1u;
+                at[k] = end;
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+        tb.entry[t + k * kLanes] = make_uint2(bytes[k], at[k] | (count[k] * 8u) << 8);
+}
+
+// The tile is written by dword and by byte and read 16 bytes at a time: types
+// that may alias each other.
+using TileDword = __attribute__((may_alias)) uint32_t;
+typedef uint32_t TileDwords __attribute__((ext_vector_type(4), may_alias));
+
+// One lane's column of the tile, filled from the top: `row8` is 8 x the next
+// row and `word` the rows of its dword so far.
+struct TileColumn {
+    uint8_t *base;
+    uint32_t row8, word;
+
+    // Append a lookup's exponent bytes (the bytes past its symbols are 0);
+    // advance8 = 8 x their number.  Every append stores the dword it began in;
+    // one that also fills it leaves the rest in the next.
+    __device__ __forceinline__ void append(uint32_t bytes, uint32_t advance8) {
+        const uint64_t placed = static_cast<uint64_t>(bytes) << (row8 & 24u);
+        const uint32_t first = word | static_cast<uint32_t>(placed);
+        *dword() = first;
+        const uint32_t next8 = row8 + advance8;
+        word = (next8 ^ row8) >= 32u ? static_cast<uint32_t>(placed >> 32) : first;
+        row8 = next8;
+    }
+
+    // Store the dword being filled (after a tile's last append).
+    __device__ __forceinline__ void flush() const { *dword() = word; }
+
+    __device__ __forceinline__ TileDword *dword() const {
+        return reinterpret_cast<TileDword *>(base + (row8 & ~31u) * (kQuadBytes / 32));
+    }
+};
+
+// Two BF16 values from their exponent bytes (bytes 2p, 2p + 1 of e) and side
+// bytes (of sm): each half becomes exponent << 8 | side, whose exponent moves
+// down one bit and whose sign moves up to bit 15.
+template <int kHalf>
+__device__ __forceinline__ uint32_t join_two(uint32_t e, uint32_t sm) {
+    const uint32_t x = __builtin_amdgcn_perm(e, sm, kHalf == 0 ? 0x05010400u : 0x07030602u);
+    uint32_t low, out;
+    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(low) : "s"(0x007F007Fu), "v"(x), "v"(x << 8));
+    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(out) : "s"(0x7F807F80u), "v"(x >> 1), "v"(low));
+    return out;
+}
+
+// Byte k of the four words of `w`, for k = 0..3: rows of a 4 x 4 byte block
+// whose columns are the words.
+__device__ __forceinline__ void transpose_bytes(TileDwords w, uint32_t &r0, uint32_t &r1, uint32_t &r2,
+                                                uint32_t &r3) {
+    // v_perm_b32(s0, s1, sel): bytes 0..3 select s1, 4..7 s0.
+    const uint32_t a01 = __builtin_amdgcn_perm(w.y, w.x, 0x05010400u);   // x0 y0 x1 y1
+    const uint32_t b01 = __builtin_amdgcn_perm(w.w, w.z, 0x05010400u);
+    const uint32_t a23 = __builtin_amdgcn_perm(w.y, w.x, 0x07030602u);   // x2 y2 x3 y3
+    const uint32_t b23 = __builtin_amdgcn_perm(w.w, w.z, 0x07030602u);
+    r0 = __builtin_amdgcn_perm(b01, a01, 0x05040100u);
+    r1 = __builtin_amdgcn_perm(b01, a01, 0x07060302u);
+    r2 = __builtin_amdgcn_perm(b23, a23, 0x05040100u);
+    r3 = __builtin_amdgcn_perm(b23, a23, 0x07060302u);
+}
+
+// Of a tile, lane j takes the 4 rows of quad 8 u + (j >> 3) and 8 columns,
+// for each u: kUnits units of 4 rows x 8 columns.
+struct GroupSides {
+    uint2 q[kUnits][4];
+};
+
+// The side bytes of this lane's units of the tile at `first_step` (0 past the
+// block's end).
+__device__ __forceinline__ void fetch_group_sides(GroupSides &s,
+                                                  __amdgpu_buffer_rsrc_t side, int first_step) {
+    const uint32_t j = threadIdx.x & (kWave - 1);
+    const uint32_t voffset = (j >> 3) * (4 * kLanes) + (threadIdx.x & ~(kWave - 1u)) + (j & 7) * 8;
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            s.q[u][i] = __builtin_bit_cast(
+                uint2, __builtin_amdgcn_raw_buffer_load_b64(
+                           side, voffset, (first_step + 32 * u + i) * kLanes, 0));
+}
+
+// The tile's rows joined with their side bytes and stored.  Row r of the block
+// has swizzle mask m = (row_base + r) & 254: lane 8 q + k of the wave holds
+// column 8 (q ^ (m >> 3 & 7)) + (k ^ (m & 6)) of its 64-column group.  In
+// row 4 R + i of the tile m & 4 is that of R, odd for half of the lanes (their
+// two 4-lane halves change places), and m & 2 that of i.
+__device__ __forceinline__ void store_tile(const uint8_t *tile, const GroupSides &s,
+                                           __amdgpu_buffer_rsrc_t out, int first_step,
+                                           int64_t row_base, bool full, uint32_t valid) {
+    const uint32_t j = threadIdx.x & (kWave - 1);
+    const uint32_t a = j >> 3, q = j & 7u;
+    const bool swap = (a & 1u) != 0;
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) {
+        const uint32_t row = static_cast<uint32_t>(first_step + 32 * u) + 4u * a;
+        const uint32_t m = static_cast<uint32_t>(row_base + row) & 254u;
+        const uint32_t column = ((threadIdx.x & ~(kWave - 1u)) ^ (m & 192u))
+            + 8u * (q ^ ((m >> 3) & 7u));
+        const uint8_t *quads = tile + (8 * u + a) * kQuadBytes + 32 * q;
+        const TileDwords left = *reinterpret_cast<const TileDwords *>(quads + (swap ? 16 : 0));
+        const TileDwords right = *reinterpret_cast<const TileDwords *>(quads + (swap ? 0 : 16));
+        uint32_t el[4], er[4];
+        transpose_bytes(left, el[0], el[1], el[2], el[3]);
+        transpose_bytes(right, er[0], er[1], er[2], er[3]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t sl = swap ? s.q[u][i].y : s.q[u][i].x;
+            const uint32_t sr = swap ? s.q[u][i].x : s.q[u][i].y;
+            const uint32_t y[4] = {join_two<0>(el[i], sl), join_two<1>(el[i], sl),
+                                   join_two<0>(er[i], sr), join_two<1>(er[i], sr)};
+            const int x = i >> 1;
+            const uint4 v = make_uint4(y[0 ^ x], y[1 ^ x], y[2 ^ x], y[3 ^ x]);
+            const uint32_t element = (row + i) * kLanes + column;
+            if (full || element + 8 <= valid) {
+                store_b128<kStreaming>(v, out, element * 2u);
+            } else if (element < valid) {
+                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (uint32_t k = 0; k < 8; ++k)
+                    if (element + k < valid)
+                        __builtin_amdgcn_raw_buffer_store_b16(
+                            static_cast<uint16_t>(w[k / 2] >> (16 * (k & 1))), out,
+                            (element + k) * 2u, 0, kStreaming);
+            }
+        }
+    }
+}
+
+// Codec block `block` of one tensor, by the workgroup.
+__device__ __forceinline__ void decode_block_grouped(
+    const int32_t *__restrict__ encoded, const uint8_t *__restrict__ side,
+    uint16_t *__restrict__ output, const int32_t *__restrict__ shifted_decode,
+    const int32_t *__restrict__ center_ptr, int64_t n_blocks, int64_t logical_numel, int S,
+    int W, int rare, const lct_overflow &ov, int has_overlay, int64_t block) {
+    extern __shared__ uint32_t stage[];   // register_stage_bytes(W): rows 3..W-1
+    __shared__ __attribute__((aligned(16))) GroupTables tb;
+    __shared__ int32_t scratch[kWavesPerBlock];
+    __shared__ uint8_t tail_lds[kTailLds];
+    __shared__ __attribute__((aligned(16))) uint8_t tiles[kWavesPerBlock][kTileBytes];
+    // The base table and the overflow maps (3 KiB) are only used before the
+    // first tile is decoded.
+    uint32_t *base = reinterpret_cast<uint32_t *>(&tiles[0][0]);
+    int32_t *map_start = reinterpret_cast<int32_t *>(base + kLanes);
+    int32_t *map_offset = map_start + kLanes;
+    const int t = threadIdx.x;
+    const int64_t row_base = block * S;
+    const int64_t logical_base = row_base * kLanes;
+    const uint32_t block_elems = static_cast<uint32_t>(S) * kLanes;
+    const int64_t remaining = logical_numel - logical_base;
+    const uint32_t valid = remaining < block_elems ? static_cast<uint32_t>(remaining) : block_elems;
+    const bool full = valid == block_elems;
+    const __amdgpu_buffer_rsrc_t side_rsrc = make_rsrc(side + logical_base, block_elems);
+    const __amdgpu_buffer_rsrc_t out_rsrc = make_rsrc(output + logical_base, 2u * valid);
+
+    const int32_t packed = shifted_decode[t];
+    const int32_t center = center_ptr[0];
+    uint32_t words[kRegisterRows];
+    load_register_rows(encoded, n_blocks * kLanes, block, words);
+    stage_payload_rows(stage, encoded, n_blocks * kLanes, block, kRegisterRows, W);
+    const OverlayHead head = load_overlay_head(ov, has_overlay != 0, block, n_blocks);
+    GroupSides sides;
+    fetch_group_sides(sides, side_rsrc, 0);
+    build_group_tables(tb, base, packed);
+    const LaneOverlay lane = build_overlay(ov, head, S, map_start, map_offset, scratch, tail_lds,
+                                           kTailLds);
+    wait_memory();
+    __syncthreads();   // payload, table and tails visible; the maps no longer read
+
+    // This stream's symbols in the payload: the rows before its overflow start
+    // that lie inside the tensor.
+    int32_t limit = lane.start;
+    if (!full) {
+        const int32_t rows = static_cast<int32_t>(valid / kLanes);
+        const uint32_t column = static_cast<uint32_t>(t)
+            ^ static_cast<uint32_t>((row_base + rows) & 254);
+        limit = min(limit, rows + (column < valid % kLanes ? 1 : 0));
+    }
+
+    uint8_t *const tile = tiles[t / kWave];
+    TileColumn column{tile + (t & (kWave - 1)) * 4, 0u, 0u};
+    const uint32_t *const stage_lane = stage + t - kRegisterRows * kLanes;
+    const uint32_t pad_row = static_cast<uint32_t>(W) - 1u;
+    uint32_t lo = words[0], hi = words[1], nx = words[2], pos = 0, next_row = kRegisterRows;
+#pragma unroll 1
+    for (int first = 0; first < S; first += kTileSteps) {
+        const int32_t target8 = 8 * min(kTileSteps, limit - first);   // may be negative
+        if (static_cast<int32_t>(column.row8) < target8) {
+            // Each lookup's bytes are appended while the next lookup is in
+            // flight (the loop's last, e2's, in the next turn).
+            uint32_t held = 0u, held8 = 0u, row8 = column.row8;
+            do {
+                const uint32_t pending = stage_lane[next_row * kLanes];
+                const uint32_t bits = __builtin_amdgcn_alignbit(hi, lo, pos);
+                uint2 e0 = tb.entry[bits & ((1u << kGroupBits) - 1u)];
+                __builtin_amdgcn_sched_barrier(0);
+                column.append(held, held8);
+                __builtin_amdgcn_sched_barrier(0);
+                uint32_t third = ~0u;
+                if (__builtin_expect(__any(e0.y == 0u), 0)) {
+                    // ESC + 8-bit literal table index (primitives.py:29-35).
+                    const bool escaped = e0.y == 0u;
+                    const int32_t literal = static_cast<int32_t>((bits >> rare) & 255u);
+                    e0.x = escaped ? static_cast<uint32_t>(index_to_exponent(literal, center) + 127)
+                                         & 255u
+                                   : e0.x;
+                    e0.y = escaped ? static_cast<uint32_t>(rare + 8) | 8u << 8 : e0.y;
+                    third = escaped ? 0u : third;   // its window would pass the 32 bits' end
+                }
+                const uint2 e1 = tb.entry[__builtin_amdgcn_ubfe(bits, e0.y, kGroupBits)];
+                __builtin_amdgcn_sched_barrier(0);
+                column.append(e0.x, e0.y >> 8);
+                __builtin_amdgcn_sched_barrier(0);
+                const uint32_t two = e0.y + e1.y;   // lengths in bits 0..4, rows from bit 8
+                uint2 e2 = tb.entry[__builtin_amdgcn_ubfe(bits, two, kGroupBits)];
+                __builtin_amdgcn_sched_barrier(0);
+                column.append(e1.x, e1.y >> 8);
+                __builtin_amdgcn_sched_barrier(0);
+                e2.y &= third;
+                held = e2.x & third;
+                held8 = e2.y >> 8;
+                const uint32_t all = two + e2.y;
+                row8 += all >> 8;
+                const uint32_t p = pos + (all & 63u);
+                const bool cross = p >= 32u;
+                pos = p & 31u;
+                lo = cross ? hi : lo;
+                hi = cross ? nx : hi;
+                nx = cross ? pending : nx;
+                next_row = cross ? min(next_row + 1u, pad_row) : next_row;
+            } while (static_cast<int32_t>(row8) < target8);
+            column.append(held, held8);
+            column.flush();
+        }
+        if (lane.wave_start < first + kTileSteps) {
+            // Rows at and past a stream's overflow start, from its tail.
+            const uint8_t *const tail = lane.lds ? nullptr : lane.tail;
+            for (int r = max(lane.start - first, 0); r < kTileSteps; ++r) {
+                const int32_t i = lane.offset + (first + r - lane.start);
+                const uint32_t byte = tail != nullptr ? tail[i] : tail_lds[i];
+                column.base[(r >> 2) * kQuadBytes + (r & 3)] = static_cast<uint8_t>(byte + 127u);
+            }
+        }
+        GroupSides next;
+        const int ahead = first + kTileSteps;
+        fetch_group_sides(next, side_rsrc, ahead);
+        __builtin_amdgcn_wave_barrier();
+        store_tile(tile, sides, out_rsrc, first, row_base, full, valid);
+        __builtin_amdgcn_wave_barrier();
+        sides = next;
+        // Rows past the tile's end move to its start.
+        uint32_t moved[kTileSpare / 4];
+#pragma unroll
+        for (int k = 0; k < kTileSpare / 4; ++k)
+            moved[k] = *reinterpret_cast<const TileDword *>(
+                column.base + (kTileSteps / 4 + k) * kQuadBytes);
+#pragma unroll
+        for (int k = 0; k < kTileSpare / 4; ++k)
+            *reinterpret_cast<TileDword *>(column.base + k * kQuadBytes) = moved[k];
+        column.row8 -= 8 * kTileSteps;
+    }
+}
+
+__global__ __launch_bounds__(kLanes) void decode_kernel_grouped(
+    const int32_t *__restrict__ encoded, const uint8_t *__restrict__ side,
+    uint16_t *__restrict__ output, const int32_t *__restrict__ shifted_decode,
+    const int32_t *__restrict__ center_ptr, int64_t n_blocks, int64_t logical_numel, int S,
+    int W, int rare, lct_overflow ov, int has_overlay) {
+    decode_block_grouped(encoded, side, output, shifted_decode, center_ptr, n_blocks,
+                         logical_numel, S, W, rare, ov, has_overlay, blockIdx.x);
+}
+
+__global__ __launch_bounds__(kLanes) void decode_batch_kernel_grouped(DecodeBatch batch) {
+    const int32_t b = static_cast<int32_t>(blockIdx.x);
+    const int j = batch_job(batch, b);
+    const DecodeBatchJob &job = batch.jobs[j];
+    decode_block_grouped(job.encoded, job.side, job.output, job.shifted_decode, job.center,
+                         job.n_blocks, job.logical_numel, job.steps, job.fixed_words, job.rare,
+                         job.ov, job.has_overlay, b - batch.first_block[j]);
+}
+
 // Workgroups of each decoder that the current device holds at once for W
 // payload words (CUs x workgroups per CU at that kernel's LDS), looked up once
 // per device and W.
+struct DecoderSlots {
+    int32_t wide, compact, grouped;
+};
+
 constexpr int kSlotDevices = 64;
+constexpr int kSlotBits = 20;
 std::atomic<int64_t> g_decoder_slots[kSlotDevices][kMaxWords + 1];
 
 // lct_set_decoder's choice (LCT_DECODER_*).
 std::atomic<int32_t> g_decoder_mode{LCT_DECODER_AUTO};
 
-int32_t decoder_slots(int W, int32_t *wide, int32_t *compact) {
+int32_t decoder_slots(int W, DecoderSlots *slots) {
     int device = 0;
     if (hipError_t e = hipGetDevice(&device)) return static_cast<int32_t>(e);
     if (device < 0 || device >= kSlotDevices || W < 0 || W > kMaxWords) return LCT_E_ARG;
     int64_t cached = g_decoder_slots[device][W].load(std::memory_order_relaxed);
     if (cached == 0) {
-        int cus = 0, per_wide = 0, per_compact = 0;
-        const size_t lds = static_cast<size_t>(register_stage_bytes(W));
+        int cus = 0;
         if (hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
                                                  device))
             return static_cast<int32_t>(e);
-        if (hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_wide, reinterpret_cast<const void *>(decode_kernel), kLanes, lds))
-            return static_cast<int32_t>(e);
-        if (hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_compact, reinterpret_cast<const void *>(decode_kernel_compact), kLanes,
-                lds))
-            return static_cast<int32_t>(e);
-        cached = (static_cast<int64_t>(cus) * per_wide << 32)
-                 | static_cast<uint32_t>(cus * per_compact);
+        const size_t lds = static_cast<size_t>(register_stage_bytes(W));
+        const void *kernels[3] = {reinterpret_cast<const void *>(decode_kernel),
+                                  reinterpret_cast<const void *>(decode_kernel_compact),
+                                  reinterpret_cast<const void *>(decode_kernel_grouped)};
+        for (int k = 0; k < 3; ++k) {
+            int per_cu = 0;
+            if (hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernels[k],
+                                                                            kLanes, lds))
+                return static_cast<int32_t>(e);
+            cached |= static_cast<int64_t>(cus * per_cu) << (k * kSlotBits);
+        }
         g_decoder_slots[device][W].store(cached, std::memory_order_relaxed);
     }
-    *wide = static_cast<int32_t>(cached >> 32);
-    *compact = static_cast<int32_t>(cached & 0xFFFFFFFF);
+    constexpr int64_t kMask = (int64_t{1} << kSlotBits) - 1;
+    *slots = {static_cast<int32_t>(cached & kMask),
+              static_cast<int32_t>((cached >> kSlotBits) & kMask),
+              static_cast<int32_t>((cached >> (2 * kSlotBits)) & kMask)};
     return LCT_OK;
+}
+
+// The decoder for a grid of n_blocks workgroups (LCT_DECODER_AUTO): the
+// grouped one, except between the grids it holds at once and those that the
+// wide or the compact one holds at once, which then run in one round where the
+// grouped one needs two.  `ragged`: the last block is partial, which costs the
+// wide and compact kernels another 3 (S = 128) to 9 us (S = 256) and the
+// grouped one nothing; it then takes every grid.  Public decompress, us
+// (wide / compact / grouped; W = 25 holds 1024 / 1536 / 768 workgroups, W = 12
+// 2048 / 2048 / 1024):
+//   W = 25:   36 blocks 24.8 / 28.8 / 15.6    688: 31.1 / 35.7 / 28.8
+//             767 ragged 39.0 / 40.7 / 29.5   1024: 39.0 / 42.1 / 43.5
+//            1536 blocks 72.2 / 77.1 / 66.1   2048: 95.5 / 115 / 92.7
+//   W = 12:   37 ragged 19.0 / 19.3 / 13.4    1024: 21.7 / 22.4 / 21.1
+//            2048 blocks 42.5 / 39.9 / 43.4   4096: 90.5 / 90.4 / 85.6
+enum class Decoder { kWide, kCompact, kGrouped };
+
+Decoder choose_decoder(int64_t n_blocks, bool ragged, const DecoderSlots &slots) {
+    if (ragged || n_blocks <= slots.grouped) return Decoder::kGrouped;
+    // The wide kernel's 16-byte stores are faster where it holds the grid too
+    // (W = 25: 81 against 90 us at 2048 blocks; C3: 40 against 44 us).
+    if (n_blocks <= slots.wide) return Decoder::kWide;
+    return n_blocks <= slots.compact ? Decoder::kCompact : Decoder::kGrouped;
 }
 
 }  // namespace
@@ -537,18 +943,17 @@ extern "C" int32_t lct_decode(const int32_t *encoded, const uint8_t *side, int16
     // a reference geometry).
     if (g.fixed_words <= kRegisterRows) return LCT_E_GEOMETRY;
     const size_t lds = static_cast<size_t>(register_stage_bytes(g.fixed_words));
-    int32_t wide_slots = 0, compact_slots = 0;
-    if (int32_t e = decoder_slots(g.fixed_words, &wide_slots, &compact_slots)) return e;
-    // The wide-tile kernel, unless the whole grid fits the device at once only
-    // with the compact one (C2: 2048 blocks at W = 19 take 1.33 rounds of the
-    // wide kernel, one of the compact; 51.5 -> 44.8 us).  With the same number
-    // of rounds the wide kernel's 16-byte stores are faster (W = 25: 81 against
-    // 90 us at 2048 blocks, 347 against 366 us at 8192; C3: 40 against 44 us).
+    DecoderSlots slots;
+    if (int32_t e = decoder_slots(g.fixed_words, &slots)) return e;
     const int32_t mode = g_decoder_mode.load(std::memory_order_relaxed);
-    const bool compact = mode == LCT_DECODER_AUTO
-                             ? n_blocks > wide_slots && n_blocks <= compact_slots
-                             : mode == LCT_DECODER_COMPACT;
-    const auto kernel = compact ? decode_kernel_compact : decode_kernel;
+    const Decoder decoder = mode == LCT_DECODER_WIDE      ? Decoder::kWide
+                            : mode == LCT_DECODER_COMPACT ? Decoder::kCompact
+                                                          : choose_decoder(n_blocks,
+                                                                           logical_numel != size,
+                                                                           slots);
+    const auto kernel = decoder == Decoder::kGrouped   ? decode_kernel_grouped
+                        : decoder == Decoder::kCompact ? decode_kernel_compact
+                                                       : decode_kernel;
     if (hipError_t e = reserve_dynamic_lds(reinterpret_cast<const void *>(kernel), lds))
         return static_cast<int32_t>(e);
     hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(n_blocks)), dim3(kLanes), lds,
@@ -572,7 +977,8 @@ extern "C" int32_t lct_decode_batch(const lct_decode_job *jobs, int32_t n_jobs,
     DecodeBatch batch{};
     batch.n_jobs = n_jobs;
     int64_t total = 0;
-    size_t lds = 0;
+    int32_t max_words = 0;
+    bool ragged = false;
     for (int32_t j = 0; j < n_jobs; ++j) {
         const lct_decode_job &in = jobs[j];
         if (!in.encoded || !in.side || !in.output || !in.shifted_decode || !in.center)
@@ -607,14 +1013,20 @@ extern "C" int32_t lct_decode_batch(const lct_decode_job *jobs, int32_t n_jobs,
         out.rare = in.rare_length;
         out.has_overlay = in.has_overflow ? 1 : 0;
         out.ov = in.has_overflow ? in.overflow : lct_overflow{};
-        const size_t job_lds = static_cast<size_t>(register_stage_bytes(g.fixed_words));
-        lds = job_lds > lds ? job_lds : lds;
+        ragged = ragged || in.logical_numel != in.size;
+        max_words = g.fixed_words > max_words ? g.fixed_words : max_words;
     }
     batch.first_block[n_jobs] = static_cast<int32_t>(total);
-    if (hipError_t e = reserve_dynamic_lds(reinterpret_cast<const void *>(&decode_batch_kernel),
-                                           lds))
+    const size_t lds = static_cast<size_t>(register_stage_bytes(max_words));
+    DecoderSlots slots;
+    if (int32_t e = decoder_slots(max_words, &slots)) return e;
+    slots.compact = 0;   // no batched form
+    const auto kernel = choose_decoder(total, ragged, slots) == Decoder::kWide
+                            ? decode_batch_kernel
+                            : decode_batch_kernel_grouped;
+    if (hipError_t e = reserve_dynamic_lds(reinterpret_cast<const void *>(kernel), lds))
         return static_cast<int32_t>(e);
-    hipLaunchKernelGGL(decode_batch_kernel, dim3(static_cast<uint32_t>(total)), dim3(kLanes), lds,
-                       stream, batch);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(total)), dim3(kLanes), lds, stream,
+                       batch);
     return static_cast<int32_t>(hipGetLastError());
 }

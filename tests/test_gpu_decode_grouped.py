@@ -1,0 +1,65 @@
+"""GPU: the grouped decoder (several symbols per table lookup) at the sizes where
+its tiles, its streams' ends and its choice against the other decoders change.
+The codec is lossless, so a decode is right exactly when it restores the input."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import require_gpu
+from losslessly_compressed_tensors_amd.codec.decode import decode_batch
+from losslessly_compressed_tensors_amd.codec.geometry import geometry
+from losslessly_compressed_tensors_amd.comp_format import Distribution, DistType, NoiseLevel
+from losslessly_compressed_tensors_amd.operations import compress, decompress
+
+pytestmark = pytest.mark.gpu
+
+LAYOUTS = [(DistType.GAUSSIAN, NoiseLevel.CLEAN), (DistType.LAPLACE, NoiseLevel.CLEAN),
+           (DistType.EMPIRICAL, NoiseLevel.SPARSE), (DistType.GAUSSIAN, NoiseLevel.MEDIUM),
+           (DistType.LAPLACE, NoiseLevel.HIGH)]
+
+
+def _values(kind: str, n: int) -> torch.Tensor:
+    rng = np.random.default_rng(n)
+    if kind == "bits":       # every exponent: escapes, and overflow in every stream
+        bits = rng.integers(0, 65536, size=n, dtype=np.uint16)
+    elif kind == "zeros":    # one symbol: the longest or the shortest codes
+        bits = np.zeros(n, dtype=np.uint16)
+    else:                    # few overflowing streams, whose tails are short
+        x = torch.from_numpy(rng.standard_normal(n, dtype=np.float32)).to(torch.bfloat16)
+        return x.cuda()
+    return torch.from_numpy(bits.view(np.int16)).view(torch.bfloat16).cuda()
+
+
+@pytest.mark.parametrize("family,noise", LAYOUTS)
+@pytest.mark.parametrize("kind", ["normal", "bits", "zeros"])
+def test_grouped_decode_restores_tile_and_block_edges(family, noise, kind):
+    """Ends inside and at the edges of a row, a 32-row unit, a 64-row tile and
+    a block."""
+    require_gpu()
+    print(f"case grouped {family.name} {noise.name} {kind}", flush=True)
+    dist = Distribution(family, noise_level=noise)
+    block = geometry(dist)[0]
+    for n in (1, 7, 8, 255, 256, 257, 32 * 256 - 1, 32 * 256 + 5, 64 * 256, 64 * 256 + 1,
+              block - 1, block, block + 1, 3 * block + 64 * 256 + 131):
+        x = _values(kind, n)
+        assert torch.equal(decompress(compress(x, dist)).view(torch.int16), x.view(torch.int16)), n
+
+
+@pytest.mark.parametrize("blocks", [767, 768, 1024, 1600])
+def test_decode_around_the_grids_held_at_once(blocks):
+    """W = 25: 768 workgroups of the grouped kernel and 1024 of the wide one are
+    resident at once; single decodes and one batched launch of two tensors on
+    either side of both, whole and ragged."""
+    require_gpu()
+    print(f"case grids {blocks}", flush=True)
+    dist = Distribution(DistType.LAPLACE)
+    block = geometry(dist)[0]
+    generator = torch.Generator(device="cuda").manual_seed(blocks)
+    for n in (blocks * block, blocks * block - 333):
+        x = torch.randn(n, device="cuda", generator=generator).to(torch.bfloat16)
+        whole = compress(x, dist)
+        assert torch.equal(decompress(whole).view(torch.int16), x.view(torch.int16))
+        half = (blocks // 2) * block
+        parts = [x[:half], x[half:]]
+        for y, part in zip(decode_batch([compress(p, dist) for p in parts]), parts):
+            assert torch.equal(y.view(torch.int16), part.view(torch.int16))
