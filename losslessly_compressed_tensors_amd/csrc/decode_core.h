@@ -49,39 +49,6 @@ struct DecodeTables {
     }
 };
 
-// Tables of the fused update kernels: the same entries with the exponent in
-// FP32 position (len | e_raw << 23), one dword each, so a decoded value is one
-// bit-field insert away from its FP32 bits (join_float) and the entry needs no
-// masking before that.  Lengths stay in bits 0..4, so (t0 + t1) & 127 still
-// adds two lengths.  An escaped literal's exponent is computed from the
-// center (index_to_exponent) instead of read from a second table: escapes are
-// rare, and the 1 KiB this saves keeps the two-operand kernel's LDS at three
-// workgroups per CU.
-struct FloatDecodeTables {
-    uint32_t entry[256];
-
-    __device__ __forceinline__ uint32_t escaped(uint32_t literal, int32_t center) const {
-        return static_cast<uint32_t>(
-                   (index_to_exponent(static_cast<int32_t>(literal), center) + 127) & 255)
-            << 23;
-    }
-    static __device__ __forceinline__ uint32_t tail(uint32_t byte) {
-        return ((byte + 127u) & 255u) << 23;
-    }
-};
-
-// FloatDecodeTables from the 1024-entry shifted decode table, one entry per
-// thread of a 256-thread block.
-__device__ __forceinline__ void build_float_decode_tables(
-    FloatDecodeTables &tb, const int32_t *__restrict__ shifted_decode) {
-    const int32_t packed = shifted_decode[threadIdx.x];
-    const int32_t length = packed & 255;
-    const uint32_t field = static_cast<uint32_t>(((packed >> 8) + 127) & 255) << 23;
-    tb.entry[threadIdx.x] = (length >= 1 && length <= 8)
-                                ? (static_cast<uint32_t>(length) | field)
-                                : static_cast<uint32_t>(kEscapeLength);
-}
-
 // Entry `t` of both tables from entry t of the 1024-entry shifted decode
 // table (len | exp << 8).
 __device__ __forceinline__ void build_decode_entry(DecodeTables &tb, int t, int32_t packed,
@@ -312,7 +279,7 @@ struct StreamCursorT {
     uint32_t pad_row;         // W: the zero row after the payload
     uint32_t pending;         // word next_row, read at the start of a pair
     int32_t rare;
-    int32_t center;           // the tensor's center (escaped literals of FloatDecodeTables)
+    int32_t center;           // the tensor's center (escaped literals of CompactDecodeTables)
 
     __device__ __forceinline__ void init(const uint32_t *stage_lane, const Tables *tables,
                                          uint32_t words, int32_t rare_length,
@@ -415,82 +382,6 @@ struct StreamCursorT {
 // The codec kernels' cursor: one lane per stream of a block, rows of 256 words.
 using StreamCursor = StreamCursorT<kLanes>;
 
-// A cursor that keeps no window in registers: each pair reads the two words at
-// its bit position (rows pos/32 and pos/32 + 1, 1 KiB apart: one
-// ds_read2st64) and extracts 32 bits with alignbit.  Fewer instructions per
-// pair than StreamCursorT (no window shifting) at the cost of one more LDS
-// round trip on the pair's dependency chain; for kernels bounded by
-// instruction issue rather than by that chain.  Needs the block's W rows and
-// two zero pad rows staged (window_stage_bytes); the row is clamped to W, so
-// no read leaves the stage whatever the payload holds.
-__host__ __device__ constexpr int32_t window_stage_bytes(int W) { return (W + 2) * kLanes * 4; }
-
-template <class Tables = DecodeTables>
-struct WindowCursorT {
-    using TablesT = Tables;
-    const uint32_t *stage;   // stage + lane; row r at stage[r * kLanes]
-    const Tables *tb;
-    uint32_t pos;            // bits consumed
-    uint32_t last_row;       // W: the first pad row
-    int32_t rare;
-    int32_t center;
-
-    __device__ __forceinline__ void init(const uint32_t *stage_lane, const Tables *tables,
-                                         uint32_t words, int32_t rare_length,
-                                         int32_t center_value = 0) {
-        stage = stage_lane;
-        tb = tables;
-        pos = 0;
-        last_row = words;
-        rare = rare_length;
-        center = center_value;
-    }
-
-    __device__ __forceinline__ void first_lookup(uint32_t &bits, uint32_t &t0) {
-        const uint32_t row = min(pos >> 5, last_row);
-        const uint32_t *at = stage + row * kLanes;
-        bits = __builtin_amdgcn_alignbit(at[kLanes], at[0], pos);
-        t0 = tb->entry[bits & 255u];
-    }
-
-    __device__ __forceinline__ uint32_t second_lookup(uint32_t bits, uint32_t t0) const {
-        return tb->entry[__builtin_amdgcn_ubfe(bits, t0, 8)];
-    }
-
-    // Escaped symbols (as StreamCursorT::resolve); returns len0 + len1.
-    __device__ __forceinline__ uint32_t resolve(uint32_t bits, uint32_t &t0, uint32_t &t1) const {
-        uint32_t sum = (t0 + t1) & 127u;
-        if (__builtin_expect(__any(sum >= 32u), 0)) {
-            const uint32_t escaped = static_cast<uint32_t>(rare) + 8u;
-            uint32_t l0 = t0 & 31u;
-            if (l0 == kEscapeLength) {
-                l0 = escaped;
-                t0 = tb->escaped((bits >> rare) & 255u, center) | escaped;
-                t1 = tb->entry[(bits >> l0) & 255u];
-            }
-            if ((t1 & 31u) == kEscapeLength)
-                t1 = tb->escaped((bits >> (l0 + static_cast<uint32_t>(rare))) & 255u, center)
-                    | escaped;
-            sum = (t0 + t1) & 127u;
-        }
-        return sum;
-    }
-
-    __device__ __forceinline__ uint32_t next_fields(uint32_t &f0, uint32_t &f1) {
-        uint32_t bits, t0;
-        first_lookup(bits, t0);
-        uint32_t t1 = second_lookup(bits, t0);
-        const uint32_t sum = resolve(bits, t0, t1);
-        f0 = t0;
-        f1 = t1;
-        return sum;
-    }
-
-    __device__ __forceinline__ void advance(uint32_t bits) { pos += bits; }
-};
-
-using WindowCursor = WindowCursorT<>;
-
 // BF16 bits of a decoded entry (exponent field at bits 7..14, nothing at bit 15
 // or above) and its side byte: one multiply and one bit-field insert
 // (v_bfi_b32 takes bits 0..6 and 15 from the spread side byte and the rest
@@ -503,7 +394,8 @@ __device__ __forceinline__ uint32_t join_entry(uint32_t entry, uint32_t sm) {
     return out;
 }
 
-// FP32 bits of a decoded FloatDecodeTables entry and its side byte: v_perm
+// FP32 bits of an entry with the exponent in FP32 position (QuadTables) and its
+// side byte: v_perm
 // copies the side byte into bytes 2 and 3 (mantissa at bits 16..22, sign at
 // bit 31, zeros below bit 16), and one bit-field insert (mask 0x807FFFFF)
 // takes those bits and the entry's exponent, dropping its length bits.

@@ -23,19 +23,28 @@
 //    result's exponent bytes written (logical order, those rows only), which
 //    is where the compaction reads their tails, as in the precomputed path.
 //
-// The encoder side writes each payload word straight to HBM when the word
-// completes (one 4-byte store by the lanes whose word completed in a pair,
-// merged in L2), so the workgroup's LDS holds only A's payload: at W = 25,
-// four blocks fit per CU.  The result's side bytes leave with the default
-// cache policy: a wave writes 64 bytes of each 128-byte row line, and
-// non-temporal stores of half lines wrote 16% more than the side bytes (C4:
-// 73.6 MB against 62.9 MB per launch; with the default policy 63.3 MB, at
-// equal kernel time).
+// Both directions work in quads of symbols (update_core.h).  The encoder side
+// writes each payload word straight to HBM when the word completes (one 4-byte
+// store by the lanes whose word a quad completed, merged in L2), so the
+// workgroup's LDS holds only A's payload (30.9 KiB in all at W = 25).  The
+// result's side bytes leave with the default cache policy: a wave writes 64
+// bytes of each 128-byte row line, and non-temporal stores of half lines wrote
+// 16% more than the side bytes (C4: 73.6 MB against 62.9 MB per launch; with
+// the default policy 63.3 MB, at equal kernel time).
+//
+// Measured (kernel trace, three operand sets in turn; pairs of symbols, a
+// register or LDS window per pair and one step loop per overlay, before ->
+// quads): pointwise_encode_kernel 64.0 -> 61.1 us at 688 blocks, 38.2 -> 36.2
+// at one; dual_encode_kernel 75.6 -> 69.2 and 46.7 -> 43.0.  A ragged tensor's
+// last block runs the same loop (the whole momentum step at 767 blocks, ragged:
+// 75.8 us, against 150 us with a separate loop for partial blocks).  The three waves a SIMD holds
+// keep its VALU 75% busy (203 and 275 instructions per 8 steps); the rest is
+// waits for the lookups' LDS round trips.
 #include <algorithm>
 
 #include "batch.h"
-#include "pointwise_ops.h"
 #include "reserve.h"
+#include "update_core.h"
 
 namespace lct {
 namespace {
@@ -166,11 +175,6 @@ __device__ __forceinline__ void publish_block(const KernelBookkeeping &bk,
                              static_cast<int32_t>(n_blocks), reserve);
     }
 }
-
-// Cursors of the fused encode kernels, over FloatDecodeTables: decoded
-// entries become FP32 operands with one v_perm and one v_bfi (join_float).
-using UpdateCursor = StreamCursorT<kLanes, FloatDecodeTables>;
-using UpdateWindow = WindowCursorT<FloatDecodeTables>;
 
 // Overflow start and tail byte index of one stream (block, lane) of A, from
 // the block's entry list (ascending lanes, tails concatenated in entry order:
@@ -320,125 +324,15 @@ __global__ __launch_bounds__(kSampleGroup) void pointwise_sample_kernel(
 // ---- the fused decode -> operation -> encode kernel
 //
 // Memory operations are arranged for gfx9's single load/store counter
-// (vmcnt): a chunk's A side bytes and B words are fetched one chunk ahead,
+// (vmcnt): a chunk's A side bytes and B words are fetched two chunks ahead,
 // before the previous chunk's stores are issued, and every store is
 // unconditional -- lanes that must not write get an out-of-range buffer offset,
 // which the hardware drops.  The compiler can then wait for exactly the loads
 // it needs without also waiting for recent stores.
-
-// Buffer offset rejected by the range check of every resource used here
-// (num_records < 2^31): loads return 0, stores are dropped.
-constexpr uint32_t kOutOfRange = 0x80000000u;
-
-// Encoder state of one lane's output stream.  Word r of the stream is at byte
-// r * row_bytes + 4 * lane of the block's payload resource.  pos counts the
-// bits of every pair so far, so once a pair does not fit, pos stays above the
-// limit and every later pair overflows too (encode.py:73-90: only the first
-// overflowing pair matters); word and row_off then keep the bits before that
-// pair, which finish() stores.
-struct StreamWriter {
-    __amdgpu_buffer_rsrc_t out;
-    uint32_t row_bytes;   // 4 * n_streams
-    uint32_t row_off;     // byte offset of the word being filled
-    uint32_t end_off;     // row_off of row W
-    uint32_t limit;       // 32 W
-    uint32_t pos;         // bits of all pairs so far
-    uint32_t word;        // bits of the word being filled
-    uint32_t fits;        // pairs that fit
-
-    __device__ __forceinline__ bool overflowed() const { return pos > limit; }
-
-    // Hold row_bytes in a VGPR from here on: a row advance is then one
-    // v_cndmask and one v_add per pair (with row_bytes in an SGPR beside the
-    // SGPR condition, gfx9's one-scalar-operand limit costs a copy per pair).
-    __device__ __forceinline__ void keep_row_bytes_in_vgpr() { asm volatile("" : "+v"(row_bytes)); }
-
-    // The first pair that did not fit is the one after the pairs that fit, so
-    // its (even) step is twice their count.
-    __device__ __forceinline__ int32_t extra_start() const { return static_cast<int32_t>(2 * fits); }
-
-    // Append the pair code of encode entries e0/e1 ({reversed code, length};
-    // {0, 0} = no code), following encode.py:66-90.  Returns whether the pair
-    // (and so every later one) overflows.  A pair that completes a word
-    // stores it.
-    __device__ __forceinline__ bool put(uint2 e0, uint2 e1) {
-        const uint32_t code = e0.x | (e1.x << e0.y);
-        const uint32_t len = e0.y + e1.y;
-        const uint32_t shift = pos & 31u;
-        const uint64_t placed = static_cast<uint64_t>(code) << shift;
-        const uint32_t new_word = word | static_cast<uint32_t>(placed);
-        const uint32_t after = pos + len;
-        const bool ok = after <= limit;
-        const bool completes = ok && shift + len >= 32u;
-        __builtin_amdgcn_raw_buffer_store_b32(new_word, out, completes ? row_off : kOutOfRange,
-                                              0, 0);
-        row_off += completes ? row_bytes : 0u;
-        word = ok ? (completes ? static_cast<uint32_t>(placed >> 32) : new_word) : word;
-        fits += ok ? 1u : 0u;
-        pos = after;
-        return !ok;
-    }
-
-    // Append a pair that is known to fit (its chunk passed fits_chunk): the
-    // same bits and stores as put() without the overflow bookkeeping; the
-    // chunk's caller adds its pairs to `fits` at the end.
-    __device__ __forceinline__ void put_fast(uint2 e0, uint2 e1) {
-        const uint32_t code = e0.x | (e1.x << e0.y);
-        const uint32_t len = e0.y + e1.y;
-        const uint32_t shift = pos & 31u;
-        const uint64_t placed = static_cast<uint64_t>(code) << shift;
-        const uint32_t new_word = word | static_cast<uint32_t>(placed);
-        const bool completes = shift + len >= 32u;
-        __builtin_amdgcn_raw_buffer_store_b32(new_word, out, completes ? row_off : kOutOfRange,
-                                              0, 0);
-        row_off += completes ? row_bytes : 0u;
-        word = completes ? static_cast<uint32_t>(placed >> 32) : new_word;
-        pos += len;
-    }
-
-    // Whether every pair of the next `steps` steps fits for every lane of the
-    // wave (a symbol's code is at most 16 bits: ESC of at most 8 bits and an
-    // 8-bit literal).  Wave-uniform.
-    __device__ __forceinline__ bool fits_chunk(int steps) const {
-        return __all(pos + 16u * static_cast<uint32_t>(steps) <= limit);
-    }
-
-    // After the last pair: the word being filled (the bits before the first
-    // pair that did not fit, for an overflowing stream), then zero words up to
-    // row W-1.
-    __device__ __forceinline__ void finish() {
-        for (; row_off < end_off; row_off += row_bytes) {
-            __builtin_amdgcn_raw_buffer_store_b32(word, out, row_off, 0, 0);
-            word = 0u;
-        }
-    }
-};
-
-// Encode-table entry as the kernel keeps it in LDS: {reversed code (<= 16
-// bits), code length}, 8 bytes, so one 8-byte read gives both without masks
-// (shifted tables: tables.py:53-67).
-__device__ __forceinline__ uint2 repack_encode_entry(uint32_t packed) {
-    return make_uint2(packed & 0xFFFFu, packed >> 20);
-}
-
-// Exponent bytes of a pair of BF16 results r (step s0 in bits 0..15, s0 + 1 in
-// bits 16..31): bytes 0 and 2 of r >> 7.  The shift is kept opaque so that
-// each encode-table address is one byte-selecting shift (SDWA) of it, where
-// the compiler would otherwise fold shift and mask into two ops per index.
-__device__ __forceinline__ uint32_t exponent_bytes(uint32_t r) {
-    uint32_t x = r >> 7;
-    asm("" : "+v"(x));
-    return x;
-}
-
-// The side byte of a high-half BF16 result in bits 16..23: the mantissa stays
-// in bits 16..22 and the sign comes down from bit 31 (one v_bfi_b32 after a
-// shift; the compiler otherwise builds it from three instructions).
-__device__ __forceinline__ uint32_t side_byte_at_16(uint32_t h) {
-    uint32_t out;
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(out) : "s"(0x007F0000u), "v"(h), "v"(h >> 8));
-    return out;
-}
+//
+// Each 8-step half is emitted (arithmetic, side bytes, codes) while the next
+// one is decoded; the two are independent, and scheduling barriers put a piece
+// of the emitting behind each of the decode's dependent lookups.
 
 struct UpdateIo {
     __amdgpu_buffer_rsrc_t side;       // A's side bytes (storage order)
@@ -448,411 +342,161 @@ struct UpdateIo {
 };
 
 // B words of the 16-step chunk at `first` (one 4-byte word per lane per step
-// pair, lane-pair layout), or zeros without memory traffic when !fetch.
+// pair, lane-pair layout), or zeros without memory traffic past the block's
+// last step.  A partial block's words are read by halves: one that straddles
+// the tensor's end would read as 0 whole.
+template <bool kFull>
 __device__ __forceinline__ void fetch_b_chunk(uint32_t (&bw)[kChunkSteps / 2],
                                               const UpdateIo &io, const LanePair &lp,
-                                              int64_t row_base, int first, bool fetch) {
-    const uint32_t mask2 = static_cast<uint32_t>((row_base + first) & 254) * 2u;
+                                              int64_t row_base, int first, int S) {
+    const uint32_t base = first < S
+                              ? lp.offset2 ^ static_cast<uint32_t>((row_base + first) & 254) * 2u
+                              : kOutOfRange;   // stays out of range under the XOR
 #pragma unroll
-    for (int j = 0; j < kChunkSteps; j += 2)
-        bw[j / 2] = __builtin_amdgcn_raw_buffer_load_b32(
-            io.other, fetch ? (lp.offset2 ^ mask2 ^ static_cast<uint32_t>(2 * j)) : kOutOfRange,
-            (first + j) * kLanes * 2, 0);
-}
-
-// Results r0/r1 (BF16 in the high halves) of this lane's pair at `step`: side
-// bytes replace A's in the wave's slice, the exponent bytes are encoded, and
-// an overflowing pair's exponent bytes go to the exponent array (positions
-// past the tensor's end are outside its resource and are dropped).
-__device__ __forceinline__ void emit_pair(StreamWriter &writer, const uint2 *enc,
-                                          uint8_t *slice, int s0, uint32_t h0, uint32_t h1,
-                                          bool v0, bool v1, uint32_t off0, const UpdateIo &io) {
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    slice[s0 * kWave + lane] = static_cast<uint8_t>(side_byte_at_16(h0) >> 16);
-    slice[(s0 + 1) * kWave + lane] = static_cast<uint8_t>(side_byte_at_16(h1) >> 16);
-    const uint32_t x0 = high_exponent_byte(h0);
-    const uint32_t x1 = high_exponent_byte(h1);
-    // Positions past the logical end carry no code (encode.py:255-256).
-    const uint2 e0 = v0 ? enc[x0] : make_uint2(0u, 0u);
-    const uint2 e1 = v1 ? enc[x1] : make_uint2(0u, 0u);
-    const bool over = writer.put(e0, e1);
-    const uint32_t exp_off = over ? off0 : kOutOfRange;
-    __builtin_amdgcn_raw_buffer_store_b8(x0, io.exponents, exp_off, 0, 0);
-    __builtin_amdgcn_raw_buffer_store_b8(x1, io.exponents, exp_off + kLanes, 0, 0);
-}
-
-// Chunks [c_begin, c_end) with one overlay variant of A.  On entry side_next
-// and b_next hold chunk c_begin's A side bytes and B words (B only for full
-// blocks); on exit those of chunk c_end.  kForm < 0: the operation is chosen at
-// run time (the last, partial block).
-template <bool kFull, Overlay kOverlay, int S, int kForm>
-__device__ __forceinline__ void update_chunks(UpdateCursor &cursor, const LaneOverlay &lane,
-                                              const uint8_t *tail_lds, uint8_t *slice,
-                                              SideChunk &side_next,
-                                              uint32_t (&b_next)[kChunkSteps / 2],
-                                              StreamWriter &writer, const uint2 *enc,
-                                              const UpdateIo &io, const LanePair &lp,
-                                              int64_t row_base, uint32_t valid_in_block,
-                                              int c_begin, int c_end, const OpParams &p) {
-    const uint32_t voffset = side_fetch_offset();
-#pragma unroll 1
-    for (int c = c_begin; c < c_end; c += kChunkSteps) {
-        store_side_chunk(slice, side_next);
-        uint32_t b_cur[kChunkSteps / 2];
-#pragma unroll
-        for (int k = 0; k < kChunkSteps / 2; ++k) b_cur[k] = b_next[k];
-        const bool more = c + kChunkSteps < S;
-        side_next = fetch_side_chunk(io.side, more ? voffset : kOutOfRange, c + kChunkSteps);
-        if (kFull) fetch_b_chunk(b_next, io, lp, row_base, c + kChunkSteps, more);
-        const uint32_t mask = static_cast<uint32_t>((row_base + c) & 254);
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            const int first = c + half * kHalfSteps;
-            uint32_t f[kHalfSteps];
-            decode_fields<kFull, kOverlay>(cursor, lane, tail_lds, first, row_base,
-                                           valid_in_block, f);
-#pragma unroll
-            for (int j = 0; j < kHalfSteps; j += 2) {
-                const int s0 = half * kHalfSteps + j;   // step within the chunk
-                const int step = c + s0;
-                // Logical offset (in the block) of this lane's element of row
-                // `step`; row step+1 shares the swizzle mask, and the chunk's
-                // first row is a multiple of 16, so the mask of row c+s0 is
-                // mask ^ s0.
-                const uint32_t off0 = static_cast<uint32_t>(step) * kLanes
-                    + (threadIdx.x ^ mask ^ static_cast<uint32_t>(s0));
-                const float a0 = __uint_as_float(join_float(f[j], side_byte(slice, s0)));
-                const float a1 = __uint_as_float(join_float(f[j + 1], side_byte(slice, s0 + 1)));
-                uint32_t h0, h1;
-                bool v0 = true, v1 = true;
-                if (kFull) {
-                    float b0, b1;
-                    pair_unpack16(lp, b_cur[s0 / 2], b0, b1);
-                    h0 = round_bf16_high(apply_form<kForm>(p, a0, b0));
-                    h1 = round_bf16_high(apply_form<kForm>(p, a1, b1));
-                } else {
-                    v0 = off0 < valid_in_block;
-                    v1 = off0 + kLanes < valid_in_block;
-                    // Outside the tensor the resource returns 0.
-                    const uint32_t b0 = __builtin_amdgcn_raw_buffer_load_b16(io.other, off0 * 2, 0, 0);
-                    const uint32_t b1 = __builtin_amdgcn_raw_buffer_load_b16(
-                        io.other, (off0 + kLanes) * 2, 0, 0);
-                    // Padding positions hold 0 (side byte 0, no code).
-                    h0 = v0 ? apply_op_f(p, a0, bf16_to_float(b0)) << 16 : 0u;
-                    h1 = v1 ? apply_op_f(p, a1, bf16_to_float(b1)) << 16 : 0u;
-                }
-                emit_pair(writer, enc, slice, s0, h0, h1, v0, v1, off0, io);
-            }
+    for (int j = 0; j < kChunkSteps; j += 2) {
+        const uint32_t off = base ^ static_cast<uint32_t>(2 * j);
+        const int row = (first + j) * kLanes * 2;
+        if (kFull) {
+            bw[j / 2] = __builtin_amdgcn_raw_buffer_load_b32(io.other, off, row, 0);
+        } else {
+            const uint32_t low = __builtin_amdgcn_raw_buffer_load_b16(io.other, off, row, 0);
+            const uint32_t high = __builtin_amdgcn_raw_buffer_load_b16(io.other, off + 2u, row, 0);
+            bw[j / 2] = low | (high << 16);
         }
-        // The slice now holds the chunk's result side bytes.
-        const uint4 q = reinterpret_cast<const uint4 *>(slice)[threadIdx.x & (kWave - 1)];
-        store_b128<kSideStore>(q, io.side_out, voffset + static_cast<uint32_t>(c) * kLanes);
     }
 }
 
-// ---- the pipelined full-block path
-//
-// Each stream's decode is a chain of dependent LDS lookups, and only about 2.7
-// waves per SIMD exist at C4's 688 blocks, so the chains' latency used to go
-// unhidden.  Here the wave interleaves, pair by pair, the arithmetic and
-// encoding of one 8-step half with the decoding of the next half: the two are
-// independent, so the compiler fills each lookup's wait with the other half's
-// work.  A chunk in which no lane of the wave can overflow (fits_chunk) also
-// skips the overflow bookkeeping and the exponent stores, which only overflow
-// rows need.
-
-// The arithmetic and encoding of this lane's pair at chunk step s0 (absolute
-// step c + s0), in stages that the caller interleaves with a decode's lookups:
-// A's entries f0/f1 joined with A's side bytes from the slice and B from the
-// pair's word (emit_operands), the operation, BF16 rounding, the result's side
-// bytes into the slice and the encode-table reads (emit_result), and the
-// exponent codes into the stream (emit_codes).
-struct EmitState {
-    uint32_t sa0, sa1;   // A's side bytes
-    float b0, b1;        // B
-    uint32_t r;          // the results' BF16 bits (step s0 low, s0 + 1 high)
-    uint2 e0, e1;        // their encode entries
-};
-
-__device__ __forceinline__ void emit_operands(EmitState &st, const uint8_t *slice, int s0,
-                                              uint32_t b_word, const LanePair &lp) {
-    st.sa0 = side_byte(slice, s0);
-    st.sa1 = side_byte(slice, s0 + 1);
-    pair_unpack16(lp, b_word, st.b0, st.b1);
-}
-
-template <int kForm>
-__device__ __forceinline__ void emit_result(EmitState &st, const uint2 *enc, uint8_t *slice,
-                                            int s0, uint32_t f0, uint32_t f1,
-                                            const OpParams &p) {
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    const float a0 = __uint_as_float(join_float(f0, st.sa0));
-    const float a1 = __uint_as_float(join_float(f1, st.sa1));
-    const uint32_t r = round_pair_bf16(apply_form<kForm>(p, a0, st.b0),
-                                       apply_form<kForm>(p, a1, st.b1));
-    // Side bytes: the mantissa and, from r >> 8, the sign of each half.
-    const uint32_t sign_down = r >> 8;
-    uint32_t side0, side1;
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(side0) : "s"(0x7Fu), "v"(r), "v"(sign_down));
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(side1) : "s"(0x007F0000u), "v"(r), "v"(sign_down));
-    slice[s0 * kWave + lane] = static_cast<uint8_t>(side0);
-    slice[(s0 + 1) * kWave + lane] = static_cast<uint8_t>(side1 >> 16);
-    const uint32_t x = exponent_bytes(r);
-    st.e0 = enc[x & 255u];
-    st.e1 = enc[(x >> 16) & 255u];
-    st.r = r;
-}
-
-template <bool kFast>
-__device__ __forceinline__ void emit_codes(const EmitState &st, StreamWriter &writer,
-                                           uint32_t off0, const UpdateIo &io) {
-    if (kFast) {
-        writer.put_fast(st.e0, st.e1);
-    } else {
-        const bool over = writer.put(st.e0, st.e1);
-        const uint32_t exp_off = over ? off0 : kOutOfRange;
-        __builtin_amdgcn_raw_buffer_store_b8(st.r >> 7, io.exponents, exp_off, 0, 0);
-        __builtin_amdgcn_raw_buffer_store_b8(st.r >> 23, io.exponents, exp_off + kLanes, 0, 0);
-    }
-}
-
-// One half (8 steps from chunk step `half` * 8) of emitting f, interleaved pair
-// by pair with decoding the 8 steps from `next_step` into g (kDecode).  The
-// order within a pair is pinned with scheduling barriers: each of the
-// decode's two dependent lookups is followed by independent emit work that
-// fills its latency.
-template <Overlay kOverlay, int kForm, bool kFast, bool kDecode, class Cursor>
-__device__ __forceinline__ void pipelined_half(Cursor &cursor, const LaneOverlay &lane,
-                                               const uint8_t *tail_lds, uint8_t *slice,
-                                               StreamWriter &writer, const uint2 *enc,
-                                               const UpdateIo &io, const LanePair &lp,
-                                               const OpParams &p, int64_t row_base, int c,
-                                               int half, uint32_t mask,
-                                               const uint32_t (&b_cur)[kChunkSteps / 2],
-                                               const uint32_t (&f)[kHalfSteps],
-                                               uint32_t (&g)[kHalfSteps], int next_step) {
-#pragma unroll
-    for (int j = 0; j < kHalfSteps; j += 2) {
-        const int s0 = half * kHalfSteps + j;
-        const uint32_t off0 = static_cast<uint32_t>(c + s0) * kLanes
-            + (threadIdx.x ^ mask ^ static_cast<uint32_t>(s0));
-        EmitState st;
-        uint32_t bits = 0, t0 = 0, t1 = 0;
-        if (kDecode) cursor.first_lookup(bits, t0);
-        __builtin_amdgcn_sched_barrier(0);
-        emit_operands(st, slice, s0, b_cur[s0 / 2], lp);
-        __builtin_amdgcn_sched_barrier(0);
-        if (kDecode) t1 = cursor.second_lookup(bits, t0);
-        __builtin_amdgcn_sched_barrier(0);
-        emit_result<kForm>(st, enc, slice, s0, f[j], f[j + 1], p);
-        __builtin_amdgcn_sched_barrier(0);
-        if (kDecode) {
-            uint32_t sum = cursor.resolve(bits, t0, t1);
-            if (kOverlay != kNoOverlay) {
-                overlay_pair<kOverlay == kLdsOverlay, typename Cursor::TablesT>(lane, tail_lds,
-                                                                                next_step + j,
-                                                                                t0, t1);
-                sum = (t0 + t1) & 127u;
-            }
-            cursor.advance(sum);
-            g[j] = t0;
-            g[j + 1] = t1;
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        emit_codes<kFast>(st, writer, off0, io);
-    }
-}
-
-// Both halves of the chunk at c; f holds the first half's entries on entry and
-// the next chunk's first half's on exit (when kDecodeNext).
-template <Overlay kOverlay, int kForm, bool kFast, bool kDecodeNext, class Cursor>
-__device__ __forceinline__ void pipelined_chunk(Cursor &cursor, const LaneOverlay &lane,
-                                                const uint8_t *tail_lds, uint8_t *slice,
-                                                StreamWriter &writer, const uint2 *enc,
-                                                const UpdateIo &io, const LanePair &lp,
-                                                const OpParams &p, int64_t row_base, int c,
-                                                uint32_t mask,
-                                                const uint32_t (&b_cur)[kChunkSteps / 2],
-                                                uint32_t (&f)[kHalfSteps]) {
-    uint32_t g[kHalfSteps];
-    pipelined_half<kOverlay, kForm, kFast, true>(cursor, lane, tail_lds, slice, writer, enc, io,
-                                                 lp, p, row_base, c, 0, mask, b_cur, f, g,
-                                                 c + kHalfSteps);
-    pipelined_half<kOverlay, kForm, kFast, kDecodeNext>(cursor, lane, tail_lds, slice, writer,
-                                                        enc, io, lp, p, row_base, c, 1, mask,
-                                                        b_cur, g, f, c + kChunkSteps);
-    if (kFast) writer.fits += kChunkSteps / 2;
-}
-
-// Chunks [c_begin, c_end) of a full block with one overlay variant of A; as
-// update_chunks<true, ...>.  The segment's first half is decoded before the
-// loop and its last chunk decodes nothing further, so no step outside the
-// segment is decoded with this variant.
-// A's side bytes and B's words of the next two chunks (fetched two chunks
-// ahead: one chunk of work is shorter than HBM's latency under load).
+// A's side bytes and B's words of one chunk.
 struct Prefetch {
-    SideChunk side1, side2;
-    uint32_t b1[kChunkSteps / 2], b2[kChunkSteps / 2];
+    SideChunk side;
+    uint32_t b[kChunkSteps / 2];
 };
 
-// One chunk at c using the side bytes and B words in (side, b) -- the copy of
-// the two that holds chunk c -- and refilling them with chunk c + 32.  The two
-// copies alternate, so a chunk's loads are issued two chunks before use and no
-// register copy of an in-flight load (which would wait for it) is made.
-template <Overlay kOverlay, int S, int kForm, class Cursor>
-__device__ __forceinline__ void pipelined_step(Cursor &cursor, const LaneOverlay &lane,
-                                               const uint8_t *tail_lds, uint8_t *slice,
-                                               SideChunk &side, uint32_t (&b)[kChunkSteps / 2],
-                                               StreamWriter &writer, const uint2 *enc,
-                                               const UpdateIo &io, const LanePair &lp,
-                                               int64_t row_base, int c, int c_end,
-                                               const OpParams &p, uint32_t (&f)[kHalfSteps]) {
-    const uint32_t voffset = side_fetch_offset();
-    store_side_chunk(slice, side);
-    uint32_t b_cur[kChunkSteps / 2];
+// What a lane walks a block with.
+struct UpdateWalk {
+    QuadCursor cursor;
+    LaneOverlay lane;
+    const uint8_t *tail_lds;
+    StreamWriter writer;
+    const uint2 *enc;
+    uint8_t *slice;        // this wave's 16 rows of side bytes
+    OpParams p;
+    int64_t row_base;
+    uint32_t valid;        // elements of the block inside the tensor
+};
+
+// Emit the half at `first` (f: its entries; rows: its side bytes in the slice;
+// bw: its B words) while decoding the next half into f.  kFast: every code is
+// known to fit.
+template <bool kFull, int kForm, bool kFast>
+__device__ __forceinline__ void update_half(UpdateWalk &u, uint32_t (&f)[kHalfSteps],
+                                            uint8_t *rows, const uint32_t *bw, const UpdateIo &io,
+                                            const LanePair &lp, int first, int S) {
+    const uint32_t mask = static_cast<uint32_t>((u.row_base + first) & 254);
+    Quad q;
+    u.cursor.first(q);
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t sa[kHalfSteps];
+    float b[kHalfSteps], x[kHalfSteps];
 #pragma unroll
-    for (int k = 0; k < kChunkSteps / 2; ++k) b_cur[k] = b[k];
-    const bool more = c + 2 * kChunkSteps < S;
-    side = fetch_side_chunk(io.side, more ? voffset : kOutOfRange, c + 2 * kChunkSteps);
-    fetch_b_chunk(b, io, lp, row_base, c + 2 * kChunkSteps, more);
-    const uint32_t mask = static_cast<uint32_t>((row_base + c) & 254);
-    const bool fast = writer.fits_chunk(kChunkSteps);
-    const bool next = c + kChunkSteps < c_end;
-#define LCT_CHUNK(FAST, NEXT)                                                                 \
-    pipelined_chunk<kOverlay, kForm, FAST, NEXT>(cursor, lane, tail_lds, slice, writer, enc, \
-                                                 io, lp, p, row_base, c, mask, b_cur, f)
-    if (fast) {
-        if (next) LCT_CHUNK(true, true);
-        else LCT_CHUNK(true, false);
+    for (int k = 0; k < kHalfSteps; ++k) sa[k] = side_byte(rows, k);
+#pragma unroll
+    for (int p = 0; p < kHalfSteps / 2; ++p) pair_unpack16(lp, bw[p], b[2 * p], b[2 * p + 1]);
+    __builtin_amdgcn_sched_barrier(0);
+    u.cursor.second(q);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < kHalfSteps; ++k)
+        x[k] = apply_form<kForm>(u.p, __uint_as_float(join_float(f[k], sa[k])), b[k]);
+    __builtin_amdgcn_sched_barrier(0);
+    u.cursor.third(q);
+    __builtin_amdgcn_sched_barrier(0);
+    HalfEmit h;
+    round_half<kFull>(h, x, first, mask, u.valid);
+    store_half_sides(h, rows);
+    __builtin_amdgcn_sched_barrier(0);
+    u.cursor.fourth(q);
+    __builtin_amdgcn_sched_barrier(0);
+    look_up_quad<kFull>(h, u.enc, 0, first, mask, u.valid);
+    __builtin_amdgcn_sched_barrier(0);
+    u.cursor.finish(q, f);
+    u.cursor.first(q);
+    __builtin_amdgcn_sched_barrier(0);
+    look_up_quad<kFull>(h, u.enc, 1, first, mask, u.valid);
+    __builtin_amdgcn_sched_barrier(0);
+    u.cursor.second(q);
+    __builtin_amdgcn_sched_barrier(0);
+    if (kFast) {
+        const QuadCodes c0(h, 0), c1(h, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        u.cursor.third(q);
+        __builtin_amdgcn_sched_barrier(0);
+        put_half(c0, c1, u.writer);
     } else {
-        if (next) LCT_CHUNK(false, true);
-        else LCT_CHUNK(false, false);
+        u.cursor.third(q);
+        put_half_by_pairs(h, u.writer, first, mask, io.exponents);
     }
-#undef LCT_CHUNK
+    __builtin_amdgcn_sched_barrier(0);
+    u.cursor.fourth(q);
+    u.cursor.finish(q, f + 4);
+    overlay_half(u.lane, u.tail_lds, first + kHalfSteps, S, f);
+}
+
+// The 16-step chunk at c, whose side bytes and B words pf holds; refills pf
+// with chunk c + 32's.
+template <bool kFull, int kForm>
+__device__ __forceinline__ void update_chunk(UpdateWalk &u, uint32_t (&f)[kHalfSteps],
+                                             Prefetch &pf, const UpdateIo &io, const LanePair &lp,
+                                             int c, int S) {
+    const uint32_t voffset = side_fetch_offset();
+    store_side_chunk(u.slice, pf.side);
+    uint32_t bw[kChunkSteps / 2];
+#pragma unroll
+    for (int k = 0; k < kChunkSteps / 2; ++k) bw[k] = pf.b[k];
+    const int ahead = c + 2 * kChunkSteps;
+    pf.side = fetch_side_chunk(io.side, ahead < S ? voffset : kOutOfRange, ahead);
+    fetch_b_chunk<kFull>(pf.b, io, lp, u.row_base, ahead, S);
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        uint8_t *const rows = u.slice + half * kHalfSteps * kWave;
+        const uint32_t *const b = bw + half * kHalfSteps / 2;
+        const int first = c + half * kHalfSteps;
+        if (__builtin_expect(u.writer.fits_half(), 1))
+            update_half<kFull, kForm, true>(u, f, rows, b, io, lp, first, S);
+        else
+            update_half<kFull, kForm, false>(u, f, rows, b, io, lp, first, S);
+    }
     // The slice now holds the chunk's result side bytes.
-    const uint4 q = reinterpret_cast<const uint4 *>(slice)[threadIdx.x & (kWave - 1)];
+    const uint4 q = reinterpret_cast<const uint4 *>(u.slice)[threadIdx.x & (kWave - 1)];
     store_b128<kSideStore>(q, io.side_out, voffset + static_cast<uint32_t>(c) * kLanes);
 }
 
-// Chunks [c_begin, c_end); pf.side1/b1 hold chunk c_begin's data and
-// side2/b2 chunk c_begin + 16's.  On exit the same holds for c_end.
-template <Overlay kOverlay, int S, int kForm, class Cursor>
-__device__ __forceinline__ void update_chunks_pipelined(
-    Cursor &cursor, const LaneOverlay &lane, const uint8_t *tail_lds, uint8_t *slice,
-    Prefetch &pf, StreamWriter &writer, const uint2 *enc, const UpdateIo &io,
-    const LanePair &lp, int64_t row_base, int c_begin, int c_end, const OpParams &p) {
-    if (c_begin >= c_end) return;
-    uint32_t f[kHalfSteps];
-    decode_fields<true, kOverlay>(cursor, lane, tail_lds, c_begin, row_base, 0u, f);
-    int c = c_begin;
-#pragma unroll 1
-    for (; c + kChunkSteps < c_end; c += 2 * kChunkSteps) {
-        pipelined_step<kOverlay, S, kForm>(cursor, lane, tail_lds, slice, pf.side1, pf.b1,
-                                           writer, enc, io, lp, row_base, c, c_end, p, f);
-        pipelined_step<kOverlay, S, kForm>(cursor, lane, tail_lds, slice, pf.side2, pf.b2,
-                                           writer, enc, io, lp, row_base, c + kChunkSteps, c_end,
-                                           p, f);
-    }
-    if (c < c_end) {
-        pipelined_step<kOverlay, S, kForm>(cursor, lane, tail_lds, slice, pf.side1, pf.b1,
-                                           writer, enc, io, lp, row_base, c, c_end, p, f);
-        // An odd number of chunks: the next chunk's data is in the second copy.
-        // Swapping waits for its loads, once per block at most.
-        const SideChunk side = pf.side1;
-        pf.side1 = pf.side2;
-        pf.side2 = side;
-#pragma unroll
-        for (int k = 0; k < kChunkSteps / 2; ++k) {
-            const uint32_t b = pf.b1[k];
-            pf.b1[k] = pf.b2[k];
-            pf.b2[k] = b;
-        }
-    }
-}
-
-template <bool kFull, int S, int kForm>
-__device__ __forceinline__ void update_rows(UpdateCursor cursor, const LaneOverlay &lane,
-                                            const uint8_t *tail_lds, uint8_t *slice,
-                                            SideChunk side_next, StreamWriter &writer,
-                                            const uint2 *enc, const UpdateIo &io,
-                                            int64_t row_base, uint32_t valid_in_block,
-                                            const OpParams &p) {
+// A whole block.  Two copies of the prefetched data alternate, so a chunk's
+// loads are issued two chunks before use and no register copy of an in-flight
+// load (which would wait for it) is made.  The last half decodes eight symbols
+// past the block's end, which nothing uses.
+template <bool kFull, int kForm>
+__device__ __forceinline__ void update_rows(UpdateWalk &u, const SideChunk &first_side,
+                                            const UpdateIo &io, int S) {
     const LanePair lp;
-    const int split = min(S, lane.wave_start & ~(kChunkSteps - 1));
-    if (kFull) {
-        // Full blocks decode with the LDS-window cursor (the stage has two pad
-        // rows); the partial block keeps the register window.
-        UpdateWindow wc;
-        wc.init(cursor.stage, cursor.tb, cursor.pad_row, cursor.rare, cursor.center);
-        Prefetch pf;
-        pf.side1 = side_next;
-        pf.side2 = fetch_side_chunk(io.side, side_fetch_offset(), kChunkSteps);
-        fetch_b_chunk(pf.b1, io, lp, row_base, 0, true);
-        fetch_b_chunk(pf.b2, io, lp, row_base, kChunkSteps, true);
-        update_chunks_pipelined<kNoOverlay, S, kForm>(wc, lane, tail_lds, slice, pf, writer,
-                                                      enc, io, lp, row_base, 0, split, p);
-        if (split == S) return;
-        if (lane.lds)
-            update_chunks_pipelined<kLdsOverlay, S, kForm>(wc, lane, tail_lds, slice, pf,
-                                                           writer, enc, io, lp, row_base, split,
-                                                           S, p);
-        else
-            update_chunks_pipelined<kHbmOverlay, S, kForm>(wc, lane, tail_lds, slice, pf,
-                                                           writer, enc, io, lp, row_base, split,
-                                                           S, p);
-        return;
-    }
-    uint32_t b_next[kChunkSteps / 2];
-    update_chunks<kFull, kNoOverlay, S, kForm>(cursor, lane, tail_lds, slice, side_next, b_next,
-                                               writer, enc, io, lp, row_base, valid_in_block, 0,
-                                               split, p);
-    if (split == S) return;
-    if (lane.lds)
-        update_chunks<kFull, kLdsOverlay, S, kForm>(cursor, lane, tail_lds, slice, side_next,
-                                                    b_next, writer, enc, io, lp, row_base,
-                                                    valid_in_block, split, S, p);
-    else
-        update_chunks<kFull, kHbmOverlay, S, kForm>(cursor, lane, tail_lds, slice, side_next,
-                                                    b_next, writer, enc, io, lp, row_base,
-                                                    valid_in_block, split, S, p);
-}
-
-// Full blocks take the operation's form as a template parameter; the last,
-// partial block decides at run time.
-template <int S>
-__device__ __forceinline__ void update_block(int32_t form, bool full, const UpdateCursor &cursor,
-                                             const LaneOverlay &lane, const uint8_t *tail_lds,
-                                             uint8_t *slice, const SideChunk &side_next,
-                                             StreamWriter &writer, const uint2 *enc,
-                                             const UpdateIo &io, int64_t row_base,
-                                             uint32_t valid_in_block, const OpParams &p) {
-    if (!full) {
-        update_rows<false, S, -1>(cursor, lane, tail_lds, slice, side_next, writer, enc, io,
-                                  row_base, valid_in_block, p);
-        return;
-    }
-    switch (form) {
-    case kFormAxpy:
-        update_rows<true, S, kFormAxpy>(cursor, lane, tail_lds, slice, side_next, writer, enc, io,
-                                        row_base, valid_in_block, p);
-        break;
-    case kFormAxpby:
-        update_rows<true, S, kFormAxpby>(cursor, lane, tail_lds, slice, side_next, writer, enc,
-                                         io, row_base, valid_in_block, p);
-        break;
-    case kFormBxpa:
-        update_rows<true, S, kFormBxpa>(cursor, lane, tail_lds, slice, side_next, writer, enc, io,
-                                        row_base, valid_in_block, p);
-        break;
-    default:
-        update_rows<true, S, kFormMul>(cursor, lane, tail_lds, slice, side_next, writer, enc, io,
-                                       row_base, valid_in_block, p);
-        break;
+    Prefetch even, odd;
+    even.side = first_side;
+    odd.side = fetch_side_chunk(io.side, side_fetch_offset(), kChunkSteps);
+    fetch_b_chunk<kFull>(even.b, io, lp, u.row_base, 0, S);
+    fetch_b_chunk<kFull>(odd.b, io, lp, u.row_base, kChunkSteps, S);
+    uint32_t f[kHalfSteps];
+    u.cursor.quad(f);
+    u.cursor.quad(f + 4);
+    overlay_half(u.lane, u.tail_lds, 0, S, f);
+#pragma unroll 1
+    for (int c = 0; c < S; c += 2 * kChunkSteps) {
+        update_chunk<kFull, kForm>(u, f, even, io, lp, c, S);
+        update_chunk<kFull, kForm>(u, f, odd, io, lp, c + kChunkSteps, S);
     }
 }
 
 // Codec block `block` of one fused update (the single launch's blockIdx.x);
-// `stage`: the dynamic LDS, window_stage_bytes(W) (A's payload).
+// `stage`: the dynamic LDS, register_stage_bytes(W) (rows 3..W-1 of A's payload).
 template <bool kBooked>
 __device__ __forceinline__ void pointwise_encode_block(
     const OperandA &a, const uint16_t *__restrict__ other, const OpArgs &args,
@@ -863,7 +507,7 @@ __device__ __forceinline__ void pointwise_encode_block(
     uint8_t *__restrict__ extra_starts, int32_t *__restrict__ summaries,
     uint8_t *__restrict__ exponents, int64_t n_blocks, int64_t logical_numel, int S, int W,
     int rare, const KernelBookkeeping &bk, int64_t block, uint32_t *stage) {
-    __shared__ FloatDecodeTables tb;
+    __shared__ QuadTables tb;
     __shared__ uint2 enc[256];
     __shared__ int32_t scratch[kWavesPerBlock];
     __shared__ int32_t shared_center;
@@ -890,10 +534,11 @@ __device__ __forceinline__ void pointwise_encode_block(
     // The result's center from the sampler's partial sums.
     raw_encode[t] = base_encode[t];
     center_from_partials(partials, n_groups, &shared_center);
-    build_float_decode_tables(tb, a.shifted_decode);
+    build_quad_tables(tb, a.shifted_decode, rare);
     const int32_t a_center = a.center[0];
-    stage_payload(stage, a.encoded, n_blocks * kLanes, block, W);
-    stage[(W + 1) * kLanes + t] = 0u;   // the window cursor's second pad row
+    uint32_t words[kRegisterRows];
+    load_register_rows(a.encoded, n_blocks * kLanes, block, words);
+    stage_payload_rows(stage, a.encoded, n_blocks * kLanes, block, kRegisterRows, W);
     __syncthreads();   // center and raw encode table
     const int32_t center = shared_center;
     enc[t] = repack_encode_entry(static_cast<uint32_t>(raw_encode[byte_to_index(t, center)]));
@@ -912,27 +557,38 @@ __device__ __forceinline__ void pointwise_encode_block(
     wait_memory();
     __syncthreads();   // payload, tails and encode table visible; maps no longer read
 
-    UpdateCursor cursor;
-    cursor.init(stage + t, &tb, static_cast<uint32_t>(W), rare, a_center);
+    UpdateWalk u;
+    u.cursor.init(stage + t, &tb, static_cast<uint32_t>(W), rare, words, a_center);
+    u.lane = lane;
+    u.tail_lds = tail_lds;
     const uint32_t row_bytes = static_cast<uint32_t>(n_blocks * kLanes * 4);
-    StreamWriter writer{make_rsrc(encoded_out + block * kLanes,
-                                  static_cast<uint32_t>(W - 1) * row_bytes + kLanes * 4),
-                        row_bytes, static_cast<uint32_t>(t) * 4u,
-                        static_cast<uint32_t>(W) * row_bytes + static_cast<uint32_t>(t) * 4u,
-                        static_cast<uint32_t>(W) * 32u, 0u, 0u, 0u};
-    writer.keep_row_bytes_in_vgpr();
-    uint8_t *slice = side_slices[t / kWave];
+    u.writer = StreamWriter{make_rsrc(encoded_out + block * kLanes,
+                                      static_cast<uint32_t>(W - 1) * row_bytes + kLanes * 4),
+                            row_bytes, static_cast<uint32_t>(t) * 4u,
+                            static_cast<uint32_t>(W) * row_bytes + static_cast<uint32_t>(t) * 4u,
+                            static_cast<uint32_t>(W) * 32u, 0u, 0u, 0u};
+    u.writer.keep_row_bytes_in_vgpr();
+    u.enc = enc;
+    u.slice = side_slices[t / kWave];
+    u.p = p;
+    u.row_base = row_base;
+    u.valid = valid;
     const bool full = valid == block_elems;
-    const int32_t form = form_of(args.op, args.alpha_is_one, args.beta_is_one);
-    if (S == 128)
-        update_block<128>(form, full, cursor, lane, tail_lds, slice, first, writer, enc, io,
-                          row_base, valid, p);
-    else
-        update_block<256>(form, full, cursor, lane, tail_lds, slice, first, writer, enc, io,
-                          row_base, valid, p);
-    writer.finish();
-    const bool overflow = writer.overflowed();
-    const int32_t extra = writer.extra_start();
+#define LCT_ROWS(FORM)                              \
+    do {                                            \
+        if (full) update_rows<true, FORM>(u, first, io, S);  \
+        else update_rows<false, FORM>(u, first, io, S);      \
+    } while (0)
+    switch (form_of(args.op, args.alpha_is_one, args.beta_is_one)) {
+    case kFormAxpy: LCT_ROWS(kFormAxpy); break;
+    case kFormAxpby: LCT_ROWS(kFormAxpby); break;
+    case kFormBxpa: LCT_ROWS(kFormBxpa); break;
+    default: LCT_ROWS(kFormMul); break;
+    }
+#undef LCT_ROWS
+    u.writer.finish();
+    const bool overflow = u.writer.overflowed();
+    const int32_t extra = u.writer.extra_start();
     extra_starts[block * kLanes + t] = static_cast<uint8_t>(overflow ? extra : 255);
     // Streams from bit 20 (at most 256), tail bytes in bits 0..19 (at most
     // 256 x 256): one block scan.
@@ -951,7 +607,7 @@ __global__ __launch_bounds__(kLanes) void pointwise_encode_kernel(
     uint8_t *__restrict__ extra_starts, int32_t *__restrict__ summaries,
     uint8_t *__restrict__ exponents, int64_t n_blocks, int64_t logical_numel, int S, int W,
     int rare, KernelBookkeeping bk) {
-    extern __shared__ uint32_t stage[];   // A's payload: window_stage_bytes(W)
+    extern __shared__ uint32_t stage[];   // register_stage_bytes(W)
     pointwise_encode_block<kBooked>(a, other, args, partials, n_groups, base_encode, base_decode,
                                     center_out, shifted_decode_out, side_out, encoded_out,
                                     extra_starts, summaries, exponents, n_blocks, logical_numel,
@@ -1043,7 +699,7 @@ struct UpdateEncodeBatch {
 };
 
 __global__ __launch_bounds__(kLanes) void pointwise_encode_batch_kernel(UpdateEncodeBatch batch) {
-    extern __shared__ uint32_t stage[];   // window_stage_bytes(max W), or the free list
+    extern __shared__ uint32_t stage[];   // register_stage_bytes(max W), or the free list
     const int32_t w = static_cast<int32_t>(blockIdx.x);
     int j = 0;
     for (int k = 1; k < batch.n_jobs; ++k)
@@ -1210,301 +866,131 @@ __device__ __forceinline__ void store_half_side(uint8_t *half, u32x2 q) {
     reinterpret_cast<u32x2 *>(half)[threadIdx.x & (kWave - 1)] = q;
 }
 
-// Halves [c_begin, c_end) (steps, multiples of 8) with one overlay variant for
-// both operands (tails read from HBM).  On entry side_a/side_b hold half
-// c_begin's side bytes of A and B.
-template <bool kFull, Overlay kOverlay, int S>
-__device__ __forceinline__ void dual_halves(UpdateCursor &ca, const LaneOverlay &lane_a,
-                                            UpdateCursor &cb, const LaneOverlay &lane_b,
-                                            uint8_t *slice, u32x2 &side_a, u32x2 &side_b,
-                                            __amdgpu_buffer_rsrc_t b_side, StreamWriter &writer,
-                                            const uint2 *enc, const UpdateIo &io,
-                                            int64_t row_base, uint32_t valid_in_block,
-                                            int c_begin, int c_end, float alpha) {
-    const uint32_t voffset = half_side_offset();
-    uint8_t *half_a = slice;
-    uint8_t *half_b = slice + kHalfSlice;
-#pragma unroll 1
-    for (int c = c_begin; c < c_end; c += kHalfSteps) {
-        store_half_side(half_a, side_a);
-        store_half_side(half_b, side_b);
-        const bool more = c + kHalfSteps < S;
-        side_a = fetch_half_side(io.side, more ? voffset : kOutOfRange, c + kHalfSteps);
-        side_b = fetch_half_side(b_side, more ? voffset : kOutOfRange, c + kHalfSteps);
-        // c is a multiple of 8 and the block's first row one of S, so the
-        // swizzle mask of row c + j (j < 8 even) is mask ^ j.
-        const uint32_t mask = static_cast<uint32_t>((row_base + c) & 254);
-        uint32_t fa[kHalfSteps], fb[kHalfSteps];
-        decode_fields<kFull, kOverlay>(ca, lane_a, nullptr, c, row_base, valid_in_block, fa);
-        decode_fields<kFull, kOverlay>(cb, lane_b, nullptr, c, row_base, valid_in_block, fb);
-#pragma unroll
-        for (int j = 0; j < kHalfSteps; j += 2) {
-            const int step = c + j;
-            const uint32_t off0 = static_cast<uint32_t>(step) * kLanes
-                + (threadIdx.x ^ mask ^ static_cast<uint32_t>(j));
-            const bool v0 = kFull || off0 < valid_in_block;
-            const bool v1 = kFull || off0 + kLanes < valid_in_block;
-            const float a0 = __uint_as_float(join_float(fa[j], side_byte(half_a, j)));
-            const float a1 = __uint_as_float(join_float(fa[j + 1], side_byte(half_a, j + 1)));
-            const float b0 = __uint_as_float(join_float(fb[j], side_byte(half_b, j)));
-            const float b1 = __uint_as_float(join_float(fb[j + 1], side_byte(half_b, j + 1)));
-            // Padding positions hold 0 (side byte 0, no code).
-            const uint32_t h0 = v0 ? round_bf16_high(__builtin_fmaf(a0, alpha, b0)) : 0u;
-            const uint32_t h1 = v1 ? round_bf16_high(__builtin_fmaf(a1, alpha, b1)) : 0u;
-            emit_pair(writer, enc, half_a, j, h0, h1, v0, v1, off0, io);
-        }
-        // A's half now holds the result's side bytes.
-        const u32x2 q = reinterpret_cast<const u32x2 *>(half_a)[threadIdx.x & (kWave - 1)];
-        __builtin_amdgcn_raw_buffer_store_b64(q, io.side_out, voffset, c * kLanes, kSideStore);
-    }
-}
-
-// ---- the pipelined full-block path of the two-operand kernel: as for one
-// operand, the arithmetic and encoding of one 8-step half are interleaved pair
-// by pair with decoding the next half, here of both operands (two independent
-// lookup chains), and chunks that cannot overflow use the lean writer.
-
-struct DualEmit {
-    uint32_t sa0, sa1, sb0, sb1;   // A's and B's side bytes
-    uint32_t r;                    // the results' BF16 bits (step s0 low, s0 + 1 high)
-    uint2 e0, e1;                  // their encode entries
+// What a lane walks a block of two operands with (tails read from HBM).
+struct DualWalk {
+    QuadCursor ca, cb;
+    LaneOverlay lane_a, lane_b;
+    StreamWriter writer;
+    const uint2 *enc;
+    uint8_t *half_a, *half_b;   // this wave's 8 rows of side bytes of each operand
+    float alpha;
+    int64_t row_base;
+    uint32_t valid;
 };
 
-__device__ __forceinline__ void dual_emit_operands(DualEmit &st, const uint8_t *half_a,
-                                                   const uint8_t *half_b, int j) {
-    st.sa0 = side_byte(half_a, j);
-    st.sa1 = side_byte(half_a, j + 1);
-    st.sb0 = side_byte(half_b, j);
-    st.sb1 = side_byte(half_b, j + 1);
-}
-
-// fma(a, alpha, b) (pointwise_scalar_dual.py:226) rounded to BF16, the result's
-// side bytes over A's in the half slice and the encode-table reads.
-__device__ __forceinline__ void dual_emit_result(DualEmit &st, const uint2 *enc, uint8_t *half_a,
-                                                 int j, uint32_t fa0, uint32_t fa1, uint32_t fb0,
-                                                 uint32_t fb1, float alpha) {
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    const float a0 = __uint_as_float(join_float(fa0, st.sa0));
-    const float a1 = __uint_as_float(join_float(fa1, st.sa1));
-    const float b0 = __uint_as_float(join_float(fb0, st.sb0));
-    const float b1 = __uint_as_float(join_float(fb1, st.sb1));
-    const uint32_t r = round_pair_bf16(__builtin_fmaf(a0, alpha, b0), __builtin_fmaf(a1, alpha, b1));
-    const uint32_t sign_down = r >> 8;
-    uint32_t side0, side1;
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(side0) : "s"(0x7Fu), "v"(r), "v"(sign_down));
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(side1) : "s"(0x007F0000u), "v"(r), "v"(sign_down));
-    half_a[j * kWave + lane] = static_cast<uint8_t>(side0);
-    half_a[(j + 1) * kWave + lane] = static_cast<uint8_t>(side1 >> 16);
-    const uint32_t x = exponent_bytes(r);
-    st.e0 = enc[x & 255u];
-    st.e1 = enc[(x >> 16) & 255u];
-    st.r = r;
-}
-
-// One operand's staged lookups for the pair at `step` (kOverlay: tails from HBM).
-template <Overlay kOverlay>
-__device__ __forceinline__ void finish_pair(UpdateCursor &cursor, const LaneOverlay &lane,
-                                            int step, uint32_t bits, uint32_t &t0,
-                                            uint32_t &t1) {
-    uint32_t sum = cursor.resolve(bits, t0, t1);
-    if (kOverlay != kNoOverlay) {
-        overlay_pair<false, FloatDecodeTables>(lane, nullptr, step, t0, t1);
-        sum = (t0 + t1) & 127u;
-    }
-    cursor.advance(sum);
-}
-
-// The half at c: emit from fa/fb while decoding the half at c + 8 into them
-// (kDecode).  Within a pair, each lookup's latency is filled with emit work
-// that does not depend on it: the first lookups with the operation on the
-// pair being emitted, the second lookups with its codes.  The side bytes of
-// the next pair are read a pair ahead.
-template <Overlay kOverlay, bool kFast, bool kDecode>
-__device__ __forceinline__ void dual_pipelined_half(UpdateCursor &ca, const LaneOverlay &lane_a,
-                                                    UpdateCursor &cb, const LaneOverlay &lane_b,
-                                                    uint8_t *half_a, const uint8_t *half_b,
-                                                    StreamWriter &writer, const uint2 *enc,
-                                                    const UpdateIo &io, int c, uint32_t mask,
-                                                    float alpha, uint32_t (&fa)[kHalfSteps],
-                                                    uint32_t (&fb)[kHalfSteps]) {
-    uint32_t ga[kHalfSteps], gb[kHalfSteps];
-    DualEmit st;
-    dual_emit_operands(st, half_a, half_b, 0);
+// Emit the half at `first` from fa/fb while decoding the next half of both
+// operands into them; the two operands' lookups are independent of each other
+// and of the emitting.  kFast: every code is known to fit.
+template <bool kFull, bool kFast>
+__device__ __forceinline__ void dual_half_emit(DualWalk &u, uint32_t (&fa)[kHalfSteps],
+                                               uint32_t (&fb)[kHalfSteps], const UpdateIo &io,
+                                               int first, int S) {
+    const uint32_t mask = static_cast<uint32_t>((u.row_base + first) & 254);
+    Quad qa, qb;
+    u.ca.first(qa);
+    u.cb.first(qb);
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t sa[kHalfSteps], sb[kHalfSteps];
 #pragma unroll
-    for (int j = 0; j < kHalfSteps; j += 2) {
-        const uint32_t off0 = static_cast<uint32_t>(c + j) * kLanes
-            + (threadIdx.x ^ mask ^ static_cast<uint32_t>(j));
-        uint32_t bits_a = 0, ta0 = 0, ta1 = 0, bits_b = 0, tb0 = 0, tb1 = 0;
-        if (kDecode) {
-            ca.first_lookup(bits_a, ta0);
-            cb.first_lookup(bits_b, tb0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        dual_emit_result(st, enc, half_a, j, fa[j], fa[j + 1], fb[j], fb[j + 1], alpha);
-        DualEmit next = st;
-        if (j + 2 < kHalfSteps) dual_emit_operands(next, half_a, half_b, j + 2);
-        __builtin_amdgcn_sched_barrier(0);
-        if (kDecode) {
-            ta1 = ca.second_lookup(bits_a, ta0);
-            tb1 = cb.second_lookup(bits_b, tb0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        if (kFast) {
-            writer.put_fast(st.e0, st.e1);
-        } else {
-            const bool over = writer.put(st.e0, st.e1);
-            const uint32_t exp_off = over ? off0 : kOutOfRange;
-            __builtin_amdgcn_raw_buffer_store_b8(st.r >> 7, io.exponents, exp_off, 0, 0);
-            __builtin_amdgcn_raw_buffer_store_b8(st.r >> 23, io.exponents, exp_off + kLanes, 0, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        if (kDecode) {
-            finish_pair<kOverlay>(ca, lane_a, c + kHalfSteps + j, bits_a, ta0, ta1);
-            finish_pair<kOverlay>(cb, lane_b, c + kHalfSteps + j, bits_b, tb0, tb1);
-            ga[j] = ta0;
-            ga[j + 1] = ta1;
-            gb[j] = tb0;
-            gb[j + 1] = tb1;
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        st = next;
+    for (int k = 0; k < kHalfSteps; ++k) {
+        sa[k] = side_byte(u.half_a, k);
+        sb[k] = side_byte(u.half_b, k);
     }
-    if (kDecode) {
+    __builtin_amdgcn_sched_barrier(0);
+    u.ca.second(qa);
+    u.cb.second(qb);
+    __builtin_amdgcn_sched_barrier(0);
+    // fma(a, alpha, b) (pointwise_scalar_dual.py:226).
+    float x[kHalfSteps];
 #pragma unroll
-        for (int k = 0; k < kHalfSteps; ++k) {
-            fa[k] = ga[k];
-            fb[k] = gb[k];
-        }
-    }
-    if (kFast) writer.fits += kHalfSteps / 2;
-}
-
-// A's and B's side bytes of the next kDualDepth halves: fetched that many
-// halves ahead (one half of work is far shorter than HBM's latency under
-// load), in copies that rotate, so no register copy of an in-flight load
-// (which would wait for it) is made.  Copy 0 holds the half being started.
-constexpr int kDualDepth = 2;
-
-struct DualPrefetch {
-    u32x2 a[kDualDepth], b[kDualDepth];
-
-    // After k halves: copy k becomes copy 0 (waits for those loads; once per
-    // overlay segment at most).
-    __device__ __forceinline__ void rotate(int k) {
-        u32x2 ta[kDualDepth], tb[kDualDepth];
-#pragma unroll
-        for (int i = 0; i < kDualDepth; ++i) {
-            ta[i] = a[(i + k) % kDualDepth];
-            tb[i] = b[(i + k) % kDualDepth];
-        }
-#pragma unroll
-        for (int i = 0; i < kDualDepth; ++i) {
-            a[i] = ta[i];
-            b[i] = tb[i];
-        }
-    }
-};
-
-// The half at c using the side bytes in (side_a, side_b) -- the copy holding
-// half c -- and refilling them with half c + 8 * kDualDepth.
-template <Overlay kOverlay, int S>
-__device__ __forceinline__ void dual_half_step(
-    UpdateCursor &ca, const LaneOverlay &lane_a, UpdateCursor &cb, const LaneOverlay &lane_b,
-    uint8_t *slice, u32x2 &side_a, u32x2 &side_b, __amdgpu_buffer_rsrc_t b_side,
-    StreamWriter &writer, const uint2 *enc, const UpdateIo &io, int64_t row_base, int c,
-    int c_end, float alpha, uint32_t (&fa)[kHalfSteps], uint32_t (&fb)[kHalfSteps]) {
-    const uint32_t voffset = half_side_offset();
-    uint8_t *half_a = slice;
-    uint8_t *half_b = slice + kHalfSlice;
-    store_half_side(half_a, side_a);
-    store_half_side(half_b, side_b);
-    const int ahead = c + kDualDepth * kHalfSteps;
-    const bool more = ahead < S;
-    side_a = fetch_half_side(io.side, more ? voffset : kOutOfRange, ahead);
-    side_b = fetch_half_side(b_side, more ? voffset : kOutOfRange, ahead);
-    const uint32_t mask = static_cast<uint32_t>((row_base + c) & 254);
-    const bool fast = writer.fits_chunk(kHalfSteps);
-    const bool next = c + kHalfSteps < c_end;
-#define LCT_HALF(FAST, NEXT)                                                                   \
-    dual_pipelined_half<kOverlay, FAST, NEXT>(ca, lane_a, cb, lane_b, half_a, half_b, writer, \
-                                              enc, io, c, mask, alpha, fa, fb)
-    if (fast) {
-        if (next) LCT_HALF(true, true);
-        else LCT_HALF(true, false);
+    for (int k = 0; k < kHalfSteps; ++k)
+        x[k] = __builtin_fmaf(__uint_as_float(join_float(fa[k], sa[k])), u.alpha,
+                              __uint_as_float(join_float(fb[k], sb[k])));
+    __builtin_amdgcn_sched_barrier(0);
+    u.ca.third(qa);
+    u.cb.third(qb);
+    __builtin_amdgcn_sched_barrier(0);
+    HalfEmit h;
+    round_half<kFull>(h, x, first, mask, u.valid);
+    store_half_sides(h, u.half_a);
+    __builtin_amdgcn_sched_barrier(0);
+    u.ca.fourth(qa);
+    u.cb.fourth(qb);
+    __builtin_amdgcn_sched_barrier(0);
+    look_up_quad<kFull>(h, u.enc, 0, first, mask, u.valid);
+    __builtin_amdgcn_sched_barrier(0);
+    u.ca.finish(qa, fa);
+    u.cb.finish(qb, fb);
+    u.ca.first(qa);
+    u.cb.first(qb);
+    __builtin_amdgcn_sched_barrier(0);
+    look_up_quad<kFull>(h, u.enc, 1, first, mask, u.valid);
+    __builtin_amdgcn_sched_barrier(0);
+    u.ca.second(qa);
+    u.cb.second(qb);
+    __builtin_amdgcn_sched_barrier(0);
+    if (kFast) {
+        const QuadCodes c0(h, 0), c1(h, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        u.ca.third(qa);
+        u.cb.third(qb);
+        __builtin_amdgcn_sched_barrier(0);
+        put_half(c0, c1, u.writer);
     } else {
-        if (next) LCT_HALF(false, true);
-        else LCT_HALF(false, false);
+        u.ca.third(qa);
+        u.cb.third(qb);
+        put_half_by_pairs(h, u.writer, first, mask, io.exponents);
     }
-#undef LCT_HALF
+    __builtin_amdgcn_sched_barrier(0);
+    u.ca.fourth(qa);
+    u.cb.fourth(qb);
+    u.ca.finish(qa, fa + 4);
+    u.cb.finish(qb, fb + 4);
+    overlay_half(u.lane_a, nullptr, first + kHalfSteps, S, fa);
+    overlay_half(u.lane_b, nullptr, first + kHalfSteps, S, fb);
+}
+
+// The half at `first`, whose side bytes come in side_a/side_b; refills them with
+// those of the half at first + 16 (two halves ahead: one half of work is far
+// shorter than HBM's latency under load).
+template <bool kFull>
+__device__ __forceinline__ void dual_half(DualWalk &u, uint32_t (&fa)[kHalfSteps],
+                                          uint32_t (&fb)[kHalfSteps], u32x2 &side_a,
+                                          u32x2 &side_b, const UpdateIo &io, int first, int S) {
+    const uint32_t voffset = half_side_offset();
+    store_half_side(u.half_a, side_a);
+    store_half_side(u.half_b, side_b);
+    const int ahead = first + 2 * kHalfSteps;
+    side_a = fetch_half_side(io.side, ahead < S ? voffset : kOutOfRange, ahead);
+    side_b = fetch_half_side(io.other, ahead < S ? voffset : kOutOfRange, ahead);
+    if (__builtin_expect(u.writer.fits_half(), 1))
+        dual_half_emit<kFull, true>(u, fa, fb, io, first, S);
+    else
+        dual_half_emit<kFull, false>(u, fa, fb, io, first, S);
     // A's half now holds the result's side bytes.
-    const u32x2 q = reinterpret_cast<const u32x2 *>(half_a)[threadIdx.x & (kWave - 1)];
-    __builtin_amdgcn_raw_buffer_store_b64(q, io.side_out, voffset, c * kLanes, kSideStore);
+    const u32x2 q = reinterpret_cast<const u32x2 *>(u.half_a)[threadIdx.x & (kWave - 1)];
+    __builtin_amdgcn_raw_buffer_store_b64(q, io.side_out, voffset, first * kLanes, kSideStore);
 }
 
-// Halves [c_begin, c_end) of a full block with one overlay variant of both
-// operands (tails from HBM); as dual_halves<true, ...>.  On entry pf's copy i
-// holds half c_begin + 8i; on exit the same holds for c_end.
-template <Overlay kOverlay, int S>
-__device__ __forceinline__ void dual_halves_pipelined(
-    UpdateCursor &ca, const LaneOverlay &lane_a, UpdateCursor &cb, const LaneOverlay &lane_b,
-    uint8_t *slice, DualPrefetch &pf, __amdgpu_buffer_rsrc_t b_side, StreamWriter &writer,
-    const uint2 *enc, const UpdateIo &io, int64_t row_base, int c_begin, int c_end,
-    float alpha) {
-    if (c_begin >= c_end) return;
+// A whole block, with two copies of the prefetched side bytes as update_rows
+// (io.other: B's side bytes).
+template <bool kFull>
+__device__ __forceinline__ void dual_rows(DualWalk &u, u32x2 side_a, u32x2 side_b,
+                                          const UpdateIo &io, int S) {
+    u32x2 next_a = fetch_half_side(io.side, half_side_offset(), kHalfSteps);
+    u32x2 next_b = fetch_half_side(io.other, half_side_offset(), kHalfSteps);
     uint32_t fa[kHalfSteps], fb[kHalfSteps];
-    decode_fields<true, kOverlay>(ca, lane_a, nullptr, c_begin, row_base, 0u, fa);
-    decode_fields<true, kOverlay>(cb, lane_b, nullptr, c_begin, row_base, 0u, fb);
-    int c = c_begin;
+    u.ca.quad(fa);
+    u.cb.quad(fb);
+    u.ca.quad(fa + 4);
+    u.cb.quad(fb + 4);
+    overlay_half(u.lane_a, nullptr, 0, S, fa);
+    overlay_half(u.lane_b, nullptr, 0, S, fb);
 #pragma unroll 1
-    for (; c + (kDualDepth - 1) * kHalfSteps < c_end; c += kDualDepth * kHalfSteps) {
-#pragma unroll
-        for (int k = 0; k < kDualDepth; ++k)
-            dual_half_step<kOverlay, S>(ca, lane_a, cb, lane_b, slice, pf.a[k], pf.b[k], b_side,
-                                        writer, enc, io, row_base, c + k * kHalfSteps, c_end,
-                                        alpha, fa, fb);
+    for (int c = 0; c < S; c += 2 * kHalfSteps) {
+        dual_half<kFull>(u, fa, fb, side_a, side_b, io, c, S);
+        dual_half<kFull>(u, fa, fb, next_a, next_b, io, c + kHalfSteps, S);
     }
-    // Fewer than kDualDepth halves left.
-    const int left = (c_end - c) / kHalfSteps;
-#pragma unroll
-    for (int k = 0; k < kDualDepth - 1; ++k)
-        if (k < left)
-            dual_half_step<kOverlay, S>(ca, lane_a, cb, lane_b, slice, pf.a[k], pf.b[k], b_side,
-                                        writer, enc, io, row_base, c + k * kHalfSteps, c_end,
-                                        alpha, fa, fb);
-    if (left == 1) pf.rotate(1);
-    else if (left == 2) pf.rotate(2);
-    else if (left == 3) pf.rotate(3);
-}
-
-template <bool kFull, int S>
-__device__ __forceinline__ void dual_rows(UpdateCursor ca, const LaneOverlay &lane_a,
-                                          UpdateCursor cb, const LaneOverlay &lane_b,
-                                          uint8_t *slice, u32x2 side_a, u32x2 side_b,
-                                          __amdgpu_buffer_rsrc_t b_side, StreamWriter &writer,
-                                          const uint2 *enc, const UpdateIo &io,
-                                          int64_t row_base, uint32_t valid_in_block, float alpha) {
-    const int split = min(S, min(lane_a.wave_start, lane_b.wave_start) & ~(kHalfSteps - 1));
-    if (kFull) {
-        DualPrefetch pf;
-        pf.a[0] = side_a;
-        pf.b[0] = side_b;
-#pragma unroll
-        for (int k = 1; k < kDualDepth; ++k) {
-            pf.a[k] = fetch_half_side(io.side, half_side_offset(), k * kHalfSteps);
-            pf.b[k] = fetch_half_side(b_side, half_side_offset(), k * kHalfSteps);
-        }
-        dual_halves_pipelined<kNoOverlay, S>(ca, lane_a, cb, lane_b, slice, pf, b_side, writer,
-                                             enc, io, row_base, 0, split, alpha);
-        dual_halves_pipelined<kHbmOverlay, S>(ca, lane_a, cb, lane_b, slice, pf, b_side, writer,
-                                              enc, io, row_base, split, S, alpha);
-        return;
-    }
-    dual_halves<kFull, kNoOverlay, S>(ca, lane_a, cb, lane_b, slice, side_a, side_b, b_side,
-                                      writer, enc, io, row_base, valid_in_block, 0, split, alpha);
-    if (split < S)
-        dual_halves<kFull, kHbmOverlay, S>(ca, lane_a, cb, lane_b, slice, side_a, side_b, b_side,
-                                           writer, enc, io, row_base, valid_in_block, split, S,
-                                           alpha);
 }
 
 template <bool kBooked>
@@ -1518,7 +1004,7 @@ __global__ __launch_bounds__(kLanes) void dual_encode_kernel(
     uint8_t *__restrict__ exponents, int64_t n_blocks, int64_t logical_numel, int S, int W,
     int rare, KernelBookkeeping bk) {
     extern __shared__ uint32_t stages[];   // A's rows 3..W-1, then B's
-    __shared__ FloatDecodeTables tba, tbb;
+    __shared__ QuadTables tba, tbb;
     __shared__ uint2 enc[256];
     __shared__ int32_t scratch[kWavesPerBlock];
     __shared__ int32_t shared_center[2];   // center, and whether its samples failed to arrive
@@ -1560,12 +1046,11 @@ __global__ __launch_bounds__(kLanes) void dual_encode_kernel(
     const uint32_t valid = remaining < block_elems ? static_cast<uint32_t>(remaining) : block_elems;
     UpdateIo io;
     io.side = make_rsrc(a.side + logical_base, block_elems);
-    io.other = make_rsrc(nullptr, 0u);
+    io.other = make_rsrc(b.side + logical_base, block_elems);   // B's side bytes
     io.side_out = make_rsrc(side_out + logical_base, block_elems);
     io.exponents = make_rsrc(exponents + logical_base, valid);
-    const __amdgpu_buffer_rsrc_t b_side = make_rsrc(b.side + logical_base, block_elems);
     const u32x2 first_a = fetch_half_side(io.side, half_side_offset(), 0);
-    const u32x2 first_b = fetch_half_side(b_side, half_side_offset(), 0);
+    const u32x2 first_b = fetch_half_side(io.other, half_side_offset(), 0);
     // Loads the prologue needs later, issued now so that they share one round
     // trip with the tables' loads instead of following its barriers.
     const OverlayHead head_a = load_overlay_head(a.ov, a.has_overlay != 0, block, n_blocks);
@@ -1584,8 +1069,8 @@ __global__ __launch_bounds__(kLanes) void dual_encode_kernel(
         center_from_partials(partials, n_groups, shared_center);
         if (t == 0) shared_center[1] = 0;
     }
-    build_float_decode_tables(tba, a.shifted_decode);
-    build_float_decode_tables(tbb, b.shifted_decode);
+    build_quad_tables(tba, a.shifted_decode, rare);
+    build_quad_tables(tbb, b.shifted_decode, rare);
     const int32_t a_center = a.center[0], b_center = b.center[0];
     stage_payload_rows(stage_a, a.encoded, n_streams, block, kRegisterRows, W);
     stage_payload_rows(stage_b, b.encoded, n_streams, block, kRegisterRows, W);
@@ -1606,34 +1091,31 @@ __global__ __launch_bounds__(kLanes) void dual_encode_kernel(
     wait_memory();
     __syncthreads();   // payloads and encode table visible; maps no longer read
 
-    UpdateCursor ca, cb;
-    ca.init_registers(stage_a + t, &tba, static_cast<uint32_t>(W), rare, wa[0], wa[1], wa[2],
-                      a_center);
-    cb.init_registers(stage_b + t, &tbb, static_cast<uint32_t>(W), rare, wb[0], wb[1], wb[2],
-                      b_center);
+    DualWalk u;
+    u.ca.init(stage_a + t, &tba, static_cast<uint32_t>(W), rare, wa, a_center);
+    u.cb.init(stage_b + t, &tbb, static_cast<uint32_t>(W), rare, wb, b_center);
+    u.lane_a = lane_a;
+    u.lane_b = lane_b;
     const uint32_t row_bytes = static_cast<uint32_t>(n_streams * 4);
-    StreamWriter writer{make_rsrc(encoded_out + block * kLanes,
-                                  static_cast<uint32_t>(W - 1) * row_bytes + kLanes * 4),
-                        row_bytes, static_cast<uint32_t>(t) * 4u,
-                        static_cast<uint32_t>(W) * row_bytes + static_cast<uint32_t>(t) * 4u,
-                        static_cast<uint32_t>(W) * 32u, 0u, 0u, 0u};
-    writer.keep_row_bytes_in_vgpr();
-    uint8_t *slice = slices[t / kWave];
-    const bool full = valid == block_elems;
-#define LCT_DUAL_ROWS(FULL, SS)                                                                \
-    dual_rows<FULL, SS>(ca, lane_a, cb, lane_b, slice, first_a, first_b, b_side, writer, enc,  \
-                        io, row_base, valid, alpha_value)
-    if (S == 128) {
-        if (full) LCT_DUAL_ROWS(true, 128);
-        else LCT_DUAL_ROWS(false, 128);
-    } else {
-        if (full) LCT_DUAL_ROWS(true, 256);
-        else LCT_DUAL_ROWS(false, 256);
-    }
-#undef LCT_DUAL_ROWS
-    writer.finish();
-    const bool overflow = writer.overflowed();
-    const int32_t extra = writer.extra_start();
+    u.writer = StreamWriter{make_rsrc(encoded_out + block * kLanes,
+                                      static_cast<uint32_t>(W - 1) * row_bytes + kLanes * 4),
+                            row_bytes, static_cast<uint32_t>(t) * 4u,
+                            static_cast<uint32_t>(W) * row_bytes + static_cast<uint32_t>(t) * 4u,
+                            static_cast<uint32_t>(W) * 32u, 0u, 0u, 0u};
+    u.writer.keep_row_bytes_in_vgpr();
+    u.enc = enc;
+    u.half_a = slices[t / kWave];
+    u.half_b = u.half_a + kHalfSlice;
+    u.alpha = alpha_value;
+    u.row_base = row_base;
+    u.valid = valid;
+    if (valid == block_elems)
+        dual_rows<true>(u, first_a, first_b, io, S);
+    else
+        dual_rows<false>(u, first_a, first_b, io, S);
+    u.writer.finish();
+    const bool overflow = u.writer.overflowed();
+    const int32_t extra = u.writer.extra_start();
     extra_starts[block * kLanes + t] = static_cast<uint8_t>(overflow ? extra : 255);
     // Streams from bit 20 (at most 256), tail bytes in bits 0..19 (at most
     // 256 x 256): one block scan.
@@ -1779,7 +1261,7 @@ int32_t launch_pointwise_encode(
                      overflow ? *overflow : lct_overflow{}, overflow != nullptr};
     const OpArgs args{alpha, beta, op, alpha_is_one, beta_is_one};
     const int32_t groups = sample_groups(sample_size);
-    size_t lds = static_cast<size_t>(window_stage_bytes(g.fixed_words));
+    size_t lds = static_cast<size_t>(register_stage_bytes(g.fixed_words));
     KernelBookkeeping bk;
     if (int32_t e = prepare_bookkeeping(bookkeeping, n_blocks, bk, lds)) return e;
     const auto kernel = bk.control != nullptr ? pointwise_encode_kernel<true>
@@ -2090,7 +1572,7 @@ extern "C" int32_t lct_pointwise_update_batch(
     hipLaunchKernelGGL(pointwise_sample_batch_kernel, dim3(static_cast<uint32_t>(groups)),
                        dim3(kSampleGroup), sample_lds, stream, sample);
     if (hipError_t e = hipGetLastError()) return static_cast<int32_t>(e);
-    const size_t encode_lds = std::max(static_cast<size_t>(window_stage_bytes(max_words)),
+    const size_t encode_lds = std::max(static_cast<size_t>(register_stage_bytes(max_words)),
                                        static_cast<size_t>(max_free_regions) * 8);
     if (hipError_t e = reserve_dynamic_lds(
             reinterpret_cast<const void *>(&pointwise_encode_batch_kernel), encode_lds))
