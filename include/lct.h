@@ -747,6 +747,40 @@ int32_t lct_set_wait_limits(int32_t lock_polls, int32_t ready_polls);
 #define LCT_DECODER_COMPACT 2
 int32_t lct_set_decoder(int32_t mode);
 
+/* ---- dense steps of the compressed layers (LCT/components/layers.py:16-71,
+ * 179-222, which leaves their fusion to torch.compile), one or two launches
+ * each.  Matrices are contiguous BF16 (passed as void *); arithmetic is FP32.
+ *
+ * lct_relu_square: relu = max(z, 0) (NaN kept, -0 gives 0), square =
+ * bf16(relu^2).  lct_relu_square_backward: grad = bf16(grad * bf16(2 relu))
+ * where relu is not zero, else 0, in place, and square = bf16(relu^2).
+ * Pointers 16-byte aligned, any n up to 2^38. */
+int32_t lct_relu_square(const void *z, void *relu, void *square, int64_t n, hipStream_t stream);
+int32_t lct_relu_square_backward(const void *relu, void *grad, void *square, int64_t n,
+                                 hipStream_t stream);
+
+/* out[c] = bf16(sum of g[r][c] over the rows), stored as BF16 (out_bf16 != 0)
+ * or FP32.  cols: a multiple of 8 up to 2^20; g 16-byte aligned.  partials:
+ * FP32 working array of partial_floats >= cols values; up to 128 cols of them
+ * are used, and the split of the rows, hence the order of the sum, follows
+ * from how many there are. */
+int32_t lct_column_sum(const void *g, int64_t rows, int32_t cols, float *partials,
+                       int64_t partial_floats, void *out, int32_t out_bf16, hipStream_t stream);
+
+/* RMSNorm over rows of cols values (a multiple of 4 up to 4096; 8-byte
+ * aligned): rstd[r] = 1 / sqrt(mean(x^2) + eps), y = bf16(x * rstd * gain).
+ * The gain (cols values, BF16 if gain_bf16 != 0, else FP32 and then 16-byte
+ * aligned) is rounded to BF16.  lct_rms_norm_backward: grad_x, grad_gain (rounded to BF16; stored as
+ * BF16 or FP32) and, where normalized is not NULL, y again.  partials:
+ * partial_floats >= cols working values, up to 512 cols of them used. */
+int32_t lct_rms_norm(const void *x, const void *gain, int32_t gain_bf16, void *y, float *rstd,
+                     int64_t rows, int32_t cols, float eps, hipStream_t stream);
+int32_t lct_rms_norm_backward(const void *grad, const void *x, const float *rstd,
+                              const void *gain, int32_t gain_bf16, void *grad_x,
+                              void *normalized, float *partials, int64_t partial_floats,
+                              void *grad_gain, int32_t grad_gain_bf16, int64_t rows,
+                              int32_t cols, hipStream_t stream);
+
 /* ---- attainable HBM bandwidth with the codec kernels' access shape (16-byte
  * non-temporal buffer accesses, `workgroups` workgroups of 256 threads each
  * walking 16 KiB passes).  kind 0: copy src -> dst (src_bytes = dst_bytes);

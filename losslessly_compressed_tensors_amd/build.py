@@ -28,6 +28,7 @@ SOURCES = [
     "pointwise.hip",
     "update.hip",
     "noalloc.hip",
+    "layers.hip",
     "bandwidth.hip",
 ]
 

@@ -1,8 +1,9 @@
 """Autograd layers that keep what backward needs compressed.
 
 Same operators, argument order and gradients as ``LCT/components/layers.py``:
-each ``torch.autograd.Function`` runs its dense math on the device's libraries
-(hipBLASLt GEMMs, ATen's fused RMSNorm and flash attention), and between
+each ``torch.autograd.Function`` runs its products and attention on the
+device's libraries (hipBLASLt, flash attention) and the steps between them in
+one pass each (``kernels/fused.py``; ATen where that does not apply), and between
 forward and backward holds its saved activation as a ``CompressedTensor``
 (when ``compressed`` and the tensor has at least ``min_elements`` elements),
 decoding and freeing it once in backward.  Weights may be ``LCTTensor``s
@@ -22,6 +23,7 @@ from torch import Tensor, nn
 
 from ..LCTensor import LCTTensor
 from ..codec.decode import decode_batch
+from ..kernels import fused
 from ..operations import compress, compress_batch, decompress
 from .dist_configs import act_dist, act_relu_dist, weight_dist
 from .ops import rms_norm, rms_norm_backward
@@ -164,6 +166,28 @@ def _normalized(x: Tensor, rstd: Tensor, gain: Tensor) -> Tensor:
     return (x.float() * rstd * gain.float()).to(x.dtype).reshape(-1, x.shape[-1])
 
 
+def _norm(x: Tensor, gain: Tensor) -> tuple[Tensor, Tensor]:
+    """RMSNorm with the gain rounded to ``x``'s dtype."""
+    result = fused.rms_norm(x, gain)
+    return rms_norm(x, gain.to(x.dtype)) if result is None else result
+
+
+def _norm_backward(grad: Tensor, x: Tensor, rstd: Tensor, norm_weight: Tensor):
+    """The gradients of :func:`_norm` and its output again, as a matrix."""
+    result = fused.rms_norm_backward(grad, x, rstd, norm_weight, norm_weight.dtype, True)
+    if result is not None:
+        return result
+    gain = norm_weight.to(x.dtype)
+    grad_x, grad_gain = rms_norm_backward(grad, x, rstd, gain)
+    return grad_x, grad_gain.to(norm_weight.dtype), _normalized(x, rstd, gain)
+
+
+def _bias_grad(g: Tensor, dtype: torch.dtype) -> Tensor:
+    """``g``'s column sums in the bias's dtype."""
+    result = fused.column_sum(g, dtype)
+    return g.sum(0).to(dtype) if result is None else result
+
+
 class RMSLinear(torch.autograd.Function):
     """RMSNorm then one projection; saves only the norm input
     (LCT/components/layers.py:22-71)."""
@@ -172,7 +196,7 @@ class RMSLinear(torch.autograd.Function):
     def forward(ctx, x, weight, norm_weight, bias, buffer=None, compressed=False,
                 distribution=None, min_elements=65536, decoded_weight=None):
         W = dense_weight(weight) if decoded_weight is None else decoded_weight
-        normalized, rstd = rms_norm(x, norm_weight.to(x.dtype))
+        normalized, rstd = _norm(x, norm_weight)
         output = F.linear(normalized, W, bias.to(x.dtype))
         del normalized
         ctx.saved = _SavedActivation(x, compressed and x.numel() >= min_elements,
@@ -187,13 +211,12 @@ class RMSLinear(torch.autograd.Function):
         x = ctx.saved.take()
         ctx.saved = None
         W = dense_weight(weight)
-        gain = norm_weight.to(x.dtype)
         g = grad.reshape(-1, grad.shape[-1])
-        grad_x, grad_gain = rms_norm_backward((g @ W).reshape(x.shape), x, rstd, gain)
-        grad_weight = g.T @ _normalized(x, rstd, gain)
-        grad_bias = g.sum(0).to(ctx.bias_dtype)
-        return (grad_x, grad_weight, grad_gain.to(norm_weight.dtype), grad_bias,
-                None, None, None, None, None)
+        grad_x, grad_gain, normalized = _norm_backward((g @ W).reshape(x.shape), x, rstd,
+                                                       norm_weight)
+        grad_weight = g.T @ normalized
+        grad_bias = _bias_grad(g, ctx.bias_dtype)
+        return grad_x, grad_weight, grad_gain, grad_bias, None, None, None, None, None
 
 
 class _RMSNormQKV(torch.autograd.Function):
@@ -205,7 +228,7 @@ class _RMSNormQKV(torch.autograd.Function):
                 q_weight, q_bias, k_weight, k_bias, v_weight, v_bias):
         weights = (q_weight, k_weight, v_weight)
         biases = (q_bias, k_bias, v_bias)
-        normalized, rstd = rms_norm(x, norm_weight.to(x.dtype))
+        normalized, rstd = _norm(x, norm_weight)
         outputs = tuple(F.linear(normalized, dense_weight(w), b.to(x.dtype))
                         for w, b in zip(weights, biases))
         del normalized
@@ -219,20 +242,19 @@ class _RMSNormQKV(torch.autograd.Function):
         norm_weight, rstd, *weights = ctx.saved_tensors
         x = ctx.saved.take()
         ctx.saved = None
-        gain = norm_weight.to(x.dtype)
         grads = [g.reshape(-1, g.shape[-1]) for g in (grad_q, grad_k, grad_v)]
         dense = [dense_weight(w) for w in weights]
         # V first, then K, then Q, accumulated in place.
         grad_normalized = grads[2] @ dense[2]
         grad_normalized.add_(grads[1] @ dense[1])
         grad_normalized.add_(grads[0] @ dense[0])
-        grad_x, grad_gain = rms_norm_backward(grad_normalized.reshape(x.shape), x, rstd, gain)
+        grad_x, grad_gain, normalized = _norm_backward(grad_normalized.reshape(x.shape), x, rstd,
+                                                       norm_weight)
         del grad_normalized, dense
-        normalized = _normalized(x, rstd, gain)
         parameter_grads = []
         for g, bias_dtype in zip(grads, ctx.bias_dtypes):
-            parameter_grads += [g.T @ normalized, g.sum(0).to(bias_dtype)]
-        return (grad_x, grad_gain.to(norm_weight.dtype), None, None, None, *parameter_grads)
+            parameter_grads += [g.T @ normalized, _bias_grad(g, bias_dtype)]
+        return (grad_x, grad_gain, None, None, None, *parameter_grads)
 
 
 def rms_norm_qkv(x, norm_weight, q, k, v, *, buffer=None, compressed=False,
@@ -275,8 +297,13 @@ class Relu2Linear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, z, weight, bias, buffer=None, compressed=False,
                 distribution=None, min_elements=65536):
-        relu = z.relu()
-        output = F.linear(relu.square(), dense_weight(weight), bias.to(z.dtype))
+        both = fused.relu_square(z)
+        if both is None:
+            relu = z.relu()
+            both = relu, relu.square()
+        relu, square = both
+        output = F.linear(square, dense_weight(weight), bias.to(z.dtype))
+        del both, square
         ctx.saved = _SavedActivation(relu, compressed and z.numel() >= min_elements,
                                      distribution or act_relu_dist, buffer)
         ctx.save_for_backward(weight)
@@ -290,10 +317,13 @@ class Relu2Linear(torch.autograd.Function):
         ctx.saved = None
         g = grad.reshape(-1, grad.shape[-1])
         grad_z = (g @ dense_weight(weight)).reshape(relu.shape)
-        grad_z.mul_(2 * relu)
-        grad_z.masked_fill_(relu == 0, 0)
-        grad_weight = g.T @ relu.square().reshape(-1, relu.shape[-1])
-        grad_bias = g.sum(0).to(ctx.bias_dtype)
+        square = fused.relu_square_backward(grad_z, relu)
+        if square is None:
+            grad_z.mul_(2 * relu)
+            grad_z.masked_fill_(relu == 0, 0)
+            square = relu.square()
+        grad_weight = g.T @ square.reshape(-1, relu.shape[-1])
+        grad_bias = _bias_grad(g, ctx.bias_dtype)
         return grad_z, grad_weight, grad_bias, None, None, None, None
 
 
@@ -344,7 +374,7 @@ class FlashAttention(torch.autograd.Function):
         g = grad_output.reshape(-1, grad_output.shape[-1])
         hidden = out.transpose(1, 2).reshape(-1, heads * head_dim)
         grad_weight = g.T @ hidden
-        grad_bias = g.sum(0).to(ctx.bias_dtype)
+        grad_bias = _bias_grad(g, ctx.bias_dtype)
         grad_attention = (g @ dense_weight(ctx.weight)).reshape(
             batch, length, heads, head_dim).transpose(1, 2)
         lse, cum_q, cum_k, max_q, max_k, seed, offset = ctx.auxiliary

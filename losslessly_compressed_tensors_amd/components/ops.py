@@ -3,7 +3,8 @@
 Same contract as ``LCT/components/ops.py:6-44``: ``rms_norm(x, gain)`` returns
 ``(y, rstd)`` over the last dimension, with the reciprocal RMS in FP32 and
 ``y`` in ``x``'s dtype; ``rms_norm_backward(grad, x, rstd, gain)`` returns
-``(grad_x, grad_gain)`` (``grad_gain`` is ``None`` without a gain).  Both run
+``(grad_x, grad_gain)`` (``grad_gain`` is ``None`` without a gain).  BF16 rows
+that fit a wave's registers run ``csrc/layers.hip`` (``kernels/fused.py``), others
 ATen's fused device kernels, so the dense regions around the codec need no
 tracing compiler.  ``rms_norm`` is differentiable through ``rms_norm_backward``.
 """
@@ -12,13 +13,23 @@ from __future__ import annotations
 import torch
 from torch import Tensor
 
+from ..kernels import fused
+
 
 def _forward(x: Tensor, gain: Tensor | None) -> tuple[Tensor, Tensor]:
+    if gain is not None and gain.dtype == x.dtype:
+        result = fused.rms_norm(x, gain)
+        if result is not None:
+            return result
     return torch.ops.aten._fused_rms_norm.default(x, [x.shape[-1]], gain, None)
 
 
 def rms_norm_backward(grad: Tensor, x: Tensor, rstd: Tensor,
                       gain: Tensor | None) -> tuple[Tensor, Tensor | None]:
+    if gain is not None and gain.dtype == x.dtype:
+        result = fused.rms_norm_backward(grad, x, rstd, gain, gain.dtype, False)
+        if result is not None:
+            return result[:2]
     return torch.ops.aten._fused_rms_norm_backward.default(
         grad, x, [x.shape[-1]], rstd, gain, [True, gain is not None])
 

@@ -1,0 +1,128 @@
+"""One-pass device kernels for the dense steps of the compressed layers.
+
+Each function is an expression of ``components/layers.py`` or
+``components/ops.py`` as one or two launches of ``csrc/layers.hip``, for the
+tensors that ``native`` accepts; the callers keep ATen's expression for the
+others (host tensors, other types, strided views, and wherever autograd,
+tracing or a transform has to see the operations).
+"""
+from __future__ import annotations
+
+import torch
+from torch import Tensor
+from torch.autograd import forward_ad
+
+from . import hip
+
+_PLAIN = (Tensor, torch.nn.Parameter)
+_MAX_COLUMNS = 4096
+# Row groups of the partial sums: the most that lct_column_sum and
+# lct_rms_norm_backward make.
+_COLUMN_GROUPS = 128
+_NORM_GROUPS = 512
+# ATen's reduction and cast take 10.5 us up to 128 rows of 768 and 14.3 at 1024,
+# the two launches here 12 at any of these: the line lies where both sides were
+# measured to have crossed.
+_MIN_SUM_ROWS = 1024
+
+
+def native(*tensors: Tensor) -> bool:
+    """Whether the kernels may read ``tensors`` directly: plain non-empty
+    contiguous device tensors of the current device, with no autograd graph,
+    forward-mode level, transform, dispatch mode, autocast or tracing that
+    would have to see the operations."""
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+            or forward_ad._current_level >= 0 or torch.is_autocast_enabled("cuda")):
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if (type(t) not in _PLAIN or not t.is_cuda or not t.is_contiguous() or t.numel() == 0
+                or (grad and t.requires_grad) or torch._C._functorch.is_functorch_wrapped_tensor(t)
+                or t.data_ptr() & 15 or t.is_conj() or t.is_neg()):
+            return False
+    return tensors[0].get_device() == torch._C._cuda_getDevice()
+
+
+def _stream(tensor: Tensor) -> int:
+    return torch._C._cuda_getCurrentRawStream(tensor.get_device())
+
+
+def relu_square(z: Tensor):
+    """``(relu(z), relu(z)^2)``, or None."""
+    if z.dtype != torch.bfloat16 or not native(z):
+        return None
+    relu, square = torch.empty_like(z), torch.empty_like(z)
+    hip.call("lct_relu_square", z.data_ptr(), relu.data_ptr(), square.data_ptr(), z.numel(),
+             _stream(z))
+    return relu, square
+
+
+def relu_square_backward(grad: Tensor, relu: Tensor):
+    """``grad`` becomes the gradient of ``relu(z)^2`` from its own, in place;
+    returns ``relu^2``, or None (``grad`` is then as it was)."""
+    if (grad.dtype != torch.bfloat16 or relu.dtype != torch.bfloat16 or grad.shape != relu.shape
+            or not native(grad, relu)):
+        return None
+    square = torch.empty_like(relu)
+    hip.call("lct_relu_square_backward", relu.data_ptr(), grad.data_ptr(), square.data_ptr(),
+             relu.numel(), _stream(relu))
+    return square
+
+
+def column_sum(g: Tensor, dtype: torch.dtype):
+    """``g.sum(0).to(dtype)`` of a matrix, or None."""
+    if (g.dtype != torch.bfloat16 or dtype not in (torch.bfloat16, torch.float32) or g.ndim != 2
+            or g.shape[0] < _MIN_SUM_ROWS or g.shape[1] % 8 or not 0 < g.shape[1] <= 1 << 20
+            or not native(g)):
+        return None
+    rows, cols = g.shape
+    partials = torch.empty(_COLUMN_GROUPS * cols, dtype=torch.float32, device=g.device)
+    out = torch.empty(cols, dtype=dtype, device=g.device)
+    hip.call("lct_column_sum", g.data_ptr(), rows, cols, partials.data_ptr(), partials.numel(),
+             out.data_ptr(), int(dtype == torch.bfloat16), _stream(g))
+    return out
+
+
+def _norm_takes(x: Tensor, gain: Tensor) -> bool:
+    return (x.dtype == torch.bfloat16 and gain.dtype in (torch.bfloat16, torch.float32)
+            and x.ndim > 0 and gain.shape == x.shape[-1:] and x.shape[-1] % 4 == 0
+            and x.shape[-1] <= _MAX_COLUMNS)
+
+
+# The epsilon ATen's fused RMSNorm takes when none is given.
+_EPSILON = torch.finfo(torch.float32).eps
+
+
+def rms_norm(x: Tensor, gain: Tensor):
+    """``(bf16(x * rstd * bf16(gain)), rstd)`` over the last dimension, or None."""
+    if not _norm_takes(x, gain) or not native(x, gain):
+        return None
+    cols = x.shape[-1]
+    y = torch.empty_like(x)
+    rstd = torch.empty((*x.shape[:-1], 1), dtype=torch.float32, device=x.device)
+    hip.call("lct_rms_norm", x.data_ptr(), gain.data_ptr(), int(gain.dtype == torch.bfloat16),
+             y.data_ptr(), rstd.data_ptr(), x.numel() // cols, cols, _EPSILON, _stream(x))
+    return y, rstd
+
+
+def rms_norm_backward(grad: Tensor, x: Tensor, rstd: Tensor, gain: Tensor, dtype: torch.dtype,
+                      rebuild: bool):
+    """``(grad_x, grad_gain, normalized)``: the gradients of :func:`rms_norm`
+    (the gain's rounded to BF16, in ``dtype``) and, with ``rebuild``, its
+    output again as a matrix (else None); or None."""
+    if (not _norm_takes(x, gain) or grad.dtype != torch.bfloat16 or grad.shape != x.shape
+            or rstd.dtype != torch.float32 or rstd.numel() * x.shape[-1] != x.numel()
+            or dtype not in (torch.bfloat16, torch.float32)
+            or not native(grad, x, gain) or not native(rstd)):
+        return None
+    cols = x.shape[-1]
+    grad_x = torch.empty_like(x)
+    normalized = torch.empty_like(x) if rebuild else None
+    grad_gain = torch.empty(cols, dtype=dtype, device=x.device)
+    partials = torch.empty(_NORM_GROUPS * cols, dtype=torch.float32, device=x.device)
+    hip.call("lct_rms_norm_backward", grad.data_ptr(), x.data_ptr(), rstd.data_ptr(),
+             gain.data_ptr(), int(gain.dtype == torch.bfloat16), grad_x.data_ptr(),
+             None if normalized is None else normalized.data_ptr(), partials.data_ptr(),
+             partials.numel(), grad_gain.data_ptr(), int(dtype == torch.bfloat16),
+             x.numel() // cols, cols, _stream(x))
+    return grad_x, grad_gain, None if normalized is None else normalized.view(-1, cols)

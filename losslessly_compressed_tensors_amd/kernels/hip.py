@@ -243,6 +243,12 @@ _SIGNATURES = {
     "lct_buffer_free_batch": [_ptr, _c_int32, ctypes.POINTER(_ptr), _c_int32, _ptr, _ptr],
     "lct_set_wait_limits": [_c_int32, _c_int32],
     "lct_set_decoder": [_c_int32],
+    "lct_relu_square": [_ptr, _ptr, _ptr, _c_int64, _ptr],
+    "lct_relu_square_backward": [_ptr, _ptr, _ptr, _c_int64, _ptr],
+    "lct_column_sum": [_ptr, _c_int64, _c_int32, _ptr, _c_int64, _ptr, _c_int32, _ptr],
+    "lct_rms_norm": [_ptr, _ptr, _c_int32, _ptr, _ptr, _c_int64, _c_int32, ctypes.c_float, _ptr],
+    "lct_rms_norm_backward": [_ptr, _ptr, _ptr, _ptr, _c_int32, _ptr, _ptr, _ptr, _c_int64, _ptr,
+                              _c_int32, _c_int64, _c_int32, _ptr],
     "lct_bandwidth_probe": [_c_int32, _ptr, _c_int64, _ptr, _c_int64, _c_int32, _ptr],
     "lct_compress_buffered_noalloc": [_ptr, _c_int64, _c_int64, Geometry, _ptr, _ptr, _ptr, _ptr,
                                       _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _c_int32, _ptr,
