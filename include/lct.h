@@ -768,13 +768,13 @@ int32_t lct_column_sum(const void *g, int64_t rows, int32_t cols, float *partial
                        int64_t partial_floats, void *out, int32_t out_bf16, hipStream_t stream);
 
 /* RMSNorm over rows of cols values (a multiple of 4 up to 4096; 8-byte
- * aligned): rstd[r] = 1 / sqrt(mean(x^2) + eps), y = bf16(x * rstd * gain).
+ * aligned): rstd[r] = 1 / sqrt(mean(x^2) + 2^-23), y = bf16(x * rstd * gain).
  * The gain (cols values, BF16 if gain_bf16 != 0, else FP32 and then 16-byte
  * aligned) is rounded to BF16.  lct_rms_norm_backward: grad_x, grad_gain (rounded to BF16; stored as
  * BF16 or FP32) and, where normalized is not NULL, y again.  partials:
  * partial_floats >= cols working values, up to 512 cols of them used. */
 int32_t lct_rms_norm(const void *x, const void *gain, int32_t gain_bf16, void *y, float *rstd,
-                     int64_t rows, int32_t cols, float eps, hipStream_t stream);
+                     int64_t rows, int32_t cols, hipStream_t stream);
 int32_t lct_rms_norm_backward(const void *grad, const void *x, const float *rstd,
                               const void *gain, int32_t gain_bf16, void *grad_x,
                               void *normalized, float *partials, int64_t partial_floats,

@@ -219,9 +219,10 @@ __device__ __forceinline__ Gain4 load_gain(const void *gain, int32_t gain_bf16, 
     return out;
 }
 
+constexpr float kEpsilon = 0x1p-23f;          // FP32's, as ATen's when none is given
 constexpr int kRowWaves = kLanes / kWave;   // rows in flight per workgroup
 
-// y = bf16(x * rstd * gain), rstd = 1 / sqrt(mean(x^2) + eps).  A wave has one
+// y = bf16(x * rstd * gain), rstd = 1 / sqrt(mean(x^2) + kEpsilon).  A wave has one
 // row and reads the gain (from L2) only for its products, so a SIMD holds
 // several rows' loads at once: 9 us at 8192 x 768 and 19 at 8192 x 3072
 // (ATen's row kernel: 14.5 and 25; waves that keep the gain and walk several
@@ -232,7 +233,7 @@ __global__ __launch_bounds__(kLanes) void rms_norm_kernel(const uint16_t *__rest
                                                           int32_t gain_bf16,
                                                           uint16_t *__restrict__ y,
                                                           float *__restrict__ rstd, int64_t rows,
-                                                          int32_t cols, float eps) {
+                                                          int32_t cols) {
     const int64_t r = int64_t{blockIdx.x} * kRowWaves + threadIdx.x / kWave;
     if (r >= rows) return;
     Row<kChunks> row;
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(kLanes) void rms_norm_kernel(const uint16_t *__rest
             sum += lo * lo + hi * hi;
         }
     }
-    const float inverse = rsqrtf(wave_sum_float(sum) / static_cast<float>(cols) + eps);
+    const float inverse = rsqrtf(wave_sum_float(sum) / static_cast<float>(cols) + kEpsilon);
     if (wave_lane() == 0) rstd[r] = inverse;
 #pragma unroll
     for (int k = 0; k < kChunks; ++k) {
@@ -443,8 +444,7 @@ extern "C" int32_t lct_column_sum(const void *g, int64_t rows, int32_t cols, flo
 }
 
 extern "C" int32_t lct_rms_norm(const void *x, const void *gain, int32_t gain_bf16, void *y,
-                                float *rstd, int64_t rows, int32_t cols, float eps,
-                                hipStream_t stream) {
+                                float *rstd, int64_t rows, int32_t cols, hipStream_t stream) {
     if (!x || !gain || !y || !rstd) return LCT_E_NULL;
     if (rows <= 0 || rows > kMaxRows || cols <= 0 || cols > kMaxColumns) return LCT_E_SIZE;
     if ((cols & 3) != 0 || !aligned(x, 8) || !aligned(y, 8)
@@ -454,7 +454,7 @@ extern "C" int32_t lct_rms_norm(const void *x, const void *gain, int32_t gain_bf
     by_chunks(cols, [&](auto chunks) {
         rms_norm_kernel<decltype(chunks)::value><<<grid, kLanes, 0, stream>>>(
             static_cast<const uint16_t *>(x), gain, gain_bf16, static_cast<uint16_t *>(y), rstd,
-            rows, cols, eps);
+            rows, cols);
     });
     return static_cast<int32_t>(hipGetLastError());
 }

@@ -89,10 +89,6 @@ def _norm_takes(x: Tensor, gain: Tensor) -> bool:
             and x.shape[-1] <= _MAX_COLUMNS)
 
 
-# The epsilon ATen's fused RMSNorm takes when none is given.
-_EPSILON = torch.finfo(torch.float32).eps
-
-
 def rms_norm(x: Tensor, gain: Tensor):
     """``(bf16(x * rstd * bf16(gain)), rstd)`` over the last dimension, or None."""
     if not _norm_takes(x, gain) or not native(x, gain):
@@ -101,7 +97,7 @@ def rms_norm(x: Tensor, gain: Tensor):
     y = torch.empty_like(x)
     rstd = torch.empty((*x.shape[:-1], 1), dtype=torch.float32, device=x.device)
     hip.call("lct_rms_norm", x.data_ptr(), gain.data_ptr(), int(gain.dtype == torch.bfloat16),
-             y.data_ptr(), rstd.data_ptr(), x.numel() // cols, cols, _EPSILON, _stream(x))
+             y.data_ptr(), rstd.data_ptr(), x.numel() // cols, cols, _stream(x))
     return y, rstd
 
 

@@ -246,7 +246,7 @@ _SIGNATURES = {
     "lct_relu_square": [_ptr, _ptr, _ptr, _c_int64, _ptr],
     "lct_relu_square_backward": [_ptr, _ptr, _ptr, _c_int64, _ptr],
     "lct_column_sum": [_ptr, _c_int64, _c_int32, _ptr, _c_int64, _ptr, _c_int32, _ptr],
-    "lct_rms_norm": [_ptr, _ptr, _c_int32, _ptr, _ptr, _c_int64, _c_int32, ctypes.c_float, _ptr],
+    "lct_rms_norm": [_ptr, _ptr, _c_int32, _ptr, _ptr, _c_int64, _c_int32, _ptr],
     "lct_rms_norm_backward": [_ptr, _ptr, _ptr, _ptr, _c_int32, _ptr, _ptr, _ptr, _c_int64, _ptr,
                               _c_int32, _c_int64, _c_int32, _ptr],
     "lct_bandwidth_probe": [_c_int32, _ptr, _c_int64, _ptr, _c_int64, _c_int32, _ptr],
