@@ -781,6 +781,13 @@ int32_t lct_rms_norm_backward(const void *grad, const void *x, const float *rstd
                               void *grad_gain, int32_t grad_gain_bf16, int64_t rows,
                               int32_t cols, hipStream_t stream);
 
+/* ---- out = A W^T for at most LCT_MAX_SKINNY_TOKENS rows of A against a dense
+ * W [rows, cols] (LCT/operations.py:31-48): contiguous BF16, FP32 sums, one
+ * rounding.  cols: a multiple of 8; a and w 16-byte aligned. */
+#define LCT_MAX_SKINNY_TOKENS 16
+int32_t lct_skinny_linear(const void *a, const void *w, void *out, int32_t tokens, int32_t rows,
+                          int32_t cols, hipStream_t stream);
+
 /* ---- attainable HBM bandwidth with the codec kernels' access shape (16-byte
  * non-temporal buffer accesses, `workgroups` workgroups of 256 threads each
  * walking 16 KiB passes).  kind 0: copy src -> dst (src_bytes = dst_bytes);

@@ -29,6 +29,7 @@ SOURCES = [
     "update.hip",
     "noalloc.hip",
     "layers.hip",
+    "linear.hip",
     "bandwidth.hip",
 ]
 

@@ -1,7 +1,8 @@
-"""One-pass device kernels for the dense steps of the compressed layers.
+"""Device kernels for the dense steps around the codec.
 
 Each function is an expression of ``components/layers.py`` or
-``components/ops.py`` as one or two launches of ``csrc/layers.hip``, for the
+``components/ops.py`` as one or two launches of ``csrc/layers.hip``, or the
+product of ``operations.A_compBT`` as one of ``csrc/linear.hip``, for the
 tensors that ``native`` accepts; the callers keep ATen's expression for the
 others (host tensors, other types, strided views, and wherever autograd,
 tracing or a transform has to see the operations).
@@ -87,6 +88,25 @@ def _norm_takes(x: Tensor, gain: Tensor) -> bool:
     return (x.dtype == torch.bfloat16 and gain.dtype in (torch.bfloat16, torch.float32)
             and x.ndim > 0 and gain.shape == x.shape[-1:] and x.shape[-1] % 4 == 0
             and x.shape[-1] <= _MAX_COLUMNS)
+
+
+# lct_skinny_linear's range of A's rows.
+MAX_SKINNY_TOKENS = 16
+
+
+def skinny_linear(a: Tensor, w: Tensor):
+    """``a @ w.T`` of at most 16 rows, or None (from there on the library's
+    product is faster: 21 us against 28 at 17 to 32 rows of 11008 x 4096)."""
+    if (a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or a.ndim != 2
+            or a.shape[0] > MAX_SKINNY_TOKENS or a.shape[1] % 8
+            or max(w.shape) > 1 << 30 or not native(a, w)):
+        return None
+    tokens, cols = a.shape
+    rows = w.shape[0]
+    out = torch.empty((tokens, rows), dtype=torch.bfloat16, device=a.device)
+    hip.call("lct_skinny_linear", a.data_ptr(), w.data_ptr(), out.data_ptr(), tokens, rows, cols,
+             _stream(a))
+    return out
 
 
 def rms_norm(x: Tensor, gain: Tensor):

@@ -249,6 +249,7 @@ _SIGNATURES = {
     "lct_rms_norm": [_ptr, _ptr, _c_int32, _ptr, _ptr, _c_int64, _c_int32, _ptr],
     "lct_rms_norm_backward": [_ptr, _ptr, _ptr, _ptr, _c_int32, _ptr, _ptr, _ptr, _c_int64, _ptr,
                               _c_int32, _c_int64, _c_int32, _ptr],
+    "lct_skinny_linear": [_ptr, _ptr, _ptr, _c_int32, _c_int32, _c_int32, _ptr],
     "lct_bandwidth_probe": [_c_int32, _ptr, _c_int64, _ptr, _c_int64, _c_int32, _ptr],
     "lct_compress_buffered_noalloc": [_ptr, _c_int64, _c_int64, Geometry, _ptr, _ptr, _ptr, _ptr,
                                       _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _c_int32, _ptr,

@@ -21,6 +21,7 @@ from .codec.pointwise import (
 )
 from .comp_format import Distribution, StorageLayout
 from .comp_tensor import CompressedTensor
+from .kernels import fused
 from .tensor_buffer import TensorBuffer
 
 
@@ -61,7 +62,9 @@ def A_compBT(A: Tensor, B_comp: CompressedTensor) -> Tensor:
     """``A @ B_comp.T``."""
     if A.ndim != 2 or A.shape[1] != B_comp.shape[1]:
         raise ValueError("activation and weight inner dimensions must match")
-    return A.contiguous() @ decompress(B_comp).T
+    A, B = A.contiguous(), decompress(B_comp)
+    product = fused.skinny_linear(A, B)
+    return A @ B.T if product is None else product
 
 
 def A_compB(A: Tensor, B_comp: CompressedTensor) -> Tensor:
