@@ -11,7 +11,7 @@ import torch
 
 from ..comp_tensor import CompressedTensor
 from ..compression.huffman_tables import get_distribution_tables
-from ..kernels import dispatch
+from ..kernels import dispatch, hip
 from ..kernels.dispatch import FallbackStorage
 
 
@@ -46,6 +46,18 @@ def overlay_of(data: CompressedTensor) -> FallbackStorage | None:
     return storage_of(data) if has_fallback(data) else None
 
 
+def overflow_argument(data: CompressedTensor) -> hip.Overflow | None:
+    """``overlay_of`` as the C ABI's record."""
+    descriptor = data.fallback_descriptor
+    if data.layout != data.layout.COMPRESSED:
+        return None
+    if descriptor is not None:
+        arena = data.fallback_buffer.data_ptr()
+        return hip.Overflow(arena, arena, arena, data.fallback_blocks.data_ptr(),
+                            data.fallback_count.data_ptr(), descriptor.data_ptr(), 0)
+    return overlay_of(data).as_overflow() if has_fallback(data) else None
+
+
 def shifted_decode_table(data: CompressedTensor) -> torch.Tensor:
     """The tensor's shifted decode table, rebuilt from its center if absent."""
     if data.decode_table is not None:
@@ -75,22 +87,32 @@ def decode_batch(tensors: list[CompressedTensor]) -> list[torch.Tensor]:
     Each result equals ``decode`` of its tensor.  For tensors of a few codec
     blocks each (a layer's weights), whose decodes are bound by one block's
     latency, one launch replaces one per tensor."""
-    from ..kernels import hip
-
     outputs = []
     jobs = []
+    held = []   # the tables that shifted_decode_table made
+    stream = None
     for data in tensors:
         if data.layout != data.layout.COMPRESSED:
             outputs.append(data.data.reshape(data.shape))
             continue
-        output = torch.empty(data.logical_numel, dtype=torch.int16, device=data.data.device)
-        outputs.append(output.view(torch.bfloat16).reshape(data.shape))
-        if not data.logical_numel:
+        payload, side = data.data, data.sign_mantissa
+        device = payload.device
+        output = torch.empty(data.shape, dtype=torch.bfloat16, device=device)
+        outputs.append(output)
+        n = output.numel()
+        if not n:
             continue
-        _, _, rare_length = get_distribution_tables(data.distribution, data.data.device)
-        jobs.append((data.data, data.sign_mantissa, output, shifted_decode_table(data),
-                     data.center, data.size, data.logical_numel, data.codec_geometry,
-                     rare_length, overlay_of(data)))
+        dispatch.require_device(payload, side)
+        if stream is None:
+            stream = torch._C._cuda_getCurrentRawStream(device.index)
+        table = shifted_decode_table(data)
+        held.append(table)
+        overflow = overflow_argument(data)
+        jobs.append(hip.DecodeJob(
+            payload.data_ptr(), side.data_ptr(), output.data_ptr(), table.data_ptr(),
+            data.center.data_ptr(), data.size, n, hip.Geometry(*data.codec_geometry),
+            get_distribution_tables(data.distribution, device)[2], int(overflow is not None),
+            overflow or hip.Overflow()))
     for start in range(0, len(jobs), hip.MAX_DECODE_BATCH):
-        dispatch.decode_batch(jobs[start:start + hip.MAX_DECODE_BATCH])
+        dispatch.decode_batch(jobs[start:start + hip.MAX_DECODE_BATCH], stream)
     return outputs

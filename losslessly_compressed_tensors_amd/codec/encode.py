@@ -134,6 +134,38 @@ def record_arrays(device, blocks: int, buffered: bool):
     return shifted, counts, count, used, descriptor, center, blocks_out
 
 
+def stored_arrays(device, storage_numel: int, payload_bytes: int, blocks: int,
+                  sample_size: int) -> torch.Tensor:
+    """One int32 allocation for every array of a buffered record: side bytes,
+    payload words, the small arrays of ``record_arrays`` and the sample values
+    (16-byte aligned up to the sample values, as ``storage_numel`` and
+    ``payload_bytes`` are multiples of 16).  ``batch_record`` makes the views."""
+    return torch.empty((storage_numel + payload_bytes) // 4 + 1033 + 3 * blocks
+                       + (sample_size + 1) // 2, dtype=torch.int32, device=device)
+
+
+def batch_record(arrays: torch.Tensor, storage_numel: int, payload_bytes: int, blocks: int,
+                 sample_size: int, buffer: TensorBuffer, distribution: Distribution, shape,
+                 stream_geometry) -> CompressedTensor:
+    """The record whose arrays are ``stored_arrays`` of the same sizes."""
+    side, payload, shifted_decode, count, used, _, descriptor, center, blocks_out, samples = (
+        arrays.split_with_sizes((storage_numel // 4, payload_bytes // 4, 1024, 1, 1, 2, 4, 1,
+                                 3 * blocks, (sample_size + 1) // 2)))
+    samples = samples.view(torch.int16)
+    return CompressedTensor(
+        payload, storage_numel, side.view(torch.uint8),
+        fallback_blocks=blocks_out,
+        fallback_buffer=buffer.data,
+        fallback_descriptor=descriptor,
+        buffer=buffer,
+        fallback_count=count,
+        fallback_used=used,
+        distribution=distribution, center=center, decode_table=shifted_decode, shape=shape,
+        layout=StorageLayout.COMPRESSED, stream_geometry=stream_geometry,
+        sample_values=samples if sample_size % 2 == 0 else samples[:sample_size],
+    )
+
+
 def _encode_fused(source_values, sign_mantissa, encoded, size, distribution, buffer, shape,
                   encode_table, decode_table, sample_size, sample_values,
                   launch) -> CompressedTensor:
@@ -516,20 +548,21 @@ def encode_batch(tensors, distributions, buffer: TensorBuffer) -> list[Compresse
         storage_numel = blocks * block_symbols
         payload_bytes = 4 * (blocks * lanes * fixed_words + 4)
         device = source.device
-        packed = torch.empty(storage_numel + payload_bytes, dtype=torch.uint8, device=device)
-        record = torch.empty(1033 + 3 * blocks, dtype=torch.int32, device=device)
         sample_size = min(logical_numel, CENTER_SAMPLE_SIZE)
-        sample_values = torch.empty(sample_size, dtype=torch.int16, device=device)
+        arrays = stored_arrays(device, storage_numel, payload_bytes, blocks, sample_size)
         encode_table, decode_table, _ = get_distribution_tables(distribution, device)
-        p_side, p_record = packed.data_ptr(), record.data_ptr()
+        p_side = arrays.data_ptr()
+        p_record = p_side + storage_numel + payload_bytes
         job = hip.CompressJob(
             source.data_ptr(), p_side, p_side + storage_numel, encode_table.data_ptr(),
-            decode_table.data_ptr(), p_record + 4 * 1032, p_record, sample_values.data_ptr(),
-            p_record + 4 * 1033, p_record + 4 * 1024, p_record + 4 * 1028, sample_size,
-            storage_numel, logical_numel, hip.Geometry(*stream_geometry))
+            decode_table.data_ptr(), p_record + 4 * 1032, p_record,
+            p_record + 4 * (1033 + 3 * blocks), p_record + 4 * 1033, p_record + 4 * 1024,
+            p_record + 4 * 1028, sample_size, storage_numel, logical_numel,
+            hip.Geometry(block_symbols, lanes, steps, fixed_words))
         pending.setdefault(steps, []).append(
-            (index, job, source, packed, record, sample_values, shape, distribution,
-             stream_geometry, storage_numel, payload_bytes, blocks))
+            (index, job, blocks, source,
+             (arrays, storage_numel, payload_bytes, blocks, sample_size, buffer, distribution,
+              shape, stream_geometry)))
     device = buffer.device
     stream = torch._C._cuda_getCurrentRawStream(device.index)
     for members in pending.values():
@@ -537,27 +570,11 @@ def encode_batch(tensors, distributions, buffer: TensorBuffer) -> list[Compresse
             part = members[start:start + hip.MAX_COMPRESS_BATCH]
             frees = buffer._take_frees()
             try:
-                dispatch.compress_batch_pointers([m[1] for m in part], buffer, frees, device,
-                                                 stream)
+                dispatch.compress_batch_pointers([m[1] for m in part], sum(m[2] for m in part),
+                                                 buffer, frees, device, stream)
             except BaseException:
                 buffer._restore_frees(frees)
                 raise
-            for (index, _, source, packed, record, sample_values, shape, distribution,
-                 stream_geometry, storage_numel, payload_bytes, blocks) in part:
-                side, payload = packed.split_with_sizes((storage_numel, payload_bytes))
-                shifted_decode, counts, descriptor, center, blocks_out = record.split_with_sizes(
-                    (1024, 4, 4, 1, 3 * blocks))
-                count_view, used_view = counts.split_with_sizes((1, 1, 2))[:2]
-                results[index] = CompressedTensor(
-                    payload.view(torch.int32), storage_numel, side,
-                    fallback_blocks=blocks_out,
-                    fallback_buffer=buffer.data,
-                    fallback_descriptor=descriptor,
-                    buffer=buffer,
-                    fallback_count=count_view,
-                    fallback_used=used_view,
-                    distribution=distribution, center=center, decode_table=shifted_decode,
-                    shape=shape, layout=StorageLayout.COMPRESSED,
-                    stream_geometry=stream_geometry, sample_values=sample_values,
-                )
+            for index, _, _, _, record in part:
+                results[index] = batch_record(*record)
     return results

@@ -27,8 +27,8 @@ from ..compression.huffman_tables import get_distribution_tables
 from ..kernels import dispatch, hip
 from ..tensor_buffer import TensorBuffer
 from .decode import decode as decode_dense
-from .decode import overlay_of, shifted_decode_table, storage_of
-from .encode import CENTER_SAMPLE_SIZE, finish_encode, finish_fused
+from .decode import overflow_argument, overlay_of, shifted_decode_table, storage_of
+from .encode import CENTER_SAMPLE_SIZE, batch_record, finish_encode, finish_fused, stored_arrays
 from .encode import encode as compress_dense
 from .encode import encode_components as compress_components
 from .geometry import geometry
@@ -373,90 +373,77 @@ def fused_update_batch(items, operation: PointwiseOp, buffer: TensorBuffer, *,
     pending: dict[int, list] = {}
     for index, (data, other, distribution) in enumerate(items):
         result_distribution = distribution or data.distribution
-        if tuple(other.shape) != data.shape:
+        shape = data.shape
+        if tuple(other.shape) != shape:
             raise ValueError(f"{operation.name} expects tensors with the same shape")
-        if (data.layout != StorageLayout.COMPRESSED or data.logical_numel == 0
-                or geometry(result_distribution) != data.codec_geometry):
+        n = data.logical_numel
+        stream_geometry = geometry(result_distribution)
+        if (data.layout != StorageLayout.COMPRESSED or n == 0
+                or stream_geometry != data.codec_geometry):
             results[index] = pointwise_compressed_dense(
                 data, other, operation, alpha=alpha, beta=beta, alpha_is_one=alpha_is_one,
                 dense_output=False, buffer=buffer, distribution=result_distribution)
             continue
         _require_bf16(other, operation)
-        dispatch.require_device(data.data, other)
-        other = other.contiguous().view(-1)
-        block_symbols, lanes, steps, fixed_words = data.codec_geometry
-        blocks = data.size // block_symbols
-        streams = blocks * lanes
-        n = data.logical_numel
-        _, _, rare_length = get_distribution_tables(data.distribution, device)
-        base_encode, base_decode, _ = get_distribution_tables(result_distribution, device)
+        payload = data.data
+        dispatch.require_device(payload, other)
+        other = other.contiguous()
+        block_symbols, lanes, steps, fixed_words = stream_geometry
+        size = data.size
+        blocks = size // block_symbols
+        base_encode, base_decode, rare_length = get_distribution_tables(result_distribution,
+                                                                        device)
+        if data.distribution is not result_distribution:
+            rare_length = get_distribution_tables(data.distribution, device)[2]
         sample_size = min(n, CENTER_SAMPLE_SIZE)
         a_samples = data.sample_values
         if a_samples is not None and a_samples.numel() != sample_size:
             a_samples = None
-        payload_bytes = 4 * (streams * fixed_words + 4)
-        packed = torch.empty(data.size + payload_bytes, dtype=torch.uint8, device=device)
-        record = torch.empty(1033 + 3 * blocks, dtype=torch.int32, device=device)
-        result_samples = torch.empty(sample_size, dtype=torch.int16, device=device)
-        # Only the rows of overflowing streams are written (and read back by
-        # the compaction); the rest stays unwritten.
-        exponents = torch.empty(n, dtype=torch.uint8, device=device)
-        overflow = overlay_of(data)
-        p_side, p_record = packed.data_ptr(), record.data_ptr()
-        job = hip.UpdateJob()
-        job.encoded, job.side = data.data.data_ptr(), data.sign_mantissa.data_ptr()
-        job.shifted_decode = shifted_decode_table(data).data_ptr()
-        job.center = data.center.data_ptr()
-        job.has_overflow = int(overflow is not None)
-        if overflow is not None:
-            job.overflow = overflow.as_overflow()
-        job.a_samples = None if a_samples is None else a_samples.data_ptr()
-        job.other = other.data_ptr()
-        job.base_encode, job.base_decode = base_encode.data_ptr(), base_decode.data_ptr()
-        job.center_out, job.shifted_decode_out = p_record + 4 * 1032, p_record
-        job.side_out, job.encoded_out = p_side, p_side + data.size
-        job.result_samples = result_samples.data_ptr()
-        job.exponents = exponents.data_ptr()
-        job.counts, job.descriptor = p_record + 4 * 1024, p_record + 4 * 1028
-        job.blocks = p_record + 4 * 1033
-        job.size, job.logical_numel, job.sample_size = data.size, n, sample_size
-        job.geometry = hip.Geometry(block_symbols, lanes, steps, fixed_words)
-        job.rare_length = rare_length
+        payload_bytes = 4 * (blocks * lanes * fixed_words + 4)
+        arrays = stored_arrays(device, size, payload_bytes, blocks, sample_size)
+        p_side = arrays.data_ptr()
+        p_record = p_side + size + payload_bytes
+        overflow = overflow_argument(data)
+        table = shifted_decode_table(data)
+        job = hip.UpdateJob(
+            payload.data_ptr(), data.sign_mantissa.data_ptr(), table.data_ptr(),
+            data.center.data_ptr(), int(overflow is not None), overflow or hip.Overflow(),
+            None if a_samples is None else a_samples.data_ptr(), other.data_ptr(),
+            base_encode.data_ptr(), base_decode.data_ptr(), p_record + 4 * 1032, p_record,
+            p_side, p_side + size, p_record + 4 * (1033 + 3 * blocks), None,
+            p_record + 4 * 1024, p_record + 4 * 1033, p_record + 4 * 1028, size, n, sample_size,
+            hip.Geometry(block_symbols, lanes, steps, fixed_words), rare_length)
         pending.setdefault(steps, []).append(
-            (index, job, (data, other, exponents), packed, record, result_samples,
-             result_distribution, blocks, payload_bytes))
+            (index, job, blocks, (other, table),
+             (arrays, size, payload_bytes, blocks, sample_size, buffer, result_distribution,
+              shape, stream_geometry)))
     stream = torch._C._cuda_getCurrentRawStream(device.index)
     for members in pending.values():
         for start in range(0, len(members), hip.MAX_UPDATE_BATCH):
             part = members[start:start + hip.MAX_UPDATE_BATCH]
+            jobs = [m[1] for m in part]
+            # Exponent bytes of the results, 16-byte aligned.  Only the rows of
+            # overflowing streams are written (and read back by the
+            # compaction); the rest stays unwritten.
+            offsets, end, groups = [], 0, 0
+            for job in jobs:
+                offsets.append(end)
+                end += -(-job.logical_numel // 16) * 16
+                groups += -(-job.sample_size // 64)
+            exponents = torch.empty(end, dtype=torch.uint8, device=device)
+            p_exponents = exponents.data_ptr()
+            for job, offset in zip(jobs, offsets):
+                job.exponents = p_exponents + offset
             frees = buffer._take_frees()
             try:
                 dispatch.pointwise_update_batch_pointers(
-                    [m[1] for m in part], operation.code, alpha_is_one, beta_is_one, alpha_arg,
-                    beta_arg, buffer, frees, device, stream)
+                    jobs, sum(m[2] for m in part), groups, operation.code, alpha_is_one,
+                    beta_is_one, alpha_arg, beta_arg, buffer, frees, device, stream)
             except BaseException:
                 buffer._restore_frees(frees)
                 raise
-            for (index, _, (data, _, _), packed, record, result_samples, result_distribution,
-                 blocks, payload_bytes) in part:
-                side, payload = packed.split_with_sizes((data.size, payload_bytes))
-                shifted_decode, counts, descriptor, center, blocks_out = record.split_with_sizes(
-                    (1024, 4, 4, 1, 3 * blocks))
-                count_view, used_view = counts.split_with_sizes((1, 1, 2))[:2]
-                results[index] = CompressedTensor(
-                    payload.view(torch.int32), data.size, side,
-                    fallback_blocks=blocks_out,
-                    fallback_buffer=buffer.data,
-                    fallback_descriptor=descriptor,
-                    buffer=buffer,
-                    fallback_count=count_view,
-                    fallback_used=used_view,
-                    distribution=result_distribution, center=center,
-                    decode_table=shifted_decode, shape=data.shape,
-                    layout=StorageLayout.COMPRESSED,
-                    stream_geometry=geometry(result_distribution),
-                    sample_values=result_samples,
-                )
+            for index, _, _, _, record in part:
+                results[index] = batch_record(*record)
     return results
 
 

@@ -21,6 +21,8 @@ class NoiseLevel(Enum):
     HIGH = auto()    # smaller blocks, more payload per stream
     SPARSE = auto()  # 2.5 fixed bits per exponent plus overflow storage
 
+    __hash__ = object.__hash__   # members are singletons; Enum's hashes the name in Python
+
 
 class DistType(Enum):
     """Codebook family (``comp_format.py:13-17``)."""
@@ -29,6 +31,8 @@ class DistType(Enum):
     GAUSSIAN = "gaussian"
     LAPLACE = "laplace"
     GAMMA = "gamma"
+
+    __hash__ = object.__hash__
 
 
 class StorageLayout(Enum):

@@ -91,6 +91,13 @@ class CompressedTensor:
             storage = value.untyped_storage()
             allocations[(value.device, storage.data_ptr())] = storage.nbytes()
         total = sum(allocations.values())
+        samples = self.sample_values
+        if samples is not None:
+            # stored_arrays keeps them behind the arrays counted here, in
+            # whole int32 words.
+            storage = samples.untyped_storage()
+            if (samples.device, storage.data_ptr()) in allocations:
+                total -= 4 * ((samples.numel() + 1) // 2)
         if self.fallback_descriptor is not None:
             total += self._reserved_bytes()
         return total
@@ -109,9 +116,9 @@ class CompressedTensor:
         ``lct::tensor_buffer_free`` operator."""
         if self.fallback_descriptor is None or self.buffer is None:
             return
-        from .tensor_buffer import Allocation
-
         if torch.compiler.is_compiling():
+            from .tensor_buffer import Allocation
+
             self.buffer.free(Allocation(self.fallback_descriptor, self.buffer))
         else:
             self.buffer._defer_free(self.fallback_descriptor)

@@ -271,6 +271,20 @@ def get_distribution_tables(dist: Distribution, device=None):
     tensors (uploaded once per distribution and device), ``rare_length`` is
     the ESC code length.
     """
+    if isinstance(dist, Distribution):
+        # Every compress, decode and update asks for these.
+        known = _by_device.get((dist.family, dist.param, dist.mean, dist.zero_prob, device))
+        if known is not None:
+            return known
+    return _device_entry(dist, device)
+
+
+# get_distribution_tables' results by the arguments that gave them, for devices
+# with an index (what "cuda" and None mean may change between calls).
+_by_device: dict = {}
+
+
+def _device_entry(dist: Distribution, device):
     import torch
 
     book = distribution_codebook(dist)
@@ -286,4 +300,7 @@ def get_distribution_tables(dist: Distribution, device=None):
                 torch.from_numpy(book.decode.copy()).to(device),
             )
             _device_tables[key] = cached
-    return cached[0], cached[1], book.rare_length
+    result = cached[0], cached[1], book.rare_length
+    if device.index is not None:
+        _by_device[(dist.family, dist.param, dist.mean, dist.zero_prob, device)] = result
+    return result

@@ -339,16 +339,15 @@ def encode_fused_pointers(source, side, encoded, sample_size, encode_table, deco
     return epoch
 
 
-def compress_batch_pointers(jobs, buffer, frees, device, stream) -> None:
+def compress_batch_pointers(jobs, total, buffer, frees, device, stream) -> None:
     """``lct_compress_batch``: the buffered compress of ``jobs`` (at most
     ``hip.MAX_COMPRESS_BATCH`` ``hip.CompressJob``s with device addresses,
-    all of one step count) into ``buffer``, applying the deferred ``frees``
-    first, on the raw stream handle ``stream`` of ``device``."""
-    n_blocks = [job.size // job.geometry.block_symbols for job in jobs]
-    total = sum(n_blocks)
+    all of one step count, ``total`` codec blocks together) into ``buffer``,
+    applying the deferred ``frees`` first, on the raw stream handle ``stream``
+    of ``device``."""
     # One working array each, partitioned by the entry point in job order:
     # extra starts (256 per block), summaries (5 nb + 1 per job) and control
-    # words (a gate word, then 64 + nb per job).
+    # words (one spare, then 64 + nb per job).
     extra_starts, summaries = compress_workspace(device, total + len(jobs), total * 256)
     control = control_array(device, total + (CONTROL_PARTIALS + 1) * len(jobs))
     pending = hip.PendingFrees()
@@ -362,16 +361,14 @@ def compress_batch_pointers(jobs, buffer, frees, device, stream) -> None:
              buffer.max_free_regions, buffer.data.data_ptr(), hip.ctypes.byref(pending), stream)
 
 
-def pointwise_update_batch_pointers(jobs, op, alpha_is_one, beta_is_one, alpha, beta, buffer,
-                                    frees, device, stream) -> None:
+def pointwise_update_batch_pointers(jobs, total, groups, op, alpha_is_one, beta_is_one, alpha,
+                                    beta, buffer, frees, device, stream) -> None:
     """``lct_pointwise_update_batch``: the fused compressed-output updates of
     ``jobs`` (at most ``hip.MAX_UPDATE_BATCH`` ``hip.UpdateJob``s with device
-    addresses, one step count) into ``buffer``, applying the deferred
-    ``frees`` first, on the raw stream handle ``stream`` of ``device``.
+    addresses, one step count, ``total`` codec blocks and ``groups`` groups of
+    64 samples together) into ``buffer``, applying the deferred ``frees``
+    first, on the raw stream handle ``stream`` of ``device``.
     ``alpha``/``beta``: float32 device scalars or None."""
-    n_blocks = [job.size // job.geometry.block_symbols for job in jobs]
-    total = sum(n_blocks)
-    groups = sum(-(-job.sample_size // 64) for job in jobs)
     extra_starts, summaries = compress_workspace(device, total + len(jobs), total * 256)
     control = control_array(device, total + (CONTROL_PARTIALS + 1) * len(jobs))
     partials = torch.empty(2 * groups, dtype=torch.int32, device=device)
@@ -537,24 +534,11 @@ def decode_kernel(encoded, side, output, shifted_decode, center, size, *, logica
              ov if ov is None else hip.ctypes.byref(ov), _stream(encoded))
 
 
-def decode_batch(jobs) -> None:
-    """Several decodes in one launch (``lct_decode_batch``).  ``jobs``: at most
-    ``hip.MAX_DECODE_BATCH`` tuples ``(encoded, side, output, shifted_decode,
-    center, size, logical_numel, (B, L, S, W), rare_length, overflow)`` with
-    ``decode_kernel``'s meanings, all on the current stream's device."""
-    array = (hip.DecodeJob * len(jobs))()
-    for job, (encoded, side, output, shifted_decode, center, size, logical_numel, geometry,
-              rare_length, overflow) in zip(array, jobs):
-        _require_device(encoded, side, output)
-        job.encoded, job.side, job.output = _ptr(encoded), _ptr(side), _ptr(output)
-        job.shifted_decode, job.center = _ptr(shifted_decode), _ptr(center)
-        job.size, job.logical_numel = int(size), int(logical_numel)
-        job.geometry = hip.Geometry(*(int(v) for v in geometry))
-        job.rare_length = int(rare_length)
-        job.has_overflow = int(overflow is not None)
-        if overflow is not None:
-            job.overflow = overflow.as_overflow()
-    hip.call("lct_decode_batch", array, len(jobs), _stream(jobs[0][0]))
+def decode_batch(jobs, stream) -> None:
+    """Several decodes in one launch (``lct_decode_batch``): at most
+    ``hip.MAX_DECODE_BATCH`` ``hip.DecodeJob``s with device addresses, on the
+    raw stream handle ``stream``."""
+    hip.call("lct_decode_batch", (hip.DecodeJob * len(jobs))(*jobs), len(jobs), stream)
 
 
 def scatter_fallback(storage: FallbackStorage, sign_mantissa, output, n_elements,
