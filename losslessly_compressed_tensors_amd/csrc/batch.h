@@ -40,8 +40,7 @@ struct CompressBatch {
     CompressBatchJob jobs[LCT_MAX_COMPRESS_BATCH];
     int32_t *buffer_meta;
     int32_t max_free_regions;
-    lct_pending_frees frees;   // job 0 applies them
-    uint64_t *gate;            // job 0's "frees applied" word, nullptr without frees
+    lct_pending_frees frees;
     uint32_t epoch;
     int32_t steps;   // every job's S (the side-store policy is chosen by it)
     int32_t lock_spins;

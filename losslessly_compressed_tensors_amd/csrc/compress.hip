@@ -47,8 +47,8 @@ namespace {
 
 // Workgroup `group` of one tensor's fused compress (the launch layout above):
 // the single launch runs it for blockIdx.x, the batched launch for its job's
-// share of the grid.  gate: GatedReserve's word (batched launches only).
-template <int kSidePolicy, bool kPrecomputed>
+// share of the grid, with `book` for its reservation.
+template <int kSidePolicy, bool kPrecomputed, class Book>
 __device__ __forceinline__ void compress_group(
     const void *__restrict__ source, uint8_t *__restrict__ side, int32_t *__restrict__ encoded,
     const int32_t *__restrict__ base_encode, const int32_t *__restrict__ base_decode,
@@ -59,7 +59,7 @@ __device__ __forceinline__ void compress_group(
     uint32_t epoch, int32_t *__restrict__ descriptor, int32_t *__restrict__ buffer_meta,
     int32_t max_free_regions, const lct_pending_frees &frees, uint64_t *host_totals,
     int32_t n_blocks, int64_t logical_numel, int S, int W, int32_t lock_spins, int32_t polls,
-    int64_t group, uint64_t *gate, bool post_gate, uint32_t *stage) {
+    int64_t group, Book book, uint32_t *stage) {
     __shared__ uint2 table[256];
     __shared__ __attribute__((aligned(16))) uint8_t slices[kWavesPerBlock * kSliceBytes];
     __shared__ int32_t scratch[kWavesPerBlock];
@@ -115,12 +115,11 @@ __device__ __forceinline__ void compress_group(
     // barriers, so it can hold the free list.
     PolledSummaries polled{control, epoch, n_blocks, polls, false};
     if (buffer_meta != nullptr) {
-        GatedReserve reserve{
-            LdsReserve<false>{AllocatorMeta(buffer_meta, max_free_regions, lock_spins),
-                              descriptor, frees, reinterpret_cast<int32_t *>(stage), {}, -1,
-                              kStatusOk},
-            gate, post_gate, epoch, polls, false};
-        scan_allocate<false>(polled, summaries, counts, blocks, n_blocks, reserve);
+        LdsReserve<false> reserve{AllocatorMeta(buffer_meta, max_free_regions, lock_spins),
+                                  descriptor, frees, reinterpret_cast<int32_t *>(stage), {}, -1,
+                                  kStatusOk};
+        book(polled, summaries, counts, blocks, n_blocks, reserve,
+             reinterpret_cast<int32_t *>(slices));
     } else {
         NoReserve reserve;
         const ScanTotals totals =
@@ -155,13 +154,13 @@ __global__ __launch_bounds__(kLanes) void compress_kernel(
         source, side, encoded, base_encode, base_decode, center_out, shifted_decode_out,
         sample_values, sample_size, n_groups, extra_starts, summaries, blocks, counts, control,
         epoch, descriptor, buffer_meta, max_free_regions, frees, host_totals, n_blocks,
-        logical_numel, S, W, lock_spins, polls, blockIdx.x, nullptr, false, stage);
+        logical_numel, S, W, lock_spins, polls, blockIdx.x, SingleBook{}, stage);
 }
 
 // Several BF16 tensors into one TensorBuffer: job j takes workgroups
 // [first_group[j], first_group[j + 1]) and runs the single launch's layout
-// over them with its own control words.  Every wait stays inside one job
-// (plus the gate on job 0, dispatched first), so each job's waits end as in
+// over them with its own control words.  Every wait stays inside one job, plus
+// job 0's for the others' requests (book_batch_job), so each job's waits end as in
 // its own launch.
 template <int kSidePolicy>
 __global__ __launch_bounds__(kLanes) void compress_batch_kernel(CompressBatch batch) {
@@ -171,15 +170,13 @@ __global__ __launch_bounds__(kLanes) void compress_batch_kernel(CompressBatch ba
     for (int k = 1; k < batch.n_jobs; ++k)
         if (w >= batch.first_group[k]) j = k;
     const CompressBatchJob &job = batch.jobs[j];
-    lct_pending_frees frees = batch.frees;
-    if (j != 0) frees.count = 0;
     compress_group<kSidePolicy, false>(
         job.source, job.side, job.encoded, job.base_encode, job.base_decode, job.center_out,
         job.shifted_decode_out, job.sample_values, job.sample_size, job.n_groups,
         job.extra_starts, job.summaries, job.blocks, job.counts, job.control, batch.epoch,
-        job.descriptor, batch.buffer_meta, batch.max_free_regions, frees, nullptr, job.n_blocks,
-        job.logical_numel, batch.steps, job.fixed_words, batch.lock_spins, batch.polls,
-        w - batch.first_group[j], batch.gate, j == 0, stage);
+        job.descriptor, batch.buffer_meta, batch.max_free_regions, batch.frees, nullptr,
+        job.n_blocks, job.logical_numel, batch.steps, job.fixed_words, batch.lock_spins,
+        batch.polls, w - batch.first_group[j], TableBook<CompressBatch>{batch, j}, stage);
 }
 
 }  // namespace
@@ -297,9 +294,9 @@ extern "C" int32_t lct_compress_batch(const lct_compress_job *jobs, int32_t n_jo
     compact.precomputed = 0;
     batch.lock_spins = lock_spins();
     batch.polls = ready_polls();
-    // Word 0 of the control array is the frees' gate; job j's words follow
-    // those of jobs before it.
-    batch.gate = batch.frees.count > 0 ? control : nullptr;
+    static_assert(LCT_MAX_COMPRESS_BATCH <= kMaxBatchJobs, "a request slot per job");
+    // Word 0 of the control array is spare; job j's words follow those of
+    // jobs before it.
     int64_t groups = 0, blocks_total = 0, extra_used = 0, summary_used = 0, control_used = 1;
     size_t lds = static_cast<size_t>(max_free_regions) * 8;
     for (int j = 0; j < n_jobs; ++j) {

@@ -401,9 +401,10 @@ struct LdsReserve {
         }
     }
 
-    int32_t status;   // the reservation's status (uniform after finish)
+    int32_t status;   // the last reservation's status (uniform after reserve)
 
-    __device__ void finish(int32_t request, int32_t *scratch, bool incomplete) {
+    // One tensor's reservation on the LDS copy, and its descriptor.
+    __device__ void reserve(int32_t *into, int32_t request, int32_t *scratch, bool incomplete) {
         const int t = threadIdx.x;
         // An incomplete scan (summaries that did not arrive) gives status 7
         // whatever the reservation did, since its request may be short: a
@@ -412,29 +413,35 @@ struct LdsReserve {
         if (held < 0) {
             outcome = kStatusLock;
             if (t == 0) {
-                descriptor[0] = -1;
-                descriptor[1] = 0;
-                descriptor[3] = -1;
+                into[0] = -1;
+                into[1] = 0;
+                into[3] = -1;
             }
         } else {
             int32_t out[3];
             lds_reserve(f, request, scratch, out);
-            if (kPublishAll)
-                lds_write_back(f, meta);
-            else
-                lds_write_back_coherent(f, meta);
             outcome = out[2];
             if (t == 0) {
-                descriptor[0] = out[0];
-                descriptor[1] = out[1];
-                descriptor[3] = f.generation;
+                into[0] = out[0];
+                into[1] = out[1];
+                into[3] = f.generation;
             }
         }
         status = incomplete ? kStatusIncomplete : outcome;
         if (t == 0) {
-            descriptor[2] = status;
+            into[2] = status;
             const int32_t bits = failure_bits(outcome, request) | (incomplete ? kFailIncomplete : 0);
             if (bits != 0) record_failure(meta, bits);
+        }
+    }
+
+    // The list back to the buffer and the lock released.
+    __device__ void close() {
+        if (held >= 0) {
+            if (kPublishAll)
+                lds_write_back(f, meta);
+            else
+                lds_write_back_coherent(f, meta);
         }
         if (kPublishAll) {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
@@ -446,47 +453,107 @@ struct LdsReserve {
             __atomic_signal_fence(__ATOMIC_SEQ_CST);
         }
         __syncthreads();
-        if (held >= 0 && t == 0)
+        if (held >= 0 && threadIdx.x == 0)
             __hip_atomic_store(meta.lock, held + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-};
-
-// The arena reservation of one tensor of a batched launch (compress or
-// fused update).  The batch's deferred frees belong to job 0, whose bookkeeping applies them right after it takes the
-// lock and then posts `gate`; the other jobs' bookkeeping waits for that word
-// (bounded) before it asks for the lock, so every reservation of the batch
-// follows the frees, as the reservations of consecutive single launches would.
-// Job 0 is dispatched first and waits for nothing of the later jobs.  A gate
-// that does not arrive marks the tensor incomplete.  gate == nullptr (no
-// frees): plain LdsReserve.
-struct GatedReserve {
-    LdsReserve<false> inner;
-    uint64_t *gate;
-    bool post;
-    uint32_t epoch;
-    int32_t polls;
-    bool late;
-
-    __device__ void begin(int32_t *scratch) {
-        __shared__ int32_t arrived;
-        if (gate != nullptr && !post) {
-            if (threadIdx.x == 0) {
-                uint64_t word = control_load(gate);
-                for (int i = 0; !tagged_with(word, epoch) && i < polls; ++i) {
-                    __builtin_amdgcn_s_sleep(8);
-                    word = control_load(gate);
-                }
-                arrived = tagged_with(word, epoch) ? 1 : 0;
-            }
-            __syncthreads();
-            late = arrived == 0;
-        }
-        inner.begin(scratch);
-        if (gate != nullptr && post && threadIdx.x == 0) control_store(gate, tagged_word(epoch, 1));
     }
 
     __device__ void finish(int32_t request, int32_t *scratch, bool incomplete) {
-        inner.finish(request, scratch, incomplete || late);
+        reserve(descriptor, request, scratch, incomplete);
+        close();
+    }
+};
+
+// The overflow bookkeeping of the tensors of a batched launch (compress or
+// fused update).  Each job's first workgroup scans its own job's summaries,
+// all jobs side by side, and posts the bytes it needs; job 0's then makes
+// every job's reservation, in job order and under one hold of the arena lock
+// that the deferred frees open, so each follows the frees, as the
+// reservations of consecutive single launches would.  (With each job taking
+// the lock in turn, eight updates of 18 blocks spent 45 us after their last
+// block handing it on: 85 us for the launch, about 40 of them encoding.)
+// Job 0 is dispatched first, and the words it waits for come from workgroups
+// that wait only for their own job's; a request that does not arrive within
+// the poll limit counts as incomplete.
+//
+// The request goes into word 0 of the job's own control array, where sample
+// group 0 posted its partial sum: every block of the job has read that before
+// it posts the summary that the scan waited for (a block that has not makes
+// the scan incomplete, and stays without a center).  Its tag differs from the
+// launch's by the top bit, so the partial sum is never taken for it.
+struct BatchJob {
+    int32_t *descriptor;
+    uint64_t *control;
+};
+
+constexpr int kMaxBatchJobs = 32;
+constexpr int kBatchWords = kMaxBatchJobs + kWavesPerBlock;   // LDS ints book_batch_job uses
+constexpr uint32_t kRequestTag = 0x80000000u;                 // flips the epoch's top bit
+constexpr uint32_t kIncompleteRequest = 0x80000000u;          // with the request's bytes
+
+// Workgroup-wide; contains barriers.  `words`: kBatchWords ints of LDS;
+// job_of(k): job k's BatchJob.
+template <class JobOf>
+__device__ __forceinline__ void book_batch_job(int32_t job, int32_t n_jobs, JobOf job_of,
+                                               PolledSummaries &polled,
+                                               int32_t *__restrict__ summaries,
+                                               int32_t *__restrict__ counts,
+                                               int32_t *__restrict__ blocks, int32_t n_blocks,
+                                               LdsReserve<false> &arena, int32_t *words) {
+    int32_t *const scratch = words + kMaxBatchJobs;
+    const uint32_t tag = polled.epoch ^ kRequestTag;
+    if (job == 0) arena.begin(scratch);
+    NoReserve none;
+    const ScanTotals totals =
+        scan_allocate<false>(polled, summaries, counts, blocks, n_blocks, none);
+    const int t = threadIdx.x;
+    if (t == 0)
+        control_store(job_of(job).control,
+                      tagged_word(tag, static_cast<uint32_t>(totals.bytes + 2 * totals.entries)
+                                           | (totals.incomplete ? kIncompleteRequest : 0u)));
+    if (job != 0) return;
+    if (t < n_jobs) {
+        const uint64_t *const posted = job_of(t).control;
+        uint64_t word = control_load(posted);
+        for (int i = 0; !tagged_with(word, tag) && i < polled.polls; ++i) {
+            __builtin_amdgcn_s_sleep(2);
+            word = control_load(posted);
+        }
+        words[t] = static_cast<int32_t>(tagged_with(word, tag) ? static_cast<uint32_t>(word)
+                                                               : kIncompleteRequest);
+    }
+    __syncthreads();
+    for (int k = 0; k < n_jobs; ++k) {
+        const uint32_t value = static_cast<uint32_t>(words[k]);
+        arena.reserve(job_of(k).descriptor, static_cast<int32_t>(value & ~kIncompleteRequest),
+                      scratch, (value & kIncompleteRequest) != 0);
+        __syncthreads();   // the list's entries before the next job's search
+    }
+    arena.close();
+}
+
+// The two forms of a buffered encoder's bookkeeping: a launch of one tensor,
+// and job `job` of a table of them.
+struct SingleBook {
+    __device__ void operator()(PolledSummaries &polled, int32_t *summaries, int32_t *counts,
+                               int32_t *blocks, int32_t n_blocks, LdsReserve<false> &arena,
+                               int32_t *) const {
+        scan_allocate<false>(polled, summaries, counts, blocks, n_blocks, arena);
+    }
+};
+
+template <class Table>
+struct TableBook {
+    const Table &table;
+    int32_t job;
+
+    __device__ void operator()(PolledSummaries &polled, int32_t *summaries, int32_t *counts,
+                               int32_t *blocks, int32_t n_blocks, LdsReserve<false> &arena,
+                               int32_t *words) const {
+        const Table &jobs = table;
+        book_batch_job(
+            job, jobs.n_jobs,
+            [&](int k) { return BatchJob{jobs.jobs[k].descriptor, jobs.jobs[k].control}; },
+            polled, summaries, counts, blocks, n_blocks, arena, words);
     }
 };
 

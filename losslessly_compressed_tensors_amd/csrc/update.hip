@@ -82,8 +82,6 @@ struct KernelBookkeeping {
     lct_pending_frees frees;
     int32_t lock_spins;
     int32_t polls;
-    uint64_t *gate;      // batched launches: GatedReserve's word (nullptr: none)
-    int32_t post_gate;   // this job applies the frees and posts the gate
     // In-launch center sampling of the two-operand launch (sample_groups > 0):
     // workgroups g < sample_groups publish sample group g's partial sums in
     // control[g] (tagged), and every block reads the center from there
@@ -140,11 +138,12 @@ __device__ __forceinline__ void store_shifted_decode(int32_t *__restrict__ out,
 // the free list in `lds_free_list` (the payload stage, free by now), the
 // polled scan into the block metadata and the overflow-block list, and the
 // reservation (lct_prefix_allocate / lct_allocate_compact's results).
-template <bool kBooked>
+template <bool kBooked, class Book>
 __device__ __forceinline__ void publish_block(const KernelBookkeeping &bk,
                                               int32_t *__restrict__ summaries, int64_t block,
                                               int64_t n_blocks, int32_t count, int32_t bytes,
-                                              int32_t *lds_free_list, bool failed = false) {
+                                              int32_t *lds_free_list, int32_t *lds_words,
+                                              Book book, bool failed = false) {
     if (!kBooked) {
         if (threadIdx.x == 0) {
             summaries[block] = count;
@@ -163,12 +162,11 @@ __device__ __forceinline__ void publish_block(const KernelBookkeeping &bk,
     if (block != 0) return;
     PolledSummaries polled{bk.control, bk.epoch, static_cast<int32_t>(n_blocks), bk.polls, false};
     if (bk.buffer_meta != nullptr) {
-        GatedReserve reserve{
-            LdsReserve<false>{AllocatorMeta(bk.buffer_meta, bk.max_free_regions, bk.lock_spins),
-                              bk.descriptor, bk.frees, lds_free_list, {}, -1, kStatusOk},
-            bk.gate, bk.post_gate != 0, bk.epoch, bk.polls, false};
-        scan_allocate<false>(polled, summaries, bk.counts, bk.blocks,
-                             static_cast<int32_t>(n_blocks), reserve);
+        LdsReserve<false> reserve{
+            AllocatorMeta(bk.buffer_meta, bk.max_free_regions, bk.lock_spins), bk.descriptor,
+            bk.frees, lds_free_list, {}, -1, kStatusOk};
+        book(polled, summaries, bk.counts, bk.blocks, static_cast<int32_t>(n_blocks), reserve,
+             lds_words);
     } else {
         NoReserve reserve;
         scan_allocate<false>(polled, summaries, bk.counts, bk.blocks,
@@ -497,7 +495,7 @@ __device__ __forceinline__ void update_rows(UpdateWalk &u, const SideChunk &firs
 
 // Codec block `block` of one fused update (the single launch's blockIdx.x);
 // `stage`: the dynamic LDS, register_stage_bytes(W) (rows 3..W-1 of A's payload).
-template <bool kBooked>
+template <bool kBooked, class Book>
 __device__ __forceinline__ void pointwise_encode_block(
     const OperandA &a, const uint16_t *__restrict__ other, const OpArgs &args,
     const int32_t *__restrict__ partials, int32_t n_groups,
@@ -506,7 +504,7 @@ __device__ __forceinline__ void pointwise_encode_block(
     uint8_t *__restrict__ side_out, int32_t *__restrict__ encoded_out,
     uint8_t *__restrict__ extra_starts, int32_t *__restrict__ summaries,
     uint8_t *__restrict__ exponents, int64_t n_blocks, int64_t logical_numel, int S, int W,
-    int rare, const KernelBookkeeping &bk, int64_t block, uint32_t *stage) {
+    int rare, const KernelBookkeeping &bk, int64_t block, uint32_t *stage, Book book) {
     __shared__ QuadTables tb;
     __shared__ uint2 enc[256];
     __shared__ int32_t scratch[kWavesPerBlock];
@@ -594,7 +592,7 @@ __device__ __forceinline__ void pointwise_encode_block(
     // 256 x 256): one block scan.
     const int32_t both = block_sum(overflow ? (S - extra) | (1 << 20) : 0, scratch);
     publish_block<kBooked>(bk, summaries, block, n_blocks, both >> 20, both & 0xFFFFF,
-                           reinterpret_cast<int32_t *>(stage));
+                           reinterpret_cast<int32_t *>(stage), map_start, book);
 }
 
 template <bool kBooked>
@@ -611,7 +609,7 @@ __global__ __launch_bounds__(kLanes) void pointwise_encode_kernel(
     pointwise_encode_block<kBooked>(a, other, args, partials, n_groups, base_encode, base_decode,
                                     center_out, shifted_decode_out, side_out, encoded_out,
                                     extra_starts, summaries, exponents, n_blocks, logical_numel,
-                                    S, W, rare, bk, blockIdx.x, stage);
+                                    S, W, rare, bk, blockIdx.x, stage, SingleBook{});
 }
 
 // ---- several fused updates of one operation in three launches
@@ -691,8 +689,7 @@ struct UpdateEncodeBatch {
     OpArgs args;
     int32_t *buffer_meta;
     int32_t max_free_regions;
-    lct_pending_frees frees;   // job 0 applies them
-    uint64_t *gate;            // nullptr without frees
+    lct_pending_frees frees;
     uint32_t epoch;
     int32_t lock_spins;
     int32_t polls;
@@ -707,14 +704,14 @@ __global__ __launch_bounds__(kLanes) void pointwise_encode_batch_kernel(UpdateEn
     const UpdateEncodeJob &job = batch.jobs[j];
     KernelBookkeeping bk{job.control, batch.epoch, job.counts, job.blocks, job.descriptor,
                          batch.buffer_meta, batch.max_free_regions, batch.frees,
-                         batch.lock_spins, batch.polls, batch.gate, j == 0 ? 1 : 0};
-    if (j != 0) bk.frees.count = 0;
+                         batch.lock_spins, batch.polls};
     pointwise_encode_block<true>(job.a, job.other, batch.args, job.partials, job.n_groups,
                                  job.base_encode, job.base_decode, job.center_out,
                                  job.shifted_decode_out, job.side_out, job.encoded_out,
                                  job.extra_starts, job.summaries, job.exponents, job.n_blocks,
                                  job.logical_numel, job.steps, job.fixed_words, job.rare, bk,
-                                 w - batch.first_block[j], stage);
+                                 w - batch.first_block[j], stage,
+                                 TableBook<UpdateEncodeBatch>{batch, j});
 }
 
 // ---- the two-compressed form: alpha * A + B with compressed output
@@ -1121,7 +1118,8 @@ __global__ __launch_bounds__(kLanes) void dual_encode_kernel(
     // 256 x 256): one block scan.
     const int32_t both = block_sum(overflow ? (S - extra) | (1 << 20) : 0, scratch);
     publish_block<kBooked>(bk, summaries, block, n_blocks, both >> 20, both & 0xFFFFF,
-                           reinterpret_cast<int32_t *>(stages), center_failed);
+                           reinterpret_cast<int32_t *>(stages), map_start, SingleBook{},
+                           center_failed);
 }
 
 int32_t check_operand(const int32_t *encoded, const uint8_t *side, const int32_t *shifted_decode,
@@ -1476,8 +1474,7 @@ extern "C" int32_t lct_pointwise_update_batch(
     encode.epoch = epoch;
     encode.lock_spins = lock_spins();
     encode.polls = ready_polls();
-    // Word 0 of the control array is the frees' gate; job j's words follow.
-    encode.gate = encode.frees.count > 0 ? control : nullptr;
+    static_assert(LCT_MAX_UPDATE_BATCH <= kMaxBatchJobs, "a request slot per job");
     compact.arena = arena;
     compact.steps = 0;
     compact.precomputed = 1;
