@@ -532,11 +532,13 @@ __device__ __forceinline__ void book_batch_job(int32_t job, int32_t n_jobs, JobO
 }
 
 // The two forms of a buffered encoder's bookkeeping: a launch of one tensor,
-// and job `job` of a table of them.
+// and job `job` of a table of them.  Inlined always: called out of line, they
+// cost the compress 5 us at every grid (a call frame in scratch memory).
 struct SingleBook {
-    __device__ void operator()(PolledSummaries &polled, int32_t *summaries, int32_t *counts,
-                               int32_t *blocks, int32_t n_blocks, LdsReserve<false> &arena,
-                               int32_t *) const {
+    __device__ __forceinline__ void operator()(PolledSummaries &polled, int32_t *summaries,
+                                               int32_t *counts, int32_t *blocks,
+                                               int32_t n_blocks, LdsReserve<false> &arena,
+                                               int32_t *) const {
         scan_allocate<false>(polled, summaries, counts, blocks, n_blocks, arena);
     }
 };
@@ -546,9 +548,10 @@ struct TableBook {
     const Table &table;
     int32_t job;
 
-    __device__ void operator()(PolledSummaries &polled, int32_t *summaries, int32_t *counts,
-                               int32_t *blocks, int32_t n_blocks, LdsReserve<false> &arena,
-                               int32_t *words) const {
+    __device__ __forceinline__ void operator()(PolledSummaries &polled, int32_t *summaries,
+                                               int32_t *counts, int32_t *blocks,
+                                               int32_t n_blocks, LdsReserve<false> &arena,
+                                               int32_t *words) const {
         const Table &jobs = table;
         book_batch_job(
             job, jobs.n_jobs,
