@@ -781,12 +781,12 @@ def main() -> int:
         "copy_gbps": round(2 * nbytes / (copy_ms * 1e-3) / 1e9, 1),
         "roofline": {
             "bound": "hbm",
-            "kernel": "decode_kernel",
+            "kernel": "decode_kernel_grouped",
             "achieved": round(dec_alg / (kernel_ms * 1e-3) / 1e9, 1),
             "peak": HBM_PEAK_GBPS,
             "unit": "GB/s",
             "frac": round(dec_alg / (kernel_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4),
-            "traffic": measured_traffic("decode_kernel", nb),
+            "traffic": measured_traffic("decode_kernel_grouped", nb),
             "traffic_source": TRAFFIC_PROFILE.relative_to(ROOT).as_posix(),
             "algorithmic_bytes": dec_alg,
             "kernel_us": round(kernel_ms * 1e3, 2),

@@ -37,9 +37,9 @@
 // quads): pointwise_encode_kernel 64.0 -> 61.1 us at 688 blocks, 38.2 -> 36.2
 // at one; dual_encode_kernel 75.6 -> 69.2 and 46.7 -> 43.0.  A ragged tensor's
 // last block runs the same loop (the whole momentum step at 767 blocks, ragged:
-// 75.8 us, against 150 us with a separate loop for partial blocks).  The three waves a SIMD holds
-// keep its VALU 75% busy (203 and 275 instructions per 8 steps); the rest is
-// waits for the lookups' LDS round trips.
+// 75.8 us, against 150 us with a separate loop for partial blocks).  With 203
+// and 275 VALU instructions per 8 steps and 2.7 waves per SIMD, the VALU is 44
+// and 55% busy; the rest is waits for the lookups' LDS round trips.
 #include <algorithm>
 
 #include "batch.h"
