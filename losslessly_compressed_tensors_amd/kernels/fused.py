@@ -17,6 +17,7 @@ from . import hip
 
 _PLAIN = (Tensor, torch.nn.Parameter)
 _MAX_COLUMNS = 4096
+_MAX_ELEMENTS = 1 << 33   # keeps every row count within the entry points' 2^31
 # Row groups of the partial sums: the most that lct_column_sum and
 # lct_rms_norm_backward make.
 _COLUMN_GROUPS = 128
@@ -50,7 +51,7 @@ def _stream(tensor: Tensor) -> int:
 
 def relu_square(z: Tensor):
     """``(relu(z), relu(z)^2)``, or None."""
-    if z.dtype != torch.bfloat16 or not native(z):
+    if z.dtype != torch.bfloat16 or z.numel() > _MAX_ELEMENTS or not native(z):
         return None
     relu, square = torch.empty_like(z), torch.empty_like(z)
     hip.call("lct_relu_square", z.data_ptr(), relu.data_ptr(), square.data_ptr(), z.numel(),
@@ -74,7 +75,7 @@ def column_sum(g: Tensor, dtype: torch.dtype):
     """``g.sum(0).to(dtype)`` of a matrix, or None."""
     if (g.dtype != torch.bfloat16 or dtype not in (torch.bfloat16, torch.float32) or g.ndim != 2
             or g.shape[0] < _MIN_SUM_ROWS or g.shape[1] % 8 or not 0 < g.shape[1] <= 1 << 20
-            or not native(g)):
+            or g.numel() > _MAX_ELEMENTS or not native(g)):
         return None
     rows, cols = g.shape
     partials = torch.empty(_COLUMN_GROUPS * cols, dtype=torch.float32, device=g.device)
@@ -87,7 +88,7 @@ def column_sum(g: Tensor, dtype: torch.dtype):
 def _norm_takes(x: Tensor, gain: Tensor) -> bool:
     return (x.dtype == torch.bfloat16 and gain.dtype in (torch.bfloat16, torch.float32)
             and x.ndim > 0 and gain.shape == x.shape[-1:] and x.shape[-1] % 4 == 0
-            and x.shape[-1] <= _MAX_COLUMNS)
+            and x.shape[-1] <= _MAX_COLUMNS and x.numel() <= _MAX_ELEMENTS)
 
 
 # lct_skinny_linear's range of A's rows.
