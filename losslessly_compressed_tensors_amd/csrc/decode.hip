@@ -495,9 +495,10 @@ __global__ __launch_bounds__(kLanes, 8) void decode_kernel_compact(
 //    next four rows, and those past its symbol count are overwritten later;
 //  * rows at and past a stream's overflow start are then filled from its tail;
 //  * the wave joins the tile's rows with their side bytes, fetched one tile
-//    ahead: lane j takes 8 columns of row 8 (j >> 3) + 2 i + h for i < 4,
-//    h < 2, so the swizzle's XOR within the 8 columns is the constant 2 i and
-//    every wave store is 8 whole 128-byte lines;
+//    ahead: lane j takes 8 columns of the four rows 4 (8 u + (j >> 3)) + i of
+//    each 32-row unit u, so a 16-byte read of the tile holds four columns of
+//    all four rows, the swizzle's XOR by i is a change of the output's words
+//    and every wave store is 8 whole 128-byte lines;
 //  * rows already decoded past the tile's end move to its start.
 // The tensor's last, partial block differs only in its streams' ends and in
 // the stores of the piece that holds the tensor's end.
@@ -632,12 +633,35 @@ struct GroupSides {
     uint2 q[kUnits][4];
 };
 
+// Offset of thread `thread`'s first unit within a row of the block's side
+// bytes; out of range for a tile past the block's last (the fetch one tile
+// ahead of the last one).
+constexpr uint32_t group_side_offset(uint32_t thread, int first_step, int S) {
+    const uint32_t j = thread & (kWave - 1);
+    return first_step < S ? (j >> 3) * (4 * kLanes) + (thread & ~(kWave - 1u)) + (j & 7) * 8
+                          : kOutOfRange;
+}
+
+// Whether every fetch of a block, the one past its end among them, reads
+// inside its S rows or is out of range by its VGPR offset alone.
+constexpr bool group_sides_in_block(int S) {
+    for (int first = 0; first <= S; first += kTileSteps)
+        for (uint32_t thread = 0; thread < kLanes; ++thread) {
+            const uint32_t offset = group_side_offset(thread, first, S);
+            const uint32_t last = static_cast<uint32_t>(first + 32 * (kUnits - 1) + 3) * kLanes;
+            if (offset != kOutOfRange && offset + last + 8 > static_cast<uint32_t>(S) * kLanes)
+                return false;
+        }
+    return true;
+}
+static_assert(group_sides_in_block(128) && group_sides_in_block(256),
+              "the side bytes' prefetch stays inside the block");
+
 // The side bytes of this lane's units of the tile at `first_step` (0 past the
 // block's end).
-__device__ __forceinline__ void fetch_group_sides(GroupSides &s,
-                                                  __amdgpu_buffer_rsrc_t side, int first_step) {
-    const uint32_t j = threadIdx.x & (kWave - 1);
-    const uint32_t voffset = (j >> 3) * (4 * kLanes) + (threadIdx.x & ~(kWave - 1u)) + (j & 7) * 8;
+__device__ __forceinline__ void fetch_group_sides(GroupSides &s, __amdgpu_buffer_rsrc_t side,
+                                                  int first_step, int S) {
+    const uint32_t voffset = group_side_offset(threadIdx.x, first_step, S);
 #pragma unroll
     for (int u = 0; u < kUnits; ++u)
 #pragma unroll
@@ -727,7 +751,7 @@ __device__ __forceinline__ void decode_block_grouped(
     stage_payload_rows(stage, encoded, n_blocks * kLanes, block, kRegisterRows, W);
     const OverlayHead head = load_overlay_head(ov, has_overlay != 0, block, n_blocks);
     GroupSides sides;
-    fetch_group_sides(sides, side_rsrc, 0);
+    fetch_group_sides(sides, side_rsrc, 0, S);
     build_group_tables(tb, base, packed);
     const LaneOverlay lane = build_overlay(ov, head, S, map_start, map_offset, scratch, tail_lds,
                                            kTailLds);
@@ -809,8 +833,7 @@ __device__ __forceinline__ void decode_block_grouped(
             }
         }
         GroupSides next;
-        const int ahead = first + kTileSteps;
-        fetch_group_sides(next, side_rsrc, ahead);
+        fetch_group_sides(next, side_rsrc, first + kTileSteps, S);
         __builtin_amdgcn_wave_barrier();
         store_tile(tile, sides, out_rsrc, first, row_base, full, valid);
         __builtin_amdgcn_wave_barrier();

@@ -33,6 +33,11 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, ui
                                              kBufferConfig);
 }
 
+// Offset (in the VGPR) rejected by the range check of every resource used here
+// (num_records < 2^31): loads return 0, stores are dropped.  An offset that is
+// past the end only with its soffset added is not relied on to be rejected.
+constexpr uint32_t kOutOfRange = 0x80000000u;
+
 // 16-byte buffer store with the whole offset in the VGPR and soffset 0.
 // A store of more than 8 bytes reads its data VGPRs after issue, and a VALU
 // write to them must wait one cycle; the compiler inserts that wait only when

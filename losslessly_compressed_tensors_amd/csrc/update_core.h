@@ -194,10 +194,6 @@ __device__ __forceinline__ void overlay_half(const LaneOverlay &lane, const uint
     settle(f[4], f[5], f[6], f[7]);
 }
 
-// Buffer offset rejected by the range check of every resource used here
-// (num_records < 2^31): loads return 0, stores are dropped.
-constexpr uint32_t kOutOfRange = 0x80000000u;
-
 // Encoder state of one lane's output stream.  Word r of the stream is at byte
 // r * row_bytes + 4 * lane of the block's payload resource.  pos counts the
 // bits of every pair so far, so once a pair does not fit, pos stays above the
