@@ -99,6 +99,7 @@ def skinny_linear(a: Tensor, w: Tensor):
     """``a @ w.T`` of at most 16 rows, or None (from there on the library's
     product is faster: 21 us against 28 at 17 to 32 rows of 11008 x 4096)."""
     if (a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or a.ndim != 2
+            or w.ndim != 2 or w.shape[1] != a.shape[1]
             or a.shape[0] > MAX_SKINNY_TOKENS or a.shape[1] % 8
             or max(w.shape) > 1 << 30 or not native(a, w)):
         return None

@@ -1,0 +1,41 @@
+"""CPU: which tensors the fused dense kernels take (``kernels/fused.py``), with
+the device and the launch stood in for."""
+from __future__ import annotations
+
+import types
+
+import pytest
+import torch
+
+from losslessly_compressed_tensors_amd import operations
+from losslessly_compressed_tensors_amd.kernels import fused
+
+
+@pytest.fixture
+def no_launch(monkeypatch):
+    """Every tensor counts as the kernels' own; a launch fails the test."""
+    monkeypatch.setattr(fused, "native", lambda *tensors: True)
+    monkeypatch.setattr(fused, "_stream", lambda tensor: 0)
+    monkeypatch.setattr(fused.hip, "call", lambda name, *args: pytest.fail(f"launched {name}"))
+
+
+@pytest.mark.parametrize("shape", [(5, 8, 3), (5, 8, 8), (2, 8, 5, 3)])
+@pytest.mark.filterwarnings("ignore:The use of `x.T`")
+def test_few_row_product_takes_matrices_only(no_launch, monkeypatch, shape):
+    """A weight of more dimensions keeps the library's broadcast product."""
+    a = torch.randn(4, 8).to(torch.bfloat16)
+    w = torch.randn(shape).to(torch.bfloat16)
+    assert fused.skinny_linear(a, w) is None
+    monkeypatch.setattr(operations, "decompress", lambda record: w)
+    try:
+        expected = a @ w.T
+    except RuntimeError as error:     # refused before, refused the same way
+        with pytest.raises(type(error)):
+            operations.A_compBT(a, types.SimpleNamespace(shape=w.shape))
+        return
+    assert torch.equal(operations.A_compBT(a, types.SimpleNamespace(shape=w.shape)), expected)
+
+
+def test_few_row_product_takes_matching_columns_only(no_launch):
+    a = torch.zeros(4, 8, dtype=torch.bfloat16)
+    assert fused.skinny_linear(a, torch.zeros(5, 16, dtype=torch.bfloat16)) is None
