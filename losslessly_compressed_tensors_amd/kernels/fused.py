@@ -38,11 +38,12 @@ def native(*tensors: Tensor) -> bool:
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:
-        if (type(t) not in _PLAIN or not t.is_cuda or not t.is_contiguous() or t.numel() == 0
+        if (type(t) not in _PLAIN or not t.is_cuda or t.get_device() != torch._C._cuda_getDevice()
+                or not t.is_contiguous() or t.numel() == 0
                 or (grad and t.requires_grad) or torch._C._functorch.is_functorch_wrapped_tensor(t)
                 or t.data_ptr() & 15 or t.is_conj() or t.is_neg()):
             return False
-    return tensors[0].get_device() == torch._C._cuda_getDevice()
+    return True
 
 
 def _stream(tensor: Tensor) -> int:
@@ -131,7 +132,7 @@ def rms_norm_backward(grad: Tensor, x: Tensor, rstd: Tensor, gain: Tensor, dtype
     if (not _norm_takes(x, gain) or grad.dtype != torch.bfloat16 or grad.shape != x.shape
             or rstd.dtype != torch.float32 or rstd.numel() * x.shape[-1] != x.numel()
             or dtype not in (torch.bfloat16, torch.float32)
-            or not native(grad, x, gain) or not native(rstd)):
+            or not native(grad, x, gain, rstd)):
         return None
     cols = x.shape[-1]
     grad_x = torch.empty_like(x)

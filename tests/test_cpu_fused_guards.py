@@ -39,3 +39,52 @@ def test_few_row_product_takes_matrices_only(no_launch, monkeypatch, shape):
 def test_few_row_product_takes_matching_columns_only(no_launch):
     a = torch.zeros(4, 8, dtype=torch.bfloat16)
     assert fused.skinny_linear(a, torch.zeros(5, 16, dtype=torch.bfloat16)) is None
+
+
+class _DeviceTensor:
+    """What ``native`` asks of a tensor, for one on device ``index``."""
+
+    is_cuda = True
+    requires_grad = False
+
+    def __init__(self, index: int = 0):
+        self.index = index
+
+    def get_device(self):
+        return self.index
+
+    def is_contiguous(self):
+        return True
+
+    def numel(self):
+        return 8
+
+    def data_ptr(self):
+        return 1 << 20
+
+    def is_conj(self):
+        return False
+
+    is_neg = is_conj
+
+
+@pytest.fixture
+def device_tensors(monkeypatch):
+    """``native`` on stand-ins for device tensors, the current device being 0."""
+    monkeypatch.setattr(fused, "_PLAIN", (_DeviceTensor,))
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0, raising=False)
+    monkeypatch.setattr(torch._C._functorch, "is_functorch_wrapped_tensor", lambda tensor: False)
+    return _DeviceTensor
+
+
+def test_every_tensor_is_on_the_current_device(device_tensors):
+    here, there = device_tensors(0), device_tensors(1)
+    assert fused.native(here) and fused.native(here, here, here)
+    assert not fused.native(there)
+    assert not fused.native(here, there)
+    assert not fused.native(here, here, there)
+    assert not fused.native(there, here)
+
+
+def test_host_tensors_are_left_to_aten():
+    assert not fused.native(torch.zeros(8))     # also without any device
