@@ -33,8 +33,9 @@ def native(*tensors: Tensor) -> bool:
     contiguous device tensors of the current device, with no autograd graph,
     forward-mode level, transform, dispatch mode, autocast or tracing that
     would have to see the operations."""
-    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
-            or forward_ad._current_level >= 0 or torch.is_autocast_enabled("cuda")):
+    if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
+            or torch._C._len_torch_dispatch_stack() or forward_ad._current_level >= 0
+            or torch.is_autocast_enabled("cuda")):
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:

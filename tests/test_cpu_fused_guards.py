@@ -88,3 +88,28 @@ def test_every_tensor_is_on_the_current_device(device_tensors):
 
 def test_host_tensors_are_left_to_aten():
     assert not fused.native(torch.zeros(8))     # also without any device
+
+
+@pytest.mark.filterwarnings("ignore::DeprecationWarning")
+def test_tracing_and_transforms_see_atens_operations(device_tensors, monkeypatch):
+    x = device_tensors()
+    assert fused.native(x)
+    seen = []
+
+    def traced(value):
+        seen.append(fused.native(x))
+        return value + 1
+
+    torch.jit.trace(traced, (torch.zeros(2),), check_trace=False)
+    assert seen and not any(seen)
+    with torch.autograd.forward_ad.dual_level():
+        assert not fused.native(x)
+
+    class Mode(torch.utils._python_dispatch.TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        assert not fused.native(x)
+    monkeypatch.setattr(torch._C._functorch, "is_functorch_wrapped_tensor", lambda tensor: True)
+    assert not fused.native(x)                  # vmap, grad and the other transforms

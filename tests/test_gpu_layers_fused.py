@@ -5,6 +5,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+from losslessly_compressed_tensors_amd.components import ops
 from losslessly_compressed_tensors_amd.kernels import fused
 
 pytestmark = pytest.mark.gpu
@@ -99,3 +100,13 @@ def test_what_the_kernels_leave_to_aten():
     assert fused.column_sum(_values(1023, 16), torch.float32) is None   # ATen is faster
     assert fused.rms_norm(_values(8, 4100), _values(4100)) is None
     assert fused.rms_norm(_values(8, 256), _values(1, 256)) is None
+
+
+@pytest.mark.filterwarnings("ignore::DeprecationWarning")
+def test_a_trace_records_the_operations():
+    """A traced norm computes its own inputs' norm."""
+    first, x, gain = _values(64, 256), _values(64, 256, seed=1), 1 + 0.1 * _values(256, seed=2)
+    traced = torch.jit.trace(lambda t: ops.rms_norm(t, gain), (first,))
+    y, rstd = torch.ops.aten._fused_rms_norm.default(x, [256], gain, None)
+    again = traced(x)
+    assert torch.equal(again[0], y) and torch.equal(again[1], rstd)
