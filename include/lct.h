@@ -754,7 +754,7 @@ int32_t lct_set_decoder(int32_t mode);
  * lct_relu_square: relu = max(z, 0) (NaN kept, -0 gives 0), square =
  * bf16(relu^2).  lct_relu_square_backward: grad = bf16(grad * bf16(2 relu))
  * where relu is not zero, else 0, in place, and square = bf16(relu^2).
- * Pointers 16-byte aligned, any n up to 2^38. */
+ * Pointers 16-byte aligned, any n up to 2^35 - 2048. */
 int32_t lct_relu_square(const void *z, void *relu, void *square, int64_t n, hipStream_t stream);
 int32_t lct_relu_square_backward(const void *relu, void *grad, void *square, int64_t n,
                                  hipStream_t stream);
@@ -767,11 +767,12 @@ int32_t lct_relu_square_backward(const void *relu, void *grad, void *square, int
 int32_t lct_column_sum(const void *g, int64_t rows, int32_t cols, float *partials,
                        int64_t partial_floats, void *out, int32_t out_bf16, hipStream_t stream);
 
-/* RMSNorm over rows of cols values (a multiple of 4 up to 4096; 8-byte
- * aligned): rstd[r] = 1 / sqrt(mean(x^2) + 2^-23), y = bf16(x * rstd * gain).
- * The gain (cols values, BF16 if gain_bf16 != 0, else FP32 and then 16-byte
- * aligned) is rounded to BF16.  lct_rms_norm_backward: grad_x, grad_gain (rounded to BF16; stored as
- * BF16 or FP32) and, where normalized is not NULL, y again.  partials:
+/* RMSNorm over rows (forward: up to 2^26 - 4; backward: up to 2^31) of cols
+ * values (a multiple of 4 up to 4096; 8-byte aligned): rstd[r] = 1 / sqrt(
+ * mean(x^2) + 2^-23), y = bf16(x * rstd * gain).  The gain (cols values, BF16 if
+ * gain_bf16 != 0, else FP32 and then 16-byte aligned) is rounded to BF16.
+ * lct_rms_norm_backward: grad_x, grad_gain (rounded to BF16; stored as BF16 or
+ * FP32) and, where normalized is not NULL, y again.  partials:
  * partial_floats >= cols working values, up to 512 cols of them used. */
 int32_t lct_rms_norm(const void *x, const void *gain, int32_t gain_bf16, void *y, float *rstd,
                      int64_t rows, int32_t cols, hipStream_t stream);
@@ -783,7 +784,8 @@ int32_t lct_rms_norm_backward(const void *grad, const void *x, const float *rstd
 
 /* ---- out = A W^T for at most LCT_MAX_SKINNY_TOKENS rows of A against a dense
  * W [rows, cols] (LCT/operations.py:31-48): contiguous BF16, FP32 sums, one
- * rounding.  cols: a multiple of 8; a and w 16-byte aligned. */
+ * rounding.  rows: up to 2^29 - 64; cols: a multiple of 8 up to 2^30; a and w
+ * 16-byte aligned. */
 #define LCT_MAX_SKINNY_TOKENS 16
 int32_t lct_skinny_linear(const void *a, const void *w, void *out, int32_t tokens, int32_t rows,
                           int32_t cols, hipStream_t stream);

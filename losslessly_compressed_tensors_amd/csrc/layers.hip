@@ -369,8 +369,11 @@ bool aligned(const void *p, uintptr_t bytes) {
 }
 
 constexpr int32_t kMaxColumns = 4096;          // 16 chunks of a row in registers
-constexpr int64_t kMaxElements = int64_t{1} << 38;
-constexpr int64_t kMaxRows = int64_t{1} << 31;
+// A launch has fewer than 2^32 threads.
+constexpr int64_t kMaxGroups = (int64_t{1} << 32) / kLanes - 1;
+constexpr int64_t kMaxElements = kMaxGroups * kLanes * 8;   // eight per thread
+constexpr int64_t kMaxNormRows = kMaxGroups * kRowWaves;    // one per wave
+constexpr int64_t kMaxRows = int64_t{1} << 31;              // where the grid does not grow with them
 
 int32_t sum_groups(const float *partials, int32_t groups, int32_t cols, void *out,
                    int32_t out_bf16, hipStream_t stream) {
@@ -446,7 +449,7 @@ extern "C" int32_t lct_column_sum(const void *g, int64_t rows, int32_t cols, flo
 extern "C" int32_t lct_rms_norm(const void *x, const void *gain, int32_t gain_bf16, void *y,
                                 float *rstd, int64_t rows, int32_t cols, hipStream_t stream) {
     if (!x || !gain || !y || !rstd) return LCT_E_NULL;
-    if (rows <= 0 || rows > kMaxRows || cols <= 0 || cols > kMaxColumns) return LCT_E_SIZE;
+    if (rows <= 0 || rows > kMaxNormRows || cols <= 0 || cols > kMaxColumns) return LCT_E_SIZE;
     if ((cols & 3) != 0 || !aligned(x, 8) || !aligned(y, 8)
         || !aligned(gain, gain_bf16 ? 8 : 16))
         return LCT_E_ARG;

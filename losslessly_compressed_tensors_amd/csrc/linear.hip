@@ -119,6 +119,9 @@ int32_t launch_skinny(const void *a, const void *w, void *out, int32_t tokens, i
 // 688 workgroups of one tile took 28 us, 230 of three 23.4 us.
 constexpr int32_t kCus = 256;
 
+// A launch has fewer than 2^32 threads; workgroups of the most tiles.
+constexpr int64_t kMaxLinearRows = ((int64_t{1} << 32) / kLinearThreads - 1) * 4 * kTile;
+
 }  // namespace
 }  // namespace lct
 
@@ -128,7 +131,7 @@ extern "C" int32_t lct_skinny_linear(const void *a, const void *w, void *out, in
                                      int32_t rows, int32_t cols, hipStream_t stream) {
     if (!a || !w || !out) return LCT_E_NULL;
     if (tokens <= 0 || tokens > LCT_MAX_SKINNY_TOKENS || rows <= 0 || cols <= 0
-        || rows > (1 << 30) || cols > (1 << 30))
+        || rows > kMaxLinearRows || cols > (1 << 30))
         return LCT_E_SIZE;
     if ((cols & 7) != 0
         || ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(w)) & 15) != 0

@@ -17,7 +17,10 @@ from . import hip
 
 _PLAIN = (Tensor, torch.nn.Parameter)
 _MAX_COLUMNS = 4096
-_MAX_ELEMENTS = 1 << 33   # keeps every row count within the entry points' 2^31
+# The entry points' limits, larger tensors being ATen's: a launch has fewer than
+# 2^32 threads (lct_relu_square: 8 elements each; lct_rms_norm: 64 per row).
+_MAX_ELEMENTS = 1 << 33
+_MAX_NORM_ROWS = (1 << 26) - 4
 # Row groups of the partial sums: the most that lct_column_sum and
 # lct_rms_norm_backward make.
 _COLUMN_GROUPS = 128
@@ -65,7 +68,7 @@ def relu_square_backward(grad: Tensor, relu: Tensor):
     """``grad`` becomes the gradient of ``relu(z)^2`` from its own, in place;
     returns ``relu^2``, or None (``grad`` is then as it was)."""
     if (grad.dtype != torch.bfloat16 or relu.dtype != torch.bfloat16 or grad.shape != relu.shape
-            or not native(grad, relu)):
+            or relu.numel() > _MAX_ELEMENTS or not native(grad, relu)):
         return None
     square = torch.empty_like(relu)
     hip.call("lct_relu_square_backward", relu.data_ptr(), grad.data_ptr(), square.data_ptr(),
@@ -93,8 +96,9 @@ def _norm_takes(x: Tensor, gain: Tensor) -> bool:
             and x.shape[-1] <= _MAX_COLUMNS and x.numel() <= _MAX_ELEMENTS)
 
 
-# lct_skinny_linear's range of A's rows.
+# lct_skinny_linear's range of A's rows, and of W's.
 MAX_SKINNY_TOKENS = 16
+_MAX_SKINNY_ROWS = (1 << 29) - 64
 
 
 def skinny_linear(a: Tensor, w: Tensor):
@@ -103,7 +107,7 @@ def skinny_linear(a: Tensor, w: Tensor):
     if (a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or a.ndim != 2
             or w.ndim != 2 or w.shape[1] != a.shape[1]
             or a.shape[0] > MAX_SKINNY_TOKENS or a.shape[1] % 8
-            or max(w.shape) > 1 << 30 or not native(a, w)):
+            or w.shape[0] > _MAX_SKINNY_ROWS or w.shape[1] > 1 << 30 or not native(a, w)):
         return None
     tokens, cols = a.shape
     rows = w.shape[0]
@@ -115,7 +119,8 @@ def skinny_linear(a: Tensor, w: Tensor):
 
 def rms_norm(x: Tensor, gain: Tensor):
     """``(bf16(x * rstd * bf16(gain)), rstd)`` over the last dimension, or None."""
-    if not _norm_takes(x, gain) or not native(x, gain):
+    if (not _norm_takes(x, gain) or x.numel() > _MAX_NORM_ROWS * x.shape[-1]
+            or not native(x, gain)):
         return None
     cols = x.shape[-1]
     y = torch.empty_like(x)

@@ -335,3 +335,16 @@ def test_fused_update_encoders_reject_bad_bookkeeping_before_launch(lib):
         assert call(record(meta=1 << 20, regions=100)) == LCT_E_ARG      # not a power of two
         assert call(record(meta=1 << 20, frees=hip.MAX_PENDING_FREES + 1)) == LCT_E_ARG
         assert call(record(meta=1 << 20, frees=1)) == LCT_E_NULL         # a missing descriptor
+
+
+def test_layer_kernels_reject_more_than_a_launch_holds(lib):
+    """A launch has fewer than 2^32 threads: sizes past what that gives each
+    kernel are LCT_E_SIZE before any launch (the pointers are never read)."""
+    fake = ctypes.c_void_p(1 << 20)
+    for n in (0, 2 ** 35 - 2047, 2 ** 35, 2 ** 38):
+        assert lib.lct_relu_square(fake, fake, fake, n, None) == LCT_E_SIZE
+        assert lib.lct_relu_square_backward(fake, fake, fake, n, None) == LCT_E_SIZE
+    for rows in (0, 2 ** 26 - 3, 2 ** 31):
+        assert lib.lct_rms_norm(fake, fake, 1, fake, fake, rows, 64, None) == LCT_E_SIZE
+    for rows in (0, 2 ** 29 - 63, 2 ** 30):
+        assert lib.lct_skinny_linear(fake, fake, fake, 16, rows, 8, None) == LCT_E_SIZE

@@ -41,6 +41,17 @@ def test_few_row_product_takes_matching_columns_only(no_launch):
     assert fused.skinny_linear(a, torch.zeros(5, 16, dtype=torch.bfloat16)) is None
 
 
+def test_tensors_past_the_launch_limits_are_left_to_aten(no_launch):
+    def empty(*shape):
+        return torch.empty(*shape, dtype=torch.bfloat16, device="meta")
+
+    assert fused.rms_norm(empty(2 ** 26 - 3, 64), empty(64)) is None
+    assert fused.rms_norm(empty(2 ** 31, 4), empty(4)) is None
+    assert fused.relu_square(empty(2 ** 33 + 8)) is None
+    assert fused.relu_square_backward(empty(2 ** 35), empty(2 ** 35)) is None
+    assert fused.skinny_linear(empty(16, 8), empty(2 ** 29 - 63, 8)) is None
+
+
 class _DeviceTensor:
     """What ``native`` asks of a tensor, for one on device ``index``."""
 
