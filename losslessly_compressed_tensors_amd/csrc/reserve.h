@@ -478,8 +478,8 @@ struct LdsReserve {
 // The request goes into word 0 of the job's own control array, where sample
 // group 0 posted its partial sum: every block of the job has read that before
 // it posts the summary that the scan waited for (a block that has not makes
-// the scan incomplete, and stays without a center).  Its tag differs from the
-// launch's by the top bit, so the partial sum is never taken for it.
+// the scan incomplete, and stays without a center).  Its tag is not the
+// launch's epoch (request_tag), so the partial sum is never taken for it.
 struct BatchJob {
     int32_t *descriptor;
     uint64_t *control;
@@ -487,8 +487,16 @@ struct BatchJob {
 
 constexpr int kMaxBatchJobs = 32;
 constexpr int kBatchWords = kMaxBatchJobs + kWavesPerBlock;   // LDS ints book_batch_job uses
-constexpr uint32_t kRequestTag = 0x80000000u;                 // flips the epoch's top bit
 constexpr uint32_t kIncompleteRequest = 0x80000000u;          // with the request's bytes
+
+// A request's tag: the launch's epoch with its top bit flipped, but never 0,
+// which a new control array's words carry.
+constexpr uint32_t request_tag(uint32_t epoch) {
+    return epoch == 0x80000000u ? 1u : epoch ^ 0x80000000u;
+}
+static_assert(request_tag(0x80000000u) != 0u && request_tag(0x80000000u) != 0x80000000u
+                  && request_tag(1u) != 0u && request_tag(0xFFFFFFFFu) != 0u,
+              "a request is told from an unwritten word and from a partial sum");
 
 // Workgroup-wide; contains barriers.  `words`: kBatchWords ints of LDS;
 // job_of(k): job k's BatchJob.
@@ -500,7 +508,7 @@ __device__ __forceinline__ void book_batch_job(int32_t job, int32_t n_jobs, JobO
                                                int32_t *__restrict__ blocks, int32_t n_blocks,
                                                LdsReserve<false> &arena, int32_t *words) {
     int32_t *const scratch = words + kMaxBatchJobs;
-    const uint32_t tag = polled.epoch ^ kRequestTag;
+    const uint32_t tag = request_tag(polled.epoch);
     if (job == 0) arena.begin(scratch);
     NoReserve none;
     const ScanTotals totals =

@@ -220,7 +220,8 @@ _control_lock = threading.Lock()
 
 # Epochs of lct_encode_fused: unique within the process (a 32-bit counter from
 # a random start, 0 skipped), so no word an earlier call left in a control
-# array matches a later call's epoch before 2^32 calls.
+# array matches a later call's epoch, or the tag that a batched launch derives
+# from it, before 2^31 calls.
 _FUSED_EPOCHS = itertools.count(int.from_bytes(os.urandom(4), "little"))
 
 

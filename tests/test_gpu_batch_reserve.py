@@ -8,6 +8,7 @@ import torch
 
 from gpu_util import require_gpu
 from losslessly_compressed_tensors_amd.comp_format import DistType, Distribution
+from losslessly_compressed_tensors_amd.kernels import dispatch
 from losslessly_compressed_tensors_amd.operations import (
     a_compA_add_b_B_batch, compress_batch, decompress)
 from losslessly_compressed_tensors_amd.tensor_buffer import (
@@ -104,3 +105,30 @@ def test_update_reservations_follow_job_order():
     for x, y, result in zip(tensors, others, results):
         want = torch.addcmul(x.float(), y.float(), beta).to(torch.bfloat16)
         assert torch.allclose(decompress(result).float(), want.float(), rtol=2 ** -7, atol=1e-30)
+
+
+@pytest.mark.parametrize("epoch", [1, 0x7FFFFFFF, 0x80000000, 0x80000001, 0xFFFFFFFF])
+@pytest.mark.parametrize("update", [False, True])
+def test_requests_are_told_from_unwritten_words(epoch, update, monkeypatch):
+    """At every epoch, the one whose top bit is its only one among them, a zeroed
+    control array holds no request: each record has its reservation."""
+    tensors = [_tensor(n, i) for i, n in enumerate(SIZES[:8])]
+    source = TensorBuffer(1 << 24, device="cuda")
+    buffer = TensorBuffer(1 << 24, device="cuda")
+    records = compress_batch(tensors, DIST, buffer=source)
+    calls = []
+    monkeypatch.setattr(dispatch, "_control_arrays", {})
+    monkeypatch.setattr(dispatch, "_next_fused_epoch", lambda: calls.append(1) or epoch)
+    if update:
+        one = torch.tensor([1.0], device="cuda")
+        results = a_compA_add_b_B_batch(records, one, [torch.zeros_like(x) for x in tensors], one,
+                                        buffer=buffer)
+    else:
+        results = compress_batch(tensors, DIST, buffer=buffer)
+    assert len(calls) == 1      # an epoch serves one launch
+    assert [tuple(_descriptor(r)[:3]) for r in results] == _first_fit(results, 1 << 24)
+    assert not buffer.failures()
+    for x, result in zip(tensors, results):
+        # (x + 0 turns -0 into 0.)
+        want = x + torch.zeros_like(x) if update else x
+        assert torch.equal(decompress(result).view(torch.int16), want.view(torch.int16))
