@@ -737,14 +737,16 @@ int32_t lct_compress_buffered_noalloc(const void *source, int64_t logical_numel,
  * drive the give-up paths from the host without long waits. */
 int32_t lct_set_wait_limits(int32_t lock_polls, int32_t ready_polls);
 
-/* ---- which decoder kernel lct_decode launches: LCT_DECODER_AUTO (the
- * default: the grouped kernel, or the wide-tile or compact one for whole grids
- * that they hold at once and it does not), LCT_DECODER_WIDE or
- * LCT_DECODER_COMPACT.  All write the same output.  Applies to launches made after the call.  No counterpart
- * in the reference: tests pin each kernel on the same inputs. */
+/* ---- which decoder kernel lct_decode and lct_decode_batch launch:
+ * LCT_DECODER_AUTO (the default: chosen by the grid), LCT_DECODER_WIDE,
+ * LCT_DECODER_COMPACT (which has no batched form: lct_decode_batch then chooses)
+ * or LCT_DECODER_GROUPED.  All write the same output.  Applies to launches made
+ * after the call.  No counterpart in the reference: tests pin each kernel on the
+ * same inputs. */
 #define LCT_DECODER_AUTO 0
 #define LCT_DECODER_WIDE 1
 #define LCT_DECODER_COMPACT 2
+#define LCT_DECODER_GROUPED 4
 int32_t lct_set_decoder(int32_t mode);
 
 /* ---- dense steps of the compressed layers (LCT/components/layers.py:16-71,

@@ -968,12 +968,13 @@ extern "C" int32_t lct_decode(const int32_t *encoded, const uint8_t *side, int16
     const size_t lds = static_cast<size_t>(register_stage_bytes(g.fixed_words));
     DecoderSlots slots;
     if (int32_t e = decoder_slots(g.fixed_words, &slots)) return e;
-    const int32_t mode = g_decoder_mode.load(std::memory_order_relaxed);
-    const Decoder decoder = mode == LCT_DECODER_WIDE      ? Decoder::kWide
-                            : mode == LCT_DECODER_COMPACT ? Decoder::kCompact
-                                                          : choose_decoder(n_blocks,
-                                                                           logical_numel != size,
-                                                                           slots);
+    Decoder decoder = choose_decoder(n_blocks, logical_numel != size, slots);
+    switch (g_decoder_mode.load(std::memory_order_relaxed)) {
+    case LCT_DECODER_WIDE: decoder = Decoder::kWide; break;
+    case LCT_DECODER_COMPACT: decoder = Decoder::kCompact; break;
+    case LCT_DECODER_GROUPED: decoder = Decoder::kGrouped; break;
+    default: break;
+    }
     const auto kernel = decoder == Decoder::kGrouped   ? decode_kernel_grouped
                         : decoder == Decoder::kCompact ? decode_kernel_compact
                                                        : decode_kernel;
@@ -987,7 +988,8 @@ extern "C" int32_t lct_decode(const int32_t *encoded, const uint8_t *side, int16
 }
 
 extern "C" int32_t lct_set_decoder(int32_t mode) {
-    if (mode != LCT_DECODER_AUTO && mode != LCT_DECODER_WIDE && mode != LCT_DECODER_COMPACT)
+    if (mode != LCT_DECODER_AUTO && mode != LCT_DECODER_WIDE && mode != LCT_DECODER_COMPACT
+        && mode != LCT_DECODER_GROUPED)
         return LCT_E_ARG;
     g_decoder_mode.store(mode, std::memory_order_relaxed);
     return LCT_OK;
@@ -1044,9 +1046,11 @@ extern "C" int32_t lct_decode_batch(const lct_decode_job *jobs, int32_t n_jobs,
     DecoderSlots slots;
     if (int32_t e = decoder_slots(max_words, &slots)) return e;
     slots.compact = 0;   // no batched form
-    const auto kernel = choose_decoder(total, ragged, slots) == Decoder::kWide
-                            ? decode_batch_kernel
-                            : decode_batch_kernel_grouped;
+    const int32_t mode = g_decoder_mode.load(std::memory_order_relaxed);
+    const bool wide = mode == LCT_DECODER_WIDE
+                      || (mode != LCT_DECODER_GROUPED
+                          && choose_decoder(total, ragged, slots) == Decoder::kWide);
+    const auto kernel = wide ? decode_batch_kernel : decode_batch_kernel_grouped;
     if (hipError_t e = reserve_dynamic_lds(reinterpret_cast<const void *>(kernel), lds))
         return static_cast<int32_t>(e);
     hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(total)), dim3(kLanes), lds, stream,

@@ -93,6 +93,9 @@ def test_decoder_choice_accepts_only_its_modes(lib):
     assert lib.lct_set_decoder(-1) == LCT_E_ARG
     for mode in (1, 2, 0):   # ends on the default (automatic)
         assert lib.lct_set_decoder(mode) == 0
+    assert lib.lct_set_decoder(5) == LCT_E_ARG
+    for mode in (4, 0):
+        assert lib.lct_set_decoder(mode) == 0
 
 
 def test_bad_geometry_is_rejected_before_launch(lib):

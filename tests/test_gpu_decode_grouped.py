@@ -9,6 +9,7 @@ from gpu_util import require_gpu
 from losslessly_compressed_tensors_amd.codec.decode import decode_batch
 from losslessly_compressed_tensors_amd.codec.geometry import geometry
 from losslessly_compressed_tensors_amd.comp_format import Distribution, DistType, NoiseLevel
+from losslessly_compressed_tensors_amd.kernels import hip
 from losslessly_compressed_tensors_amd.operations import compress, decompress
 
 pytestmark = pytest.mark.gpu
@@ -43,6 +44,27 @@ def test_grouped_decode_restores_tile_and_block_edges(family, noise, kind):
               block - 1, block, block + 1, 3 * block + 64 * 256 + 131):
         x = _values(kind, n)
         assert torch.equal(decompress(compress(x, dist)).view(torch.int16), x.view(torch.int16)), n
+
+
+@pytest.mark.parametrize("family,noise", LAYOUTS)
+@pytest.mark.parametrize("mode", [1, 2, 4])
+def test_each_decoder_restores_whole_and_partial_blocks(family, noise, mode):
+    """The wide, the compact and the grouped kernel pinned, singly and in one
+    batched launch, on values of every exponent and with few overflows."""
+    require_gpu()
+    print(f"case pinned {mode} {family.name} {noise.name}", flush=True)
+    dist = Distribution(family, noise_level=noise)
+    block = geometry(dist)[0]
+    hip.call("lct_set_decoder", mode)
+    try:
+        for kind in ("normal", "bits"):
+            tensors = [_values(kind, n) for n in (777, block, 2 * block - 1, 2 * block + 33 * 256 + 5)]
+            records = [compress(x, dist) for x in tensors]
+            for x, record, y in zip(tensors, records, decode_batch(records)):
+                assert torch.equal(decompress(record).view(torch.int16), x.view(torch.int16))
+                assert torch.equal(y.view(torch.int16), x.view(torch.int16))
+    finally:
+        hip.call("lct_set_decoder", 0)
 
 
 @pytest.mark.parametrize("blocks", [767, 768, 1024, 1600])
