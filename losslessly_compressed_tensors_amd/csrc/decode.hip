@@ -869,16 +869,16 @@ __global__ __launch_bounds__(kLanes) void decode_batch_kernel_grouped(DecodeBatc
                          job.ov, job.has_overlay, b - batch.first_block[j]);
 }
 
-// Workgroups of each decoder that the current device holds at once for W
-// payload words (CUs x workgroups per CU at that kernel's LDS), looked up once
-// per device and W.
+// The current device's CUs and the workgroups of each decoder that it holds at
+// once for W payload words (CUs x workgroups per CU at that kernel's LDS),
+// looked up once per device and W.
 struct DecoderSlots {
-    int32_t wide, compact, grouped;
+    int32_t cus, wide, compact, grouped;
 };
 
 constexpr int kSlotDevices = 64;
-constexpr int kSlotBits = 20;
-std::atomic<int64_t> g_decoder_slots[kSlotDevices][kMaxWords + 1];
+constexpr size_t kLdsGrant = 1280;
+std::atomic<uint64_t> g_decoder_slots[kSlotDevices][kMaxWords + 1];   // CUs << 24 | 8 bits each
 
 // lct_set_decoder's choice (LCT_DECODER_*).
 std::atomic<int32_t> g_decoder_mode{LCT_DECODER_AUTO};
@@ -887,7 +887,7 @@ int32_t decoder_slots(int W, DecoderSlots *slots) {
     int device = 0;
     if (hipError_t e = hipGetDevice(&device)) return static_cast<int32_t>(e);
     if (device < 0 || device >= kSlotDevices || W < 0 || W > kMaxWords) return LCT_E_ARG;
-    int64_t cached = g_decoder_slots[device][W].load(std::memory_order_relaxed);
+    uint64_t cached = g_decoder_slots[device][W].load(std::memory_order_relaxed);
     if (cached == 0) {
         int cus = 0;
         if (hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
@@ -898,43 +898,104 @@ int32_t decoder_slots(int W, DecoderSlots *slots) {
                                   reinterpret_cast<const void *>(decode_kernel_compact),
                                   reinterpret_cast<const void *>(decode_kernel_grouped)};
         for (int k = 0; k < 3; ++k) {
-            int per_cu = 0;
-            if (hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernels[k],
-                                                                            kLanes, lds))
+            // LDS is granted in units of kLdsGrant, which the lookup leaves out
+            // (compact at W = 22: 23056 bytes, 6 workgroups per CU and not 7:
+            // 32.4 us at 1536 blocks, 41.3 at 1600).
+            hipFuncAttributes attributes;
+            if (hipError_t e = hipFuncGetAttributes(&attributes, kernels[k]))
                 return static_cast<int32_t>(e);
-            cached |= static_cast<int64_t>(cus * per_cu) << (k * kSlotBits);
+            const size_t fixed = attributes.sharedSizeBytes;
+            const size_t granted = (fixed + lds + kLdsGrant - 1) / kLdsGrant * kLdsGrant;
+            int per_cu = 0;
+            if (hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                    &per_cu, kernels[k], kLanes, granted - fixed))
+                return static_cast<int32_t>(e);
+            cached |= static_cast<uint64_t>(per_cu) << (8 * k);
         }
+        cached |= static_cast<uint64_t>(cus) << 24;
         g_decoder_slots[device][W].store(cached, std::memory_order_relaxed);
     }
-    constexpr int64_t kMask = (int64_t{1} << kSlotBits) - 1;
-    *slots = {static_cast<int32_t>(cached & kMask),
-              static_cast<int32_t>((cached >> kSlotBits) & kMask),
-              static_cast<int32_t>((cached >> (2 * kSlotBits)) & kMask)};
+    const int32_t cus = static_cast<int32_t>(cached >> 24);
+    *slots = {cus, cus * static_cast<int32_t>(cached & 255u),
+              cus * static_cast<int32_t>((cached >> 8) & 255u),
+              cus * static_cast<int32_t>((cached >> 16) & 255u)};
     return LCT_OK;
 }
 
-// The decoder for a grid of n_blocks workgroups (LCT_DECODER_AUTO): the
-// grouped one, except between the grids it holds at once and those that the
-// wide or the compact one holds at once, which then run in one round where the
-// grouped one needs two.  `ragged`: the last block is partial, which costs the
-// wide and compact kernels another 3 (S = 128) to 9 us (S = 256) and the
-// grouped one nothing; it then takes every grid.  Public decompress, us
-// (wide / compact / grouped; W = 25 holds 1024 / 1536 / 768 workgroups, W = 12
-// 2048 / 2048 / 1024):
-//   W = 25:   36 blocks 24.8 / 28.8 / 15.6    688: 31.1 / 35.7 / 28.8
-//             767 ragged 39.0 / 40.7 / 29.5   1024: 39.0 / 42.1 / 43.5
-//            1536 blocks 72.2 / 77.1 / 66.1   2048: 95.5 / 115 / 92.7
-//   W = 12:   37 ragged 19.0 / 19.3 / 13.4    1024: 21.7 / 22.4 / 21.1
-//            2048 blocks 42.5 / 39.9 / 43.4   4096: 90.5 / 90.4 / 85.6
+// The decoder for a grid of n_blocks workgroups (LCT_DECODER_AUTO).  A grid that
+// the grouped kernel holds at once is its own.  Just past that the others still
+// run one round where it needs two, of which the second is far from full, and
+// from some size on its shorter lookup chain is worth more than their fuller
+// rounds.  Public decompress, us, wide / compact / grouped, last block whole |
+// partial (which costs the wide and compact kernels up to 7 us for a lone block
+// and next to nothing in a grid of several workgroups per CU); 256 CUs:
+//   W = 12 (2048 / 2048 / 1024 held), S = 128
+//      36: 15.4 / 15.7 / 12.3 | 17.6 / 17.8 / 12.3    1100: 24.6 / 25.0 / 29.7 | 25.6 / 26.7 / 29.8
+//    1350: 28.8 / 28.2 / 34.0 | 29.8 / 29.0 / 34.0    2048: 42.5 / 40.3 / 45.2 | 42.2 / 40.5 / 45.1
+//    2100: 45.9 / 46.6 / 44.1 | 47.2 / 47.7 / 44.1    2400: 49.8 / 51.6 / 51.4 | 50.0 / 51.8 / 51.3
+//    3072: 65.1 / 66.0 / 64.7 | 65.5 / 66.5 / 64.9    4096: 89.4 / 89.7 / 86.2 | 89.8 / 90.0 / 86.3
+//   W = 19 (1536 / 2048 / 768), S = 128
+//     800: 21.4 / 22.2 / 26.6 | 22.9 / 23.9 / 26.6    1300: 31.1 / 32.0 / 32.7 | 31.9 / 32.9 / 32.9
+//    1536: 32.6 / 32.1 / 37.5 | 33.2 / 32.5 / 37.7    2048: 51.7 / 44.5 / 50.6 | 51.1 / 44.9 / 50.7
+//    2560: 54.5 / 57.0 / 56.5 | 55.3 / 57.0 / 56.7    4096: 93.8 / 96.5 / 92.3 | 93.8 / 95.7 / 92.9
+//   W = 22 (1280 / 1536 / 768), S = 128
+//     900: 22.3 / 22.7 / 27.4 | 23.4 / 24.3 / 27.3    1450: 37.3 / 32.2 / 37.3 | 39.5 / 33.6 / 37.3
+//    1600: 39.5 / 41.3 / 40.7 | 41.6 / 43.6 / 40.8    2200: 49.7 / 51.2 / 52.0 | 50.7 / 51.9 / 52.0
+//    2560: 53.4 / 55.7 / 57.6 | 54.5 / 56.6 / 57.4    3328: 75.1 / 81.2 / 75.1 | 76.2 / 81.8 / 75.0
+//   W = 20 (1280 / 1792 / 768), S = 256
+//     900: 38.6 / 41.6 / 45.3 | 41.9 / 42.0 / 45.3    1100: 48.2 / 47.2 / 51.8 | 49.5 / 47.9 / 51.7
+//    1300: 65.2 / 67.3 / 58.9 | 70.8 / 68.2 / 59.6    1536: 76.9 / 76.1 / 69.3 | 78.3 / 76.2 / 68.9
+//   W = 25 (1024 / 1536 / 768), S = 256
+//      36: 24.4 / 28.7 / 15.6 | 32.5 / 32.7 / 15.6     900: 38.2 / 41.6 / 43.0 | 41.3 / 42.0 / 43.1
+//    1100: 56.0 / 47.8 / 51.1 | 62.6 / 49.0 / 50.6    1300: 59.9 / 66.6 / 56.1 | 65.7 / 67.9 / 57.4
+//    1536: 70.2 / 74.8 / 66.5 | 74.2 / 74.6 / 66.5    4096: 180 / 191 / 171 | 186 / 191 / 171
+// At S = 256 every kernel slows down where its output comes near 160 MiB (5
+// blocks per CU), the compact one most and from 4.7 blocks per CU on in some
+// runs (W = 20, 1215 blocks: 49 / 47 / 51 or 58 / 65 / 54): the line lies below.
+// A batched launch, which has no compact form, takes 48.8 | 52.0 wide and
+// 51.5 | 51.6 grouped at 1100 blocks of W = 20, and 50.3 | 64.1 and 50.5 | 57.9
+// at 1200.
 enum class Decoder { kWide, kCompact, kGrouped };
 
-Decoder choose_decoder(int64_t n_blocks, bool ragged, const DecoderSlots &slots) {
-    if (ragged || n_blocks <= slots.grouped) return Decoder::kGrouped;
-    // The wide kernel's 16-byte stores are faster where it holds the grid too
-    // (W = 25: 81 against 90 us at 2048 blocks; C3: 40 against 44 us).
-    if (n_blocks <= slots.wide) return Decoder::kWide;
-    return n_blocks <= slots.compact ? Decoder::kCompact : Decoder::kGrouped;
+constexpr Decoder choose_decoder(int64_t n_blocks, int S, const DecoderSlots &slots) {
+    const int64_t n = n_blocks, cus = slots.cus;
+    if (n <= slots.grouped) return Decoder::kGrouped;
+    if (S == 256) {
+        if (2 * n > 9 * cus) return Decoder::kGrouped;
+        if (n > 4 * cus && n <= slots.compact) return Decoder::kCompact;
+        return n <= slots.wide ? Decoder::kWide : Decoder::kGrouped;
+    }
+    // The compact kernel where only it holds the grid, and from 5.5 blocks per CU.
+    if (n <= slots.compact && (n > slots.wide || 2 * n >= 11 * cus)) return Decoder::kCompact;
+    if (n <= slots.wide) return Decoder::kWide;
+    // None holds it: the wide kernel's larger rounds where the grouped one has
+    // three workgroups per CU.
+    return slots.grouped < 4 * cus && n <= 12 * cus ? Decoder::kWide : Decoder::kGrouped;
 }
+
+// The table's grids.
+constexpr bool chooses(const DecoderSlots &slots, int S, int64_t n, Decoder decoder) {
+    return choose_decoder(n, S, slots) == decoder;
+}
+constexpr DecoderSlots kW12{256, 2048, 2048, 1024}, kW19{256, 1536, 2048, 768},
+    kW22{256, 1280, 1536, 768}, kW20{256, 1280, 1792, 768}, kW25{256, 1024, 1536, 768};
+static_assert(chooses(kW12, 128, 36, Decoder::kGrouped) && chooses(kW12, 128, 1100, Decoder::kWide)
+              && chooses(kW12, 128, 2048, Decoder::kCompact)
+              && chooses(kW12, 128, 2100, Decoder::kGrouped)
+              && chooses(kW12, 128, 4096, Decoder::kGrouped));
+static_assert(chooses(kW19, 128, 800, Decoder::kWide) && chooses(kW19, 128, 1300, Decoder::kWide)
+              && chooses(kW19, 128, 1536, Decoder::kCompact)
+              && chooses(kW19, 128, 2048, Decoder::kCompact)
+              && chooses(kW19, 128, 2560, Decoder::kWide)
+              && chooses(kW19, 128, 4096, Decoder::kGrouped));
+static_assert(chooses(kW22, 128, 900, Decoder::kWide) && chooses(kW22, 128, 1450, Decoder::kCompact)
+              && chooses(kW22, 128, 1600, Decoder::kWide)
+              && chooses(kW22, 128, 3328, Decoder::kGrouped));
+static_assert(chooses(kW20, 256, 900, Decoder::kWide) && chooses(kW20, 256, 1100, Decoder::kCompact)
+              && chooses(kW20, 256, 1300, Decoder::kGrouped));
+static_assert(chooses(kW25, 256, 36, Decoder::kGrouped) && chooses(kW25, 256, 900, Decoder::kWide)
+              && chooses(kW25, 256, 1100, Decoder::kCompact)
+              && chooses(kW25, 256, 1536, Decoder::kGrouped));
 
 }  // namespace
 }  // namespace lct
@@ -968,7 +1029,7 @@ extern "C" int32_t lct_decode(const int32_t *encoded, const uint8_t *side, int16
     const size_t lds = static_cast<size_t>(register_stage_bytes(g.fixed_words));
     DecoderSlots slots;
     if (int32_t e = decoder_slots(g.fixed_words, &slots)) return e;
-    Decoder decoder = choose_decoder(n_blocks, logical_numel != size, slots);
+    Decoder decoder = choose_decoder(n_blocks, g.steps, slots);
     switch (g_decoder_mode.load(std::memory_order_relaxed)) {
     case LCT_DECODER_WIDE: decoder = Decoder::kWide; break;
     case LCT_DECODER_COMPACT: decoder = Decoder::kCompact; break;
@@ -1003,7 +1064,7 @@ extern "C" int32_t lct_decode_batch(const lct_decode_job *jobs, int32_t n_jobs,
     batch.n_jobs = n_jobs;
     int64_t total = 0;
     int32_t max_words = 0;
-    bool ragged = false;
+    int32_t max_steps = 0;
     for (int32_t j = 0; j < n_jobs; ++j) {
         const lct_decode_job &in = jobs[j];
         if (!in.encoded || !in.side || !in.output || !in.shifted_decode || !in.center)
@@ -1038,7 +1099,7 @@ extern "C" int32_t lct_decode_batch(const lct_decode_job *jobs, int32_t n_jobs,
         out.rare = in.rare_length;
         out.has_overlay = in.has_overflow ? 1 : 0;
         out.ov = in.has_overflow ? in.overflow : lct_overflow{};
-        ragged = ragged || in.logical_numel != in.size;
+        max_steps = g.steps > max_steps ? g.steps : max_steps;
         max_words = g.fixed_words > max_words ? g.fixed_words : max_words;
     }
     batch.first_block[n_jobs] = static_cast<int32_t>(total);
@@ -1049,7 +1110,7 @@ extern "C" int32_t lct_decode_batch(const lct_decode_job *jobs, int32_t n_jobs,
     const int32_t mode = g_decoder_mode.load(std::memory_order_relaxed);
     const bool wide = mode == LCT_DECODER_WIDE
                       || (mode != LCT_DECODER_GROUPED
-                          && choose_decoder(total, ragged, slots) == Decoder::kWide);
+                          && choose_decoder(total, max_steps, slots) == Decoder::kWide);
     const auto kernel = wide ? decode_batch_kernel : decode_batch_kernel_grouped;
     if (hipError_t e = reserve_dynamic_lds(reinterpret_cast<const void *>(kernel), lds))
         return static_cast<int32_t>(e);

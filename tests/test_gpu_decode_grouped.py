@@ -85,3 +85,28 @@ def test_decode_around_the_grids_held_at_once(blocks):
         parts = [x[:half], x[half:]]
         for y, part in zip(decode_batch([compress(p, dist) for p in parts]), parts):
             assert torch.equal(y.view(torch.int16), part.view(torch.int16))
+
+
+@pytest.mark.parametrize("family,noise,blocks",
+                         [(DistType.GAUSSIAN, NoiseLevel.CLEAN, (1024, 1025, 1410, 2049)),
+                          (DistType.GAUSSIAN, NoiseLevel.MEDIUM, (769, 1410, 2049, 3073)),
+                          (DistType.LAPLACE, NoiseLevel.HIGH, (769, 1281, 1537)),
+                          (DistType.EMPIRICAL, NoiseLevel.SPARSE, (769, 1025, 1153)),
+                          (DistType.LAPLACE, NoiseLevel.CLEAN, (1025, 1153))])
+def test_decode_where_the_choice_changes(family, noise, blocks):
+    """Grids on either side of the lines of choose_decoder, whole and ragged,
+    single and batched."""
+    require_gpu()
+    dist = Distribution(family, noise_level=noise)
+    block = geometry(dist)[0]
+    for count in blocks:
+        print(f"case choice {family.name} {noise.name} {count}", flush=True)
+        generator = torch.Generator(device="cuda").manual_seed(count)
+        x = torch.randn(count * block, device="cuda", generator=generator).to(torch.bfloat16)
+        for y in (x, x[:-12345]):
+            records = [compress(y, dist)]
+            assert torch.equal(decompress(records[0]).view(torch.int16), y.view(torch.int16))
+            cut = (count // 3) * block
+            parts = [y[:cut], y[cut:]]
+            for out, part in zip(decode_batch([compress(p, dist) for p in parts]), parts):
+                assert torch.equal(out.view(torch.int16), part.view(torch.int16))
