@@ -168,7 +168,7 @@ def _normalized(x: Tensor, rstd: Tensor, gain: Tensor) -> Tensor:
 
 def _norm(x: Tensor, gain: Tensor) -> tuple[Tensor, Tensor]:
     """RMSNorm with the gain rounded to ``x``'s dtype."""
-    result = fused.rms_norm(x, gain)
+    result = fused.rms_norm(x, gain) if fused.norm_pays(x, gain) else None
     return rms_norm(x, gain.to(x.dtype)) if result is None else result
 
 
@@ -184,7 +184,7 @@ def _norm_backward(grad: Tensor, x: Tensor, rstd: Tensor, norm_weight: Tensor):
 
 def _bias_grad(g: Tensor, dtype: torch.dtype) -> Tensor:
     """``g``'s column sums in the bias's dtype."""
-    result = fused.column_sum(g, dtype)
+    result = fused.column_sum(g, dtype) if fused.column_sum_pays(g, dtype) else None
     return g.sum(0).to(dtype) if result is None else result
 
 

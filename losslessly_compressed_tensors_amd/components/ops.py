@@ -4,9 +4,9 @@ Same contract as ``LCT/components/ops.py:6-44``: ``rms_norm(x, gain)`` returns
 ``(y, rstd)`` over the last dimension, with the reciprocal RMS in FP32 and
 ``y`` in ``x``'s dtype; ``rms_norm_backward(grad, x, rstd, gain)`` returns
 ``(grad_x, grad_gain)`` (``grad_gain`` is ``None`` without a gain).  BF16 rows
-that fit a wave's registers run ``csrc/layers.hip`` (``kernels/fused.py``), others
-ATen's fused device kernels, so the dense regions around the codec need no
-tracing compiler.  ``rms_norm`` is differentiable through ``rms_norm_backward``.
+that fit a wave's registers run ``csrc/layers.hip`` where that is faster
+(``kernels/fused.py``), others ATen's fused device kernels, so the dense regions
+around the codec need no tracing compiler.  ``rms_norm`` is differentiable through ``rms_norm_backward``.
 """
 from __future__ import annotations
 
@@ -17,7 +17,8 @@ from ..kernels import fused
 
 
 def _forward(x: Tensor, gain: Tensor | None) -> tuple[Tensor, Tensor]:
-    if gain is not None and gain.dtype == x.dtype:
+    if (gain is not None and x.numel() >= fused.MIN_NORM_ELEMENTS and gain.dtype == x.dtype
+            and fused.norm_pays(x, gain)):
         result = fused.rms_norm(x, gain)
         if result is not None:
             return result
@@ -26,7 +27,7 @@ def _forward(x: Tensor, gain: Tensor | None) -> tuple[Tensor, Tensor]:
 
 def rms_norm_backward(grad: Tensor, x: Tensor, rstd: Tensor,
                       gain: Tensor | None) -> tuple[Tensor, Tensor | None]:
-    if gain is not None and gain.dtype == x.dtype:
+    if gain is not None and gain.dtype == x.dtype and fused.norm_backward_pays(x):
         result = fused.rms_norm_backward(grad, x, rstd, gain, gain.dtype, False)
         if result is not None:
             return result[:2]

@@ -25,9 +25,6 @@ _MAX_NORM_ROWS = (1 << 26) - 4
 # lct_rms_norm_backward make.
 _COLUMN_GROUPS = 128
 _NORM_GROUPS = 512
-# ATen's reduction and cast take 10.5 us up to 128 rows of 768 and 14.3 at 1024,
-# the two launches here 12 at any of these: the line lies where both sides were
-# measured to have crossed.
 _MIN_SUM_ROWS = 1024
 
 
@@ -74,6 +71,57 @@ def relu_square_backward(grad: Tensor, relu: Tensor):
     hip.call("lct_relu_square_backward", relu.data_ptr(), grad.data_ptr(), square.data_ptr(),
              relu.numel(), _stream(relu))
     return square
+
+
+# Where a kernel is faster than the expression it replaces, from host time per
+# call and kernel time together (us per call of calls in a row, the kernel's
+# against ATen's).
+
+
+def column_sum_pays(g: Tensor, dtype: torch.dtype) -> bool:
+    """:func:`column_sum`, about 13 us up to 8192 x 4096, against ``g.sum(0)`` and,
+    unless ``dtype`` is ``g``'s, its cast.  With the cast: 12.7 | 11.9 at 1024 x
+    64, 12.8 | 14.3 at 1536 x 64, 13.0 | 15.4 at 1024 x 128, 12.7 | 23.5 at 8192 x
+    768.  Without: 13.1 | 12.4 at 1536 x 768, 13.0 | 13.5 at 2048 x 768, 13.0 |
+    11.6 at 4096 x 128, 13.0 | 16.0 at 4096 x 256, 12.9 | 20.9 at 8192 x 768."""
+    numel = g.numel()
+    if g.shape[0] < _MIN_SUM_ROWS:
+        return False
+    if dtype != g.dtype:
+        return numel > 1 << 16
+    return numel >= 3 << 19 or (numel >= 1 << 20 and g.shape[0] >= 4096 and g.shape[1] >= 256)
+
+
+MIN_NORM_ELEMENTS = 1 << 20   # below, norm_pays is False for a gain of x's dtype
+
+
+def norm_pays(x: Tensor, gain: Tensor) -> bool:
+    """:func:`rms_norm`, 11.7 us up to 8192 x 1024.  With a gain that ATen has to
+    have cast: 12.0 | 13.5 at any smaller size, 12.4 | 14.9 at 8192 x 1024, 29.6 |
+    31.6 at 8192 x 4096.  Without: 11.7 | 7.3 at 1024 x 768, 11.9 | 11.3 at 8192 x
+    768, 11.8 to 13.9 | 12.4 at 8192 x 1024, 13.5 | 13.0 at 16384 x 64, 11.8 | 13.8
+    at 16384 x 256, 11.8 | 10.4 at 4096 x 2048, 13.5 | 13.5 at 4096 x 3072, 16.0 |
+    16.5 at 4096 x 4096, 13.2 | 17.4 at 8192 x 2048: ATen's time follows the
+    elements and, as 1024 more of them, the rows."""
+    if gain.dtype != x.dtype:
+        return True
+    numel = x.numel()
+    return (numel >= MIN_NORM_ELEMENTS
+            and numel + 1024 * (numel // x.shape[-1]) >= 18 << 20)
+
+
+def norm_backward_pays(x: Tensor) -> bool:
+    """:func:`rms_norm_backward` without ``rebuild``, 17.3 us up to 8192 x 1024,
+    for a gain of ``x``'s dtype: 17.4 | 10.1 at 16 x 768, 17.3 | 15.0 at 2048 x
+    768, 17.2 | 22.0 at 4096 x 768, 17.4 | 14.8 at 4096 x 64, 17.3 | 20.4 at 8192 x
+    64, 17.3 | 16.5 at 1024 x 2048, 17.2 | 23.8 at 2048 x 2048, 18.7 | 18.6 at 512 x
+    3072, 18.6 | 17.8 at 256 x 4096, 19.1 | 21.7 at 512 x 4096, 74 | 144 at 8192 x
+    4096.  (With ``rebuild``: 19.2 | 35 at 16 x 768 and more apart from there.)"""
+    numel = x.numel()
+    if numel < 1 << 18:
+        return False
+    cols = x.shape[-1]
+    return numel + 512 * (numel // cols) > (2 << 20 if cols > 2048 else 3 << 20)
 
 
 def column_sum(g: Tensor, dtype: torch.dtype):

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from losslessly_compressed_tensors_amd import operations
+from losslessly_compressed_tensors_amd.components import layers, ops
 from losslessly_compressed_tensors_amd.kernels import fused
 
 
@@ -50,6 +51,50 @@ def test_tensors_past_the_launch_limits_are_left_to_aten(no_launch):
     assert fused.relu_square(empty(2 ** 33 + 8)) is None
     assert fused.relu_square_backward(empty(2 ** 35), empty(2 ** 35)) is None
     assert fused.skinny_linear(empty(16, 8), empty(2 ** 29 - 63, 8)) is None
+
+
+def test_small_calls_stay_with_aten(no_launch):
+    """Where ATen's call takes less time than a launch of the row kernels."""
+    for rows, cols in ((1, 256), (64, 768), (1024, 64)):
+        x = torch.randn(rows, cols).to(torch.bfloat16)
+        gain = torch.ones(cols, dtype=torch.bfloat16)
+        y, rstd = ops._forward(x, gain)
+        want = torch.ops.aten._fused_rms_norm.default(x, [cols], gain, None)
+        assert torch.equal(y, want[0]) and torch.equal(rstd, want[1])
+    g = torch.randn(1024, 64).to(torch.bfloat16)
+    for dtype in (torch.bfloat16, torch.float32):
+        assert torch.equal(layers._bias_grad(g, dtype), g.sum(0).to(dtype))
+
+
+def test_where_the_row_kernels_pay():
+    """Both sides of each line, at sizes where both were timed."""
+    def empty(rows, cols, dtype=torch.bfloat16):
+        return torch.empty(rows, cols, dtype=dtype, device="meta")
+
+    def gain(cols, dtype=torch.bfloat16):
+        return torch.empty(cols, dtype=dtype, device="meta")
+
+    for rows, cols, pays in ((0, 256, False), (1, 64, False), (8192, 64, False), (16384, 64, False),
+                             (8192, 768, False), (8192, 1024, False), (16384, 256, True),
+                             (4096, 2048, False), (4096, 3072, False), (2048, 4096, False),
+                             (4096, 4096, True), (8192, 2048, True)):
+        assert fused.norm_pays(empty(rows, cols), gain(cols)) == pays, (rows, cols)
+        assert fused.norm_pays(empty(rows, cols), gain(cols, torch.float32))
+    for rows, cols, pays in ((0, 256, False), (16, 768, False), (4096, 64, False),
+                             (8192, 64, True), (2048, 768, False), (4096, 768, True),
+                             (2048, 1024, False), (1024, 2048, False), (2048, 2048, True),
+                             (512, 3072, False), (1024, 3072, True), (256, 4096, False),
+                             (512, 4096, True)):
+        assert fused.norm_backward_pays(empty(rows, cols)) == pays, (rows, cols)
+    assert not fused.norm_pays(torch.empty((), dtype=torch.bfloat16), gain(1))
+    for rows, cols, bf16, fp32 in ((1023, 4096, False, False), (1024, 64, False, False), (1536, 64, False, True),
+                                   (1024, 128, False, True), (8192, 8, False, False),
+                                   (16384, 64, False, True), (4096, 128, False, True),
+                                   (2048, 256, False, True), (4096, 256, True, True),
+                                   (1536, 768, False, True), (2048, 768, True, True),
+                                   (1024, 3072, True, True), (8192, 768, True, True)):
+        assert fused.column_sum_pays(empty(rows, cols), torch.bfloat16) == bf16, (rows, cols)
+        assert fused.column_sum_pays(empty(rows, cols), torch.float32) == fp32, (rows, cols)
 
 
 class _DeviceTensor:

@@ -105,7 +105,9 @@ def test_what_the_kernels_leave_to_aten():
 @pytest.mark.filterwarnings("ignore::DeprecationWarning")
 def test_a_trace_records_the_operations():
     """A traced norm computes its own inputs' norm."""
-    first, x, gain = _values(64, 256), _values(64, 256, seed=1), 1 + 0.1 * _values(256, seed=2)
+    first, x = _values(16384, 256), _values(16384, 256, seed=1)
+    gain = 1 + 0.1 * _values(256, seed=2)
+    assert fused.norm_pays(first, gain)
     traced = torch.jit.trace(lambda t: ops.rms_norm(t, gain), (first,))
     y, rstd = torch.ops.aten._fused_rms_norm.default(x, [256], gain, None)
     again = traced(x)
