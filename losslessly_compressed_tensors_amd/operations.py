@@ -63,7 +63,7 @@ def A_compBT(A: Tensor, B_comp: CompressedTensor) -> Tensor:
     if A.ndim != 2 or A.shape[1] != B_comp.shape[1]:
         raise ValueError("activation and weight inner dimensions must match")
     A, B = A.contiguous(), decompress(B_comp)
-    product = fused.skinny_linear(A, B)
+    product = fused.skinny_linear(A, B) if A.shape[0] <= fused.MAX_SKINNY_TOKENS else None
     return A @ B.T if product is None else product
 
 
