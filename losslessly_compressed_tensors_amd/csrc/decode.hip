@@ -718,6 +718,20 @@ __device__ __forceinline__ void store_tile(const uint8_t *tile, const GroupSides
     }
 }
 
+// An escape (y = 0) at bit `offset` (low 5 bits, at most 16) of `bits` becomes one
+// symbol of at most 16 bits: ESC + 8-bit literal table index (primitives.py:
+// 29-35).  A third lookup's window would then pass the 32 bits' end.
+__device__ __forceinline__ void take_escape(uint2 &entry, uint32_t &third, uint32_t bits,
+                                            uint32_t offset, int rare, int32_t center) {
+    const bool escaped = entry.y == 0u;
+    const uint32_t literal = __builtin_amdgcn_ubfe(bits, (offset & 31u) + rare, 8);
+    const uint32_t exponent = static_cast<uint32_t>(
+        index_to_exponent(static_cast<int32_t>(literal), center) + 127) & 255u;
+    entry.x = escaped ? exponent : entry.x;
+    entry.y = escaped ? static_cast<uint32_t>(rare + 8) | 8u << 8 : entry.y;
+    third = escaped ? 0u : third;
+}
+
 // Codec block `block` of one tensor, by the workgroup.
 __device__ __forceinline__ void decode_block_grouped(
     const int32_t *__restrict__ encoded, const uint8_t *__restrict__ side,
@@ -787,28 +801,41 @@ __device__ __forceinline__ void decode_block_grouped(
                 __builtin_amdgcn_sched_barrier(0);
                 column.append(held, held8);
                 __builtin_amdgcn_sched_barrier(0);
-                uint32_t third = ~0u;
+                uint32_t two;
+                uint2 e2;
                 if (__builtin_expect(__any(e0.y == 0u), 0)) {
-                    // ESC + 8-bit literal table index (primitives.py:29-35).
-                    const bool escaped = e0.y == 0u;
-                    const int32_t literal = static_cast<int32_t>((bits >> rare) & 255u);
-                    e0.x = escaped ? static_cast<uint32_t>(index_to_exponent(literal, center) + 127)
-                                         & 255u
-                                   : e0.x;
-                    e0.y = escaped ? static_cast<uint32_t>(rare + 8) | 8u << 8 : e0.y;
-                    third = escaped ? 0u : third;   // its window would pass the 32 bits' end
+                    // A turn of its own, which takes the second lookup's escape
+                    // too: escapes come in runs, a row of larger values lying
+                    // 30 steps long in every stream (a 2282 x 7616 tensor of
+                    // such rows, 531 blocks of W = 22: 23.0 us with one escape
+                    // per turn, 20.4 with two, the wide kernel 21.3; without
+                    // escapes the same within 2 %).
+                    uint32_t third = ~0u;
+                    take_escape(e0, third, bits, 0u, rare, center);
+                    uint2 e1 = tb.entry[__builtin_amdgcn_ubfe(bits, e0.y, kGroupBits)];
+                    __builtin_amdgcn_sched_barrier(0);
+                    column.append(e0.x, e0.y >> 8);
+                    __builtin_amdgcn_sched_barrier(0);
+                    take_escape(e1, third, bits, e0.y, rare, center);
+                    two = e0.y + e1.y;
+                    e2 = tb.entry[__builtin_amdgcn_ubfe(bits, two, kGroupBits)];
+                    __builtin_amdgcn_sched_barrier(0);
+                    column.append(e1.x, e1.y >> 8);
+                    __builtin_amdgcn_sched_barrier(0);
+                    e2.x &= third;
+                    e2.y &= third;
+                } else {
+                    const uint2 e1 = tb.entry[__builtin_amdgcn_ubfe(bits, e0.y, kGroupBits)];
+                    __builtin_amdgcn_sched_barrier(0);
+                    column.append(e0.x, e0.y >> 8);
+                    __builtin_amdgcn_sched_barrier(0);
+                    two = e0.y + e1.y;   // lengths in bits 0..5, rows from bit 8
+                    e2 = tb.entry[__builtin_amdgcn_ubfe(bits, two, kGroupBits)];
+                    __builtin_amdgcn_sched_barrier(0);
+                    column.append(e1.x, e1.y >> 8);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                const uint2 e1 = tb.entry[__builtin_amdgcn_ubfe(bits, e0.y, kGroupBits)];
-                __builtin_amdgcn_sched_barrier(0);
-                column.append(e0.x, e0.y >> 8);
-                __builtin_amdgcn_sched_barrier(0);
-                const uint32_t two = e0.y + e1.y;   // lengths in bits 0..4, rows from bit 8
-                uint2 e2 = tb.entry[__builtin_amdgcn_ubfe(bits, two, kGroupBits)];
-                __builtin_amdgcn_sched_barrier(0);
-                column.append(e1.x, e1.y >> 8);
-                __builtin_amdgcn_sched_barrier(0);
-                e2.y &= third;
-                held = e2.x & third;
+                held = e2.x;
                 held8 = e2.y >> 8;
                 const uint32_t all = two + e2.y;
                 row8 += all >> 8;

@@ -47,6 +47,28 @@ def test_grouped_decode_restores_tile_and_block_edges(family, noise, kind):
 
 
 @pytest.mark.parametrize("family,noise", LAYOUTS)
+@pytest.mark.parametrize("run", [1, 2, 3, 5, 30, 64, 70])
+def test_runs_of_escapes(family, noise, run):
+    """Rows of 256 values whose exponents no code has, `run` at a time at every
+    distance from a tile's edges, in all lanes and in every third."""
+    require_gpu()
+    print(f"case runs {family.name} {noise.name} {run}", flush=True)
+    dist = Distribution(family, noise_level=noise)
+    block = geometry(dist)[0]
+    generator = torch.Generator(device="cuda").manual_seed(run)
+    x = torch.randn(3 * block + 777, device="cuda", generator=generator).to(torch.bfloat16)
+    rows = x[:3 * block].view(-1, 256)
+    start, far = 0, 2.0 ** -70
+    for gap in range(1, 40):
+        rows[start:start + run] *= far
+        start += run + gap
+    rows[block // 256:2 * block // 256, 1::3] *= far
+    record = compress(x, dist)
+    assert torch.equal(decompress(record).view(torch.int16), x.view(torch.int16))
+    assert torch.equal(decode_batch([record, record])[1].view(torch.int16), x.view(torch.int16))
+
+
+@pytest.mark.parametrize("family,noise", LAYOUTS)
 @pytest.mark.parametrize("mode", [1, 2, 4])
 def test_each_decoder_restores_whole_and_partial_blocks(family, noise, mode):
     """The wide, the compact and the grouped kernel pinned, singly and in one
