@@ -505,10 +505,9 @@ __global__ __launch_bounds__(kLanes, 8) void decode_kernel_compact(
 //
 // What bounds it: with up to one workgroup per CU the chain of lookups (27 turns
 // of three per 256 symbols; 15.6 us per public decompress at 36 blocks of 256
-// steps against the wide kernel's 24.8), then the LDS (23.0 us at 512 blocks),
-// from about 688 blocks on HBM (28.8 us, 5.3 TB/s; 85.6 us at 4096 blocks of
-// 128 steps against 90.5, inputs and outputs rotating over three sets).
-// Measured against it: the exponent bytes stored one by one in row-major tiles
+// steps against the wide kernel's 24.4), then the LDS (22.5 us at 512 blocks),
+// from about 688 blocks on HBM (28.1 us, 5.4 TB/s; 86.2 us at 4096 blocks of
+// 128 steps against 89.4).  Measured against an earlier form (28.8 us at 688): the exponent bytes stored one by one in row-major tiles
 // (12 byte stores per turn: 29.6 against 28.8 us at 688 blocks, 23.2 at 512);
 // 9-bit tables or 32-row tiles (more workgroups per CU, but 15.3 to 17.7 us at
 // 36 blocks and 0.4 to 2 us slower at 4096).

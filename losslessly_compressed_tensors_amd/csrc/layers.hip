@@ -103,7 +103,8 @@ __global__ __launch_bounds__(kLanes) void relu_square_backward_kernel(
 // hold a row's 128 bytes, so its 32 rows in flight are whole lines, and about
 // 2048 workgroups share the matrix whatever its width (ATen's reduction ran 3
 // workgroups for 768 columns and 12 for 3072: 21 and 23 us at 8192 rows; here
-// 8.8 and 13.5 with the second launch).  The partial sums of the row
+// 8.8 and 13.5 with the second launch; per call, host time included, 13 against 20
+// to 25).  Where it is called: column_sum_pays in kernels/fused.py.  The partial sums of the row
 // groups are added in their order by sum_groups_kernel, so the result does not
 // depend on timing.
 constexpr int kSumColumns = 64;
@@ -271,7 +272,11 @@ __global__ __launch_bounds__(kLanes) void rms_norm_kernel(const uint16_t *__rest
 // in three launches and 40 us to rebuild the rows in FP32 steps at 8192 x 768;
 // here 17.7 in two launches.)  A wave walks rows `waves in the grid` apart with
 // the next row's loads in flight, since its sums of the gain's gradient stay in
-// registers.
+// registers: 250 of them at 2048 columns, 349 and 460 (accumulation registers
+// among them) at 3072 and 4096, one wave per SIMD from 2049 columns on, where
+// rows of HBM's bytes still keep it ahead (with the rows rebuilt, us per call
+// here | ATen: 27 | 63 at 2048 x 2304, 55 | 230 at 8192 x 3072, 23 | 54 at 1024 x
+// 4096, 78 | 302 at 8192 x 4096).
 template <int kChunks>
 __global__ __launch_bounds__(kLanes) void rms_norm_backward_kernel(
     const uint16_t *__restrict__ grad, const uint16_t *__restrict__ x,

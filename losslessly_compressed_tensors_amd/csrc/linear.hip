@@ -12,7 +12,11 @@
 // (the library's product: 25.1, 36.7 and 12.0), of which the read of W at the
 // 6.9 TB/s that a plain read reaches is 13, 13 and 5.  Loading the next four
 // steps during the product made no difference.  From 17 rows on the library's
-// tiles, which share A's loads, are faster.
+// tiles, which share A's loads, are faster.  Fewer rows and smaller weights, us
+// per call here | library, W rotating over four to six: 9.7 | 21 from 64 x 64 to
+// 8192 x 2048 at 1 to 16 rows (host time), 15.7 | 21 at one row of 32768 x 1024,
+// 21.5 | 26.4 at one of 11008 x 4096, 19.6 | 38.5 at one of 4096 x 11008, 53.7 |
+// 63.8 at one and 60.0 | 68.8 at 16 of 16384 x 8192.
 #include "lct_device.h"
 
 namespace lct {
